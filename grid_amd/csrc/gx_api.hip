@@ -552,11 +552,26 @@ static void build_smats(Op *op) {
   product(op->smat[Op::S_MOOEEINVDAG], op->smat[Op::S_MEOOEDAG5D], op->smat[Op::S_INVDAG_MEODAG5D]);
 }
 
+// whether a banded operator's chirality 0 couples to s + 1 (the adjoints) rather than s - 1
+static bool band_dag(int which) {
+  return which == Op::S_MEOOEDAG5D || which == Op::S_MOOEEDAG || which == Op::S_M5DDAG_OFF;
+}
+
 static int upload_smats(Op *op) {
   const int Ls = op->g.Ls;
   const size_t per = 2 * (size_t)Ls * Ls;
-  std::vector<double> all(per * Op::S_COUNT);
-  for (int i = 0; i < Op::S_COUNT; i++) std::memcpy(&all[i * per], op->smat[i].m.data(), per * sizeof(double));
+  std::vector<double> all((per + 4 * (size_t)Ls) * Op::S_COUNT);
+  for (int i = 0; i < Op::S_COUNT; i++) {
+    std::memcpy(&all[i * per], op->smat[i].m.data(), per * sizeof(double));
+    const bool dag = band_dag(i);
+    double *b = &all[per * Op::S_COUNT + 4 * (size_t)Ls * i];
+    for (int chi = 0; chi < 2; chi++)
+      for (int s = 0; s < Ls; s++) {
+        const int n = ((chi == 0) == dag) ? (s + 1) % Ls : (s + Ls - 1) % Ls;
+        b[2 * chi * Ls + s] = all[i * per + ((size_t)chi * Ls + s) * Ls + s];
+        b[(2 * chi + 1) * Ls + s] = all[i * per + ((size_t)chi * Ls + s) * Ls + n];
+      }
+  }
   std::vector<float> allf(all.begin(), all.end());
   for (int p = 0; p < 2; p++)
     if (op->smat_dev[p]) {
@@ -574,21 +589,13 @@ static int upload_smats(Op *op) {
 // FP64 and FP32, in place when the arrays exist (captured graphs keep their pointers valid).
 int op_upload_coefs(Op *op) {
   const int Ls = op->g.Ls;
-  std::vector<double> c(4 * (size_t)Ls);
-  for (int s = 0; s < Ls; s++) {
-    if (op->kind == GX_WILSON) {
-      const double m = op->slice_mass.empty() ? op->mass : op->slice_mass[s];
-      const double d = 4.0 + m;  // WilsonFermionImplementation.h:71, diag_mass = 4 + m
-      c[s] = -1.0 / d;
-      c[Ls + s] = d;
-      c[2 * Ls + s] = 1.0 / d;
-      c[3 * Ls + s] = d;
-    } else {
-      c[s] = -1.0;
-      c[Ls + s] = 1.0;
-      c[2 * Ls + s] = 1.0;
-      c[3 * Ls + s] = 1.0;
-    }
+  std::vector<double> c(4 * (size_t)Ls, 1.0);
+  for (int s = 0; s < Ls && op->kind == GX_WILSON; s++) {
+    const double m = op->slice_mass.empty() ? op->mass : op->slice_mass[s];
+    const double d = 4.0 + m;  // WilsonFermionImplementation.h:71, diag_mass = 4 + m
+    c[Op::C_MINUS_INV * Ls + s] = -1.0 / d;
+    c[Op::C_D * Ls + s] = d;
+    c[Op::C_INV * Ls + s] = 1.0 / d;
   }
   op->coef_host = c;
   op->coef_host_f.assign(c.begin(), c.end());
@@ -605,12 +612,14 @@ int op_upload_coefs(Op *op) {
   return GX_OK;
 }
 
-int op_coef(Op *op, int prec, const void **coef) {
-  *coef = op->coef_dev[prec == GX_F64 ? 0 : 1];
-  if (!*coef) {
+int op_coef(Op *op, int prec, int which, const void **coef) {
+  const void *c = op->coef_dev[prec == GX_F64 ? 0 : 1];
+  if (!c) {
     set_error("operator coefficients missing");
     return GX_EINVAL;
   }
+  const size_t at = (size_t)which * op->g.Ls;
+  *coef = prec == GX_F64 ? (const void *)((const double *)c + at) : (const void *)((const float *)c + at);
   return GX_OK;
 }
 
@@ -619,6 +628,13 @@ int op_smat(Op *op, int prec, int which, const void **mats) {
   const size_t per = 2 * (size_t)op->g.Ls * op->g.Ls;
   if (prec == GX_F64) *mats = (const double *)op->smat_dev[GX_F64] + which * per;
   else *mats = (const float *)op->smat_dev[GX_F32] + which * per;
+  return GX_OK;
+}
+
+int op_band(Op *op, int prec, int which, const void **bands) {
+  const size_t Ls = op->g.Ls, at = Op::S_COUNT * 2 * Ls * Ls + 4 * Ls * which;
+  if (prec == GX_F64) *bands = (const double *)op->smat_dev[GX_F64] + at;
+  else *bands = (const float *)op->smat_dev[GX_F32] + at;
   return GX_OK;
 }
 
@@ -633,12 +649,16 @@ int apply_dhop_half(Op *op, Field *in, Field *out, int cb_out, int dag, const Ga
   });
 }
 
+// out = A(in) (+ phi): the two-band operators through launch_band (phi: these only), the others dense
 static int apply_smat(Op *op, Field *in, Field *phi, Field *out, int which, const Gate *gate) {
   const void *m;
-  GX_TRY(op_smat(op, in->prec, which, &m));
+  const bool dense = which == Op::S_MOOEEINV || which == Op::S_MOOEEINVDAG;
+  GX_TRY(dense ? op_smat(op, in->prec, which, &m) : op_band(op, in->prec, which, &m));
   out->cb = in->cb;
   return by_prec(in->prec, [&](auto t) {
-    return launch_smat<decltype(t)>(op->g, in->data, phi ? phi->data : nullptr, out->data, m, gate, op->ctx->stream);
+    if (dense) return launch_smat<decltype(t)>(op->g, in->data, out->data, m, gate, op->ctx->stream);
+    return launch_band<decltype(t)>(op->g, in->data, phi ? phi->data : nullptr, out->data, m, band_dag(which), gate,
+                                    op->ctx->stream);
   });
 }
 
@@ -659,10 +679,8 @@ int apply_meooe(Op *op, Field *in, Field *out, int dag, const Gate *gate) {
 int apply_mooee(Op *op, Field *in, Field *out, int which, const Gate *gate) {
   if (op->kind == GX_WILSON) {
     if (!op->slice_mass.empty()) {  // d_s (Mooee) or 1/d_s (MooeeInv) on each slice
-      const void *c;
-      GX_TRY(op_coef(op, in->prec, &c));
-      const size_t off = (size_t)(which < 2 ? 3 : 2) * op->g.Ls;
-      const void *cs = in->prec == GX_F64 ? (const void *)((const double *)c + off) : (const void *)((const float *)c + off);
+      const void *cs;
+      GX_TRY(op_coef(op, in->prec, which < 2 ? Op::C_D : Op::C_INV, &cs));
       out->cb = in->cb;
       return by_prec(in->prec, [&](auto t) {
         return launch_scale_slices<decltype(t)>(op->g, in->data, out->data, cs, gate, op->ctx->stream);
@@ -680,8 +698,11 @@ int apply_mooee(Op *op, Field *in, Field *out, int which, const Gate *gate) {
 //   Wilson  Mpc    = d in - (1/d) Dhop(Dhop(in)),  d = 4 + m                      2 kernels
 //   Cayley  Mpc    = Mooee in - Dhop(P1 Dhop(Meooe5D in)),  P1 = Meooe5D MooeeInv   3 kernels
 //           MpcDag = MooeeDag in - MeooeDag5D Dhop^dag(P2 Dhop^dag in),
-//                    P2 = MooeeInvDag MeooeDag5D                                   3 kernels
-// The fifth-dimension matrices act across each site's s-row in the hop kernel's epilogue.
+//                    P2 = MooeeInvDag MeooeDag5D                                   2 kernels
+// The fifth-dimension matrices act across each site's s-row in the hop kernel's epilogue; the second
+// hop's reads in itself for Mooee in (both its matrices have two bands).  A field pass that writes Mooee
+// in for the second hop costs more than the epilogue's few LDS reads: MpcDagMpc FP32 on 20 x 12 x 18 x 28
+// x 10 265 us with it, 223 us without.
 template <typename T>
 static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, const HopFuse *fz) {
   const int prec = in->prec, cb_in = in->cb, cb_mid = 1 - cb_in;
@@ -690,35 +711,67 @@ static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, c
   void *U_mid = cb_mid == 0 ? Ue : Uo, *U_in = cb_in == 0 ? Ue : Uo;
   hipStream_t st = op->ctx->stream;
   const Geom &g = op->g;
-  Field *t0 = op_tmp(op, prec, 0), *t1 = op_tmp(op, prec, 1), *t3 = op_tmp(op, prec, 3);
-  if (!t0 || !t1 || !t3) return GX_ENOMEM;
-  const void *coef;  // per-slice (alpha_s, beta_s) of the EPI 1 hops: Wilson (-1/d_s, d_s), Cayley (-1, 1)
-  GX_TRY(op_coef(op, prec, &coef));
+  Field *t0 = op_tmp(op, prec, 0), *t3 = op_tmp(op, prec, 3);
+  if (!t0 || !t3) return GX_ENOMEM;
   if (op->kind == GX_WILSON) {
-    GX_TRY(launch_dhop_epi<T>(g, in->data, t0->data, U_mid, cb_mid, dag, gate, st, 0, nullptr, nullptr, 1.0, 0.0));
-    GX_TRY(launch_dhop_epi<T>(g, t0->data, out->data, U_in, cb_in, dag, gate, st, 1, in->data, nullptr, 0.0, 0.0, 0,
-                              coef, fz));
-  } else if (!dag) {
-    const void *m_meo, *m_mooee, *m_p1;
-    GX_TRY(op_smat(op, prec, Op::S_MEOOE5D, &m_meo));
-    GX_TRY(op_smat(op, prec, Op::S_MOOEE, &m_mooee));
-    GX_TRY(op_smat(op, prec, Op::S_MEO5D_INV, &m_p1));
-    // t0 = Meooe5D in, t1 = Mooee in (one read of in)
-    GX_TRY(launch_smat2<T>(g, in->data, nullptr, 0.0, t0->data, m_meo, t1->data, m_mooee, gate, st));
-    GX_TRY(launch_dhop_epi<T>(g, t0->data, t3->data, U_mid, cb_mid, 0, gate, st, 2, nullptr, m_p1, 1.0, 0.0));
-    GX_TRY(launch_dhop_epi<T>(g, t3->data, out->data, U_in, cb_in, 0, gate, st, 1, t1->data, nullptr, 0.0, 0.0, 0,
-                              coef, fz));
+    const void *minus_inv, *d;  // -1/d_s, d_s
+    GX_TRY(op_coef(op, prec, Op::C_MINUS_INV, &minus_inv));
+    GX_TRY(op_coef(op, prec, Op::C_D, &d));
+    GX_TRY(launch_dhop_epi<T>(g, in->data, t0->data, U_mid, cb_mid, dag, gate, st, 0, nullptr, nullptr, 1.0));
+    GX_TRY(launch_dhop_epi<T>(g, t0->data, out->data, U_in, cb_in, dag, gate, st, 1, in->data, d, 0.0, 0, minus_inv,
+                              fz));
   } else {
-    const void *m_mooeedag, *m_p2, *m_meodag;
-    GX_TRY(op_smat(op, prec, Op::S_MOOEEDAG, &m_mooeedag));
-    GX_TRY(op_smat(op, prec, Op::S_INVDAG_MEODAG5D, &m_p2));
-    GX_TRY(op_smat(op, prec, Op::S_MEOOEDAG5D, &m_meodag));
-    GX_TRY(launch_smat2<T>(g, in->data, nullptr, 0.0, t1->data, m_mooeedag, nullptr, nullptr, gate, st));
-    GX_TRY(launch_dhop_epi<T>(g, in->data, t3->data, U_mid, cb_mid, 1, gate, st, 2, nullptr, m_p2, 1.0, 0.0));
-    GX_TRY(launch_dhop_epi<T>(g, t3->data, out->data, U_in, cb_in, 1, gate, st, 2, t1->data, m_meodag, -1.0, 1.0, 0,
-                              nullptr, fz));
+    const void *m_p, *b_meo, *b_mooee;
+    GX_TRY(op_smat(op, prec, dag ? Op::S_INVDAG_MEODAG5D : Op::S_MEO5D_INV, &m_p));
+    GX_TRY(op_band(op, prec, dag ? Op::S_MEOOEDAG5D : Op::S_MEOOE5D, &b_meo));
+    GX_TRY(op_band(op, prec, dag ? Op::S_MOOEEDAG : Op::S_MOOEE, &b_mooee));
+    const void *first = in->data;
+    if (!dag) {
+      GX_TRY(launch_band<T>(g, in->data, nullptr, t0->data, b_meo, 0, gate, st));
+      first = t0->data;
+    }
+    GX_TRY(launch_dhop_epi<T>(g, first, t3->data, U_mid, cb_mid, dag, gate, st, 2, nullptr, m_p, 1.0));
+    GX_TRY(launch_dhop_epi<T>(g, t3->data, out->data, U_in, cb_in, dag, gate, st, 3, in->data, dag ? b_meo : nullptr,
+                              -1.0, 0, b_mooee, fz));
   }
   out->cb = cb_in;
+  return GX_OK;
+}
+
+// Fused M and Mdag, one hop per checkerboard whose epilogue adds the diagonal part from in:
+//   Wilson  M    = Dhop in + d in                              3 field passes per checkerboard
+//   Cayley  M    = Dhop(Meooe5D in) + Mooee in                 5 (Meooe5D in its own kernel)
+//           Mdag = MeooeDag5D Dhop^dag in + MooeeDag in        3
+// Mdag in FP64 on 24^4 x 12: 842 us, 1653 us as four kernels and 9 passes per checkerboard (the floor, one
+// read and one write of the field and the links, is 306 us at 6.25 TB/s; the hops' neighbours bound it).
+template <typename T>
+static int full_m_fused(Op *op, Field *in, Field *out, int dag) {
+  const int prec = in->prec;
+  void *U[2];
+  GX_TRY(op_gauge(op, prec, &U[0], &U[1]));
+  hipStream_t st = op->ctx->stream;
+  const Geom &g = op->g;
+  const void *one, *d, *b_meo = nullptr, *b_mooee = nullptr;
+  GX_TRY(op_coef(op, prec, Op::C_ONE, &one));
+  GX_TRY(op_coef(op, prec, Op::C_D, &d));
+  Field *t = nullptr;
+  if (op->kind == GX_MOBIUS) {
+    GX_TRY(op_band(op, prec, dag ? Op::S_MEOOEDAG5D : Op::S_MEOOE5D, &b_meo));
+    GX_TRY(op_band(op, prec, dag ? Op::S_MOOEEDAG : Op::S_MOOEE, &b_mooee));
+    if (!dag && !(t = op_tmp(op, prec, 3))) return GX_ENOMEM;
+  }
+  for (int cb = 0; cb < 2; cb++) {
+    const void *same = in->half(cb), *other = in->half(1 - cb);
+    if (t) {
+      GX_TRY(launch_band<T>(g, other, nullptr, t->data, b_meo, 0, nullptr, st));
+      other = t->data;
+    }
+    if (op->kind == GX_WILSON)
+      GX_TRY(launch_dhop_epi<T>(g, other, out->half(cb), U[cb], cb, dag, nullptr, st, 1, same, d, 0.0, 0, one));
+    else
+      GX_TRY(launch_dhop_epi<T>(g, other, out->half(cb), U[cb], cb, dag, nullptr, st, 3, same, dag ? b_meo : nullptr, 1.0,
+                                0, b_mooee));
+  }
   return GX_OK;
 }
 
@@ -825,6 +878,8 @@ static void scatter_from_device_layout(const Field *f, const T *stage, double *h
 }
 
 int apply_full_m(Op *op, Field *in, Field *out, int dag) {
+  if (tune_get(GX_TUNE_FUSED, in->prec))
+    return by_prec(in->prec, [&](auto t) { return full_m_fused<decltype(t)>(op, in, out, dag); });
   for (int cb = 0; cb < 2; cb++) {
     Field in_other = half_view(in, 1 - cb), in_same = half_view(in, cb), o = half_view(out, cb);
     GX_TRY(apply_meooe(op, &in_other, &o, dag));
@@ -1374,7 +1429,8 @@ int gx_op_footprint(gx_op op, size_t *bytes) {
   for (int p = 0; p < 2; p++)
     if (op->coef_dev[p]) b += (size_t)4 * op->g.Ls * (p == 0 ? 8 : 4);
   for (int p = 0; p < 3; p++) {
-    if (op->smat_dev[p]) b += (size_t)Op::S_COUNT * 2 * op->g.Ls * op->g.Ls * (p == GX_F64 ? 8 : 4);
+    if (op->smat_dev[p])
+      b += (size_t)Op::S_COUNT * (2 * op->g.Ls * op->g.Ls + 4 * op->g.Ls) * (p == GX_F64 ? 8 : 4);
     for (int i = 0; i < Op::kTmp; i++)
       if (op->tmp[p][i]) b += op->tmp[p][i]->bytes;
   }

@@ -186,7 +186,9 @@ struct Op {
     S_MEO5D_INV, S_INVDAG_MEODAG5D, S_COUNT
   };
   SMat smat[S_COUNT];
-  void *smat_dev[3] = {};       // [prec] device copy of all S_COUNT matrices (2*Ls*Ls each)
+  // [prec] device copy of all S_COUNT matrices (2*Ls*Ls each), then of their bands (4*Ls each; those of
+  // the dense ones are not used)
+  void *smat_dev[3] = {};
   // per precision temporaries (half fields): 0-3 operator compositions, 4-6 CG vectors,
   // 7-8 mixed-precision outer vectors, 10-14 the red-black solve's source and solution halves
   static constexpr int kTmp = 16;
@@ -194,9 +196,9 @@ struct Op {
   Field *full_tmp = nullptr;    // F64 full field: the red-black solve's residual check
   SolverWork *work = nullptr;   // solver state, created on the first solve
   uint64_t epoch = 0;           // bumped whenever links, mass or matrices change (invalidates graphs)
-  // Per-slice coefficients of the Schur operator, in FP64 (coef_dev[0]) and FP32 (coef_dev[1], also
-  // FP16 storage), 4 Ls values: [0, Ls) alpha_s and [Ls, 2 Ls) beta_s of the fused Mpc epilogue
-  // (Wilson -1/d_s, d_s with d_s = 4 + m_s; Cayley -1, 1), [2 Ls, 3 Ls) 1/d_s, [3 Ls, 4 Ls) d_s.
+  // Per-slice coefficients of the Wilson operators, in FP64 (coef_dev[0]) and FP32 (coef_dev[1], also
+  // FP16 storage), 4 Ls values with d_s = 4 + m_s: -1/d_s, d_s, 1/d_s, 1 (C_*)
+  enum { C_MINUS_INV = 0, C_D, C_INV, C_ONE };
   // slice_mass: Wilson per-slice masses m_s (empty: every slice has `mass`).
   std::vector<double> slice_mass;
   void *coef_dev[2] = {};
@@ -222,18 +224,20 @@ template <typename S>
 int launch_dhop(const Geom &g, const void *in, void *out, const void *U, int cb_out, int dag, const Gate *gate,
                 hipStream_t st);
 // hop with an epilogue: epi 0 out = hop; 1 out_s = alpha_s hop_s + beta_s phi_s with per-slice
-// coefficients coef (device, 2 Ls in T: alpha_s then beta_s); 2 out = alpha A(hop) [+ beta phi] with A
-// a per-chirality matrix applied across each site's s-row, block diagonal in groups of lb consecutive
-// slices (2*lb*lb in T; lb = 0: one group of Ls).  fz: reductions fused into the epilogue (HopFuse).
+// coefficients (device, Ls in T each: alpha in coef, beta in mat); 2 out = alpha A(hop) with A a
+// per-chirality matrix mat applied across each site's s-row, block diagonal in groups of lb consecutive
+// slices (2*lb*lb in T; lb = 0: one group of Ls); 3 out = alpha A(hop) + B(phi), A (dag; dag 0: A = 1)
+// and B two-band matrices (mat and coef hold their bands, 4*lb in T: op_band).  fz: reductions fused
+// into the epilogue (HopFuse).
 //
 // HopFuse, on Ls >= 2 where the tuned kernel is the 4-wave whole-site one or a general shape:
-//   r == nullptr, epi 1, dag 0: out as epi 1, and the per-tile slice sums of |out|^2 in npart;
-//   r != nullptr, epi 1 or 2 with phi, dag 1: r_s -= a[astride s] (the epilogue's result)_s and out
+//   r == nullptr, epi 1 or 3, dag 0: out as without, and the per-tile slice sums of |out|^2 in npart;
+//   r != nullptr, epi 1 or 3, dag 1: r_s -= a[astride s] (the epilogue's result)_s and out
 //   is NOT written; per-tile slice sums of |r_s|^2 in npart (a on the device: astride 1, one value
 //   per slice (multi-RHS); astride 0, one value (single-RHS CG)).
 // npart holds [tile][Ls] doubles, at most hop_norm_tiles(g.H4, g.Ls) tiles; *nparts = the tiles
-// written, or 0 when the kernel has no such epilogue: out is then written as plain epi 1 and the
-// caller reduces itself.
+// written, or 0 when the kernel has no such epilogue: out is then written and the caller reduces
+// itself.
 struct HopFuse {
   double *npart = nullptr;
   int64_t *nparts = nullptr;
@@ -243,7 +247,7 @@ struct HopFuse {
 };
 template <typename T>
 int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int cb_out, int dag, const Gate *gate,
-                    hipStream_t st, int epi, const void *phi, const void *mat, double alpha, double beta, int lb = 0,
+                    hipStream_t st, int epi, const void *phi, const void *mat, double alpha, int lb = 0,
                     const void *coef = nullptr, const HopFuse *fz = nullptr);
 // upper bound of the tiles of a norm-producing hop over H4 half sites of Ls slices (the 4-wave
 // kernel has 4 (64 / Ls) sites per tile, a general shape of W waves 64 W / Ls >= 64 / Ls), and the
@@ -263,14 +267,15 @@ int launch_fold_cg(Ctx *ctx, const double *npart, int64_t ntiles, int Ls, CGStat
 // out_e = c[s] in_e on the (h, s) entries of half fields (c: Ls values in the arithmetic type)
 template <typename S>
 int launch_scale_slices(const Geom &g, const void *in, void *out, const void *c, const Gate *gate, hipStream_t st);
-// out = A_chi(in) per chirality (+ phi if phi), mats = 2*lb*lb device matrix in T (groups as above)
+// out = A_chi(in) per chirality, mats = 2*lb*lb device matrix in T (groups as above)
 template <typename T>
-int launch_smat(const Geom &g, const void *in, const void *phi, void *out, const void *mats, const Gate *gate,
-                hipStream_t st, int lb = 0);
-// out = A(in) + beta phi and, if out2, out2 = C(in) from one read of in
+int launch_smat(const Geom &g, const void *in, void *out, const void *mats, const Gate *gate, hipStream_t st,
+                int lb = 0);
+// out = A(in) (+ phi if phi) with A a two-band matrix (op_band; dag: the adjoint operators' neighbours);
+// out may be phi, not in
 template <typename T>
-int launch_smat2(const Geom &g, const void *in, const void *phi, double beta, void *out, const void *mats, void *out2,
-                 const void *mats2, const Gate *gate, hipStream_t st, int lb = 0);
+int launch_band(const Geom &g, const void *in, const void *phi, void *out, const void *bands, int dag,
+                const Gate *gate, hipStream_t st);
 // z = a x + b y over nsites sites (stride sites per half; a, b real; y optional)
 template <typename S>
 int launch_axpby(int64_t nsites, int64_t stride, double a, const void *x, double b, const void *y, void *z,
@@ -388,7 +393,11 @@ bool same_geom(const Geom &a, const Geom &b);
 Field half_view(const Field *full, int cb);  // non-owning view of one checkerboard of a full field
 int op_prepare(Op *op, int prec);  // allocate lazily created resources of a precision ahead of capture
 int op_smat(Op *op, int prec, int which, const void **mats);
-int op_coef(Op *op, int prec, const void **coef);  // coef_dev of the arithmetic precision of prec
+// bands of operator which (S_MEOOE5D .. S_MOOEEDAG, S_M5D_OFF, S_M5DDAG_OFF): [chi][2][Ls], the diagonal
+// and the coefficient of the neighbour slice
+int op_band(Op *op, int prec, int which, const void **bands);
+// coefficients which (C_*) of the Ls slices, in the arithmetic precision of prec
+int op_coef(Op *op, int prec, int which, const void **coef);
 int op_upload_coefs(Op *op);                       // (re)build coef_dev from mass / slice_mass
 int reduce_read(Ctx *ctx, int slot, int n, double *out);
 

@@ -554,24 +554,41 @@ __device__ __forceinline__ void hop_site(cx<T> *acc, cx<T> *fa, cx<T> *fb, T &sa
 
 // Epilogue of the hop.  EPI 0: out = hop; 1: out_s = alpha_s hop_s + beta_s phi_s (per-slice
 // coefficients, so one multi-RHS launch can carry a different mass per right-hand side);
-// 2: out = alpha A(hop); 3: out = alpha A(hop) + beta phi, with A a per-chirality Ls x Ls matrix applied across the s-row
-// of each site from LDS and phi in the layout of out.  Whether phi is read is a template choice: a
+// 2: out = alpha A(hop) with A a dense per-chirality Ls x Ls matrix applied across the s-row of each
+// site from LDS; 3: out = alpha A(hop) + B(phi) with A (dag; without dag A = 1) and B two-band matrices
+// (slice_nbr) and phi in the layout of out.  Whether phi is read is a template choice: a
 // run-time null test inside the unrolled epilogue makes the compiler spill the whole hop.
 template <typename S>
 struct HopEpi {
   typedef typename Sto<S>::C T;
   const cx<S> *phi;
-  const T *mat;   // EPI 2, 3: [2][LS][LS], chirality 0 = spins 0,1
-  T alpha, beta;  // EPI 2, 3
-  const T *coef;  // EPI 1, 5, 6: per-slice coefficients, alpha_s = coef[s], beta_s = coef[LS + s]
-  // k_dhop only.  EPI 5: out as EPI 1, and the per-tile slice sums of |out|^2 in npart [tile][LS];
-  // EPI 6 (EPI 1 result) and 7 (EPI 3 result): rv_s -= acoef[astride s] (result)_s in place of
-  // storing out, per-tile slice sums of |rv_s|^2
+  const T *mat;   // EPI 1, 5, 6: beta_s; EPI 2: [2][LS][LS], chirality 0 = spins 0,1; EPI 3, 7 with dag:
+                  // A's bands [2][2][LS]
+  T alpha;        // EPI 2, 3
+  const T *coef;  // EPI 1, 5, 6: alpha_s; EPI 3, 7, 8: B's bands [2][2][LS]
+  // k_dhop and hop_tile.  EPI 5 (EPI 1 result) and 8 (EPI 3 result): out, and the per-tile slice sums of
+  // |out|^2 in npart [tile][LS]; EPI 6 (EPI 1 result) and 7 (EPI 3 result): rv_s -= acoef[astride s]
+  // (result)_s in place of storing out, per-tile slice sums of |rv_s|^2
   double *npart;
   cx<S> *rv;
   const double *acoef;
   int astride;
 };
+
+// The fifth-dimension operators but MooeeInv and its products have two bands per chirality: slice s
+// couples to itself and to one neighbour, s - 1 for chirality 0 and s + 1 for chirality 1 (the other
+// way round for the adjoints), cyclic within the LB slices of one operator.  Bands: [chi][2][LS] values,
+// the diagonal, then the coefficient of the neighbour slice_nbr(s, chi, dag).
+__host__ __device__ __forceinline__ uint32_t slice_nbr(uint32_t s, int chi, bool dag, uint32_t LB) {
+  return ((chi == 0) == dag) ? (s + 1 == LB ? 0 : s + 1) : (s == 0 ? LB - 1 : s - 1);
+}
+
+// LDS written by a wave and read by other lanes of the same wave
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // One lane per (4D half-site h, s): s fastest, 64/LS sites per wave, 4 waves per workgroup, so a
 // wave reads each neighbour's s-row contiguously and the lanes of one site share its links.
@@ -597,9 +614,9 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   constexpr int SPB = 4 * SPW;
   constexpr bool LDSU = (LS > 1) && (SPB * kLinkPad * sizeof(cx<T>) <= 40960);
   constexpr int NLINK = LDSU ? SPB * kLinkPad : 1;
-  constexpr bool MAT = EPI == 2 || EPI == 3 || EPI == 7, PHI = EPI == 1 || EPI == 3 || EPI >= 5;
+  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || EPI == 7 || EPI == 8, PHI = EPI == 1 || EPI == 5 || EPI == 6;
   constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7;
-  constexpr int NSTAGE = MAT ? 4 * 12 * 64 : 1;
+  constexpr int NSTAGE = MAT || BAND ? 4 * 12 * 64 : 1;
   __shared__ cx<T> lds[NLINK > NSTAGE ? NLINK : NSTAGE];  // links, then (MAT) the hop results
   const bool sweep = map == 4;  // blocked sweep: tiles are runs of the sweep order, XCD slabs
   const uint32_t tile = tile_of_block(blockIdx.x, gridDim.x, sweep ? 1 : map);
@@ -647,7 +664,7 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
-  if (!MAT && !NORM && !valid) return;
+  if (!MAT && !BAND && !NORM && !valid) return;
   const cx<T> *ul = lds + (LDSU ? lsb * kLinkPad : 0);
   cx<T> acc[12];
 #pragma unroll
@@ -679,15 +696,58 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
       }
     }
   }
-  if (EPI != 0 && valid) {
-    const bool pc = EPI == 1 || EPI == 5 || EPI == 6;
-    const T al = pc ? ep.coef[s] : ep.alpha, be = pc ? ep.coef[LS + s] : ep.beta;
+  if constexpr (BAND) {
+    // A's and B's neighbour slices come from the lanes of the same site, through LDS: 12 (24 with
+    // A) 16-byte reads per FP64 lane where a dense matrix takes 12 LS.  Computing B(phi) here instead of
+    // reading it also saves the pass that wrote it.
+    __syncthreads();  // every wave has finished reading links
+    cx<T> *stg = lds + w * 12 * 64;
+    const int row = ls * LS;
+    if constexpr (DAG) {
+#pragma unroll
+      for (int k = 0; k < 12; k++) stg[k * 64 + lane] = acc[k];
+      wave_sync();
+#pragma unroll
+      for (int chi = 0; chi < 2; chi++) {
+        const int n = row + (int)slice_nbr(s, chi, true, LS);
+        const T d = ep.alpha * ep.mat[2 * chi * LS + s], f = ep.alpha * ep.mat[(2 * chi + 1) * LS + s];
+#pragma unroll
+        for (int k = 6 * chi; k < 6 * chi + 6; k++) {
+          const cx<T> v = stg[k * 64 + (n & 63)];
+          acc[k] = {fma(f, v.r, d * acc[k].r), fma(f, v.i, d * acc[k].i)};
+        }
+      }
+      wave_sync();
+    } else {
+#pragma unroll
+      for (int k = 0; k < 12; k++) acc[k] = {ep.alpha * acc[k].r, ep.alpha * acc[k].i};
+    }
+    cx<T> fv[12];
+    load_site<S>(fv, ep.phi, valid ? o : h * LS);
+#pragma unroll
+    for (int k = 0; k < 12; k++) stg[k * 64 + lane] = fv[k];
+    wave_sync();
+#pragma unroll
+    for (int chi = 0; chi < 2; chi++) {
+      const int n = row + (int)slice_nbr(s, chi, DAG, LS);
+      const T d = ep.coef[2 * chi * LS + s], f = ep.coef[(2 * chi + 1) * LS + s];
+#pragma unroll
+      for (int k = 6 * chi; k < 6 * chi + 6; k++) {
+        const cx<T> v = stg[k * 64 + (n & 63)];
+        acc[k].r = fma(f, v.r, fma(d, fv[k].r, acc[k].r));
+        acc[k].i = fma(f, v.i, fma(d, fv[k].i, acc[k].i));
+      }
+    }
+    if (!NORM && !valid) return;
+  }
+  if (EPI != 0 && !BAND && valid) {
+    const T al = PHI ? ep.coef[s] : ep.alpha;
 #pragma unroll
     for (int k = 0; k < 12; k++) acc[k] = {al * acc[k].r, al * acc[k].i};
-    if (PHI) axpy_site<S>(acc, be, ep.phi, o);
+    if (PHI) axpy_site<S>(acc, ep.mat[s], ep.phi, o);
   }
   if constexpr (NORM) {
-    // per-slice |out|^2 (EPI 5) or |rv|^2 (EPI 6) of the tile's sites: lane sums in FP64, then the
+    // per-slice |out|^2 (EPI 5, 8) or |rv|^2 (EPI 6, 7) of the tile's sites: lane sums in FP64, then the
     // tile's sites in fixed order
     __shared__ double nsh[256];
     double nv = 0;
@@ -769,6 +829,48 @@ __device__ __forceinline__ void group_matrix(cx<T> *acc, cx<T> *stg, const T *ma
   }
 }
 
+// The band epilogue (k_dhop's EPI 3): acc = alpha A(acc) + B(phi entry o), one chirality at a time through
+// the 6 columns of EPB entries
+template <typename S, bool DAG>
+__device__ __forceinline__ void group_band(cx<typename Sto<S>::C> *acc, cx<typename Sto<S>::C> *stg, const HopEpi<S> &ep,
+                                           const GShape &sh, uint32_t t, uint32_t hl, uint32_t s, uint32_t epb,
+                                           uint32_t o) {
+  typedef typename Sto<S>::C T;
+  const uint32_t sg = s - fdiv(s, sh.fLB) * sh.LB, row = hl * sh.LS + (s - sg), LB = sh.LB;
+  cx<T> fv[12];
+  load_site<S>(fv, ep.phi, o);
+#pragma unroll
+  for (int chi = 0; chi < 2; chi++) {
+    const uint32_t n = row + slice_nbr(sg, chi, DAG, LB);
+    if constexpr (DAG) {
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 6; k++) stg[k * epb + t] = acc[6 * chi + k];
+      __syncthreads();
+      const T d = ep.alpha * ep.mat[2 * chi * LB + sg], f = ep.alpha * ep.mat[(2 * chi + 1) * LB + sg];
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        const cx<T> v = stg[k * epb + n];
+        acc[6 * chi + k] = {fma(f, v.r, d * acc[6 * chi + k].r), fma(f, v.i, d * acc[6 * chi + k].i)};
+      }
+    } else {
+#pragma unroll
+      for (int k = 6 * chi; k < 6 * chi + 6; k++) acc[k] = {ep.alpha * acc[k].r, ep.alpha * acc[k].i};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 6; k++) stg[k * epb + t] = fv[6 * chi + k];
+    __syncthreads();
+    const T d = ep.coef[2 * chi * LB + sg], f = ep.coef[(2 * chi + 1) * LB + sg];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      const cx<T> v = stg[k * epb + n];
+      acc[6 * chi + k].r = fma(f, v.r, fma(d, fv[6 * chi + k].r, acc[6 * chi + k].r));
+      acc[6 * chi + k].i = fma(f, v.i, fma(d, fv[6 * chi + k].i, acc[6 * chi + k].i));
+    }
+  }
+}
+
 // The hop of k_dhop (same legs, projectors, link staging and epilogues) in the general tile shape,
 // for one tile.  Every thread of the workgroup calls it (it synchronises the workgroup).
 template <typename S, bool DAG, int EPI>
@@ -777,7 +879,7 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
                                          bool sweep, int flags, const HopEpi<S> &ep, const GShape &sh,
                                          cx<typename Sto<S>::C> *lds) {
   typedef typename Sto<S>::C T;
-  constexpr bool MAT = EPI == 2 || EPI == 3 || EPI == 7, PHI = EPI == 1 || EPI == 3 || EPI >= 5;
+  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || EPI == 7 || EPI == 8, PHI = EPI == 1 || EPI == 5 || EPI == 6;
   constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7;
   const uint32_t H4 = (uint32_t)g.H4, LS = sh.LS, epb = blockDim.x;
   const uint32_t t = threadIdx.x;
@@ -809,16 +911,16 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
 #pragma unroll
   for (int k = 0; k < 12; k++) acc[k] = {0, 0};
   if (valid) hop_site<T, S, DAG, true, 0, true>(acc, fa, fb, sa, sb, in, U, lds + hl * kLinkPad, nb, LS, s, h, H4);
+  const uint32_t o = h * LS + s;
   if (MAT) group_matrix<T>(acc, lds, ep.mat, sh, t, hl, s, epb);
+  if constexpr (BAND) group_band<S, DAG>(acc, lds, ep, sh, t, hl, s, epb, o);
   double nv = 0;
   if (valid) {
-    const uint32_t o = h * LS + s;
-    if (EPI != 0) {
-      const bool pc = EPI == 1 || EPI == 5 || EPI == 6;
-      const T al = pc ? ep.coef[s] : ep.alpha, be = pc ? ep.coef[LS + s] : ep.beta;
+    if (EPI != 0 && !BAND) {
+      const T al = PHI ? ep.coef[s] : ep.alpha;
 #pragma unroll
       for (int k = 0; k < 12; k++) acc[k] = {al * acc[k].r, al * acc[k].i};
-      if (PHI) axpy_site<S>(acc, be, ep.phi, o);
+      if (PHI) axpy_site<S>(acc, ep.mat[s], ep.phi, o);
     }
     if (RUPD) {
       // the residual update in place of storing the result (k_dhop's EPI 6 / 7)
@@ -989,7 +1091,7 @@ __global__ void __launch_bounds__(rows_max_threads<S>())
                 int cb_out, const Gate *__restrict__ gate, uint32_t ntiles, int map, int flags, HopEpi<S> ep,
                 GShape sh, RowTile rt) {
   typedef typename Sto<S>::C T;
-  constexpr bool MAT = EPI >= 2, PHI = (EPI & 1) != 0;
+  constexpr bool MAT = EPI == 2, PHI = EPI == 1;
   if (gated(gate)) return;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const uint32_t nent = 4 * rt.RW;                 // entries of the tile (= threads)
@@ -1053,10 +1155,10 @@ __global__ void __launch_bounds__(rows_max_threads<S>())
   if (MAT) group_matrix<T>(acc, lin, ep.mat, sh, t, t / LS, s, blockDim.x);
   const uint32_t o = h * LS + s;
   if (EPI != 0) {
-    const T al = EPI == 1 ? ep.coef[s] : ep.alpha, be = EPI == 1 ? ep.coef[LS + s] : ep.beta;
+    const T al = PHI ? ep.coef[s] : ep.alpha;
 #pragma unroll
     for (int k = 0; k < 12; k++) acc[k] = {al * acc[k].r, al * acc[k].i};
-    if (PHI) axpy_site<S>(acc, be, ep.phi, o);
+    if (PHI) axpy_site<S>(acc, ep.mat[s], ep.phi, o);
   }
   store_site<S>(out, acc, o, (flags & 1) != 0);
 }
@@ -1173,7 +1275,7 @@ __global__ void __launch_bounds__(64 * kGenMaxWaves)
   if (!valid) return;
   const uint32_t o = h * LS + s;
   if (EPI != 0) {
-    const float al = ep.coef[s], be = ep.coef[LS + s];  // EPI 1
+    const float al = ep.coef[s], be = ep.mat[s];  // EPI 1
 #pragma unroll
     for (int k = 0; k < 12; k++) acc[k] = {al * acc[k].r, al * acc[k].i};
     if (PHI) axpy_site<float>(acc, be, ep.phi, o);
@@ -1181,13 +1283,11 @@ __global__ void __launch_bounds__(64 * kGenMaxWaves)
   store_site<float>(out, acc, o, (flags & 1) != 0);
 }
 
-// k_smat in the general tile shape: out = A(in) (+ beta phi) and optionally out2 = C(in), with A and
-// C block diagonal in groups of LB slices.
-template <typename S, bool OUT2, bool PHI>
+// k_smat in the general tile shape: out = A(in), A block diagonal in groups of LB slices.
+template <typename S>
 __global__ void __launch_bounds__(64 * kGenMaxWaves)
-    k_smat_g(const cx<S> *__restrict__ in, const cx<S> *__restrict__ phi, typename Sto<S>::C beta,
-             cx<S> *__restrict__ out, const typename Sto<S>::C *__restrict__ mats, cx<S> *__restrict__ out2,
-             const typename Sto<S>::C *__restrict__ mats2, uint32_t H4, const Gate *__restrict__ gate, GShape sh) {
+    k_smat_g(const cx<S> *__restrict__ in, cx<S> *__restrict__ out, const typename Sto<S>::C *__restrict__ mats,
+             uint32_t H4, const Gate *__restrict__ gate, GShape sh) {
   typedef typename Sto<S>::C T;
   if (gated(gate)) return;
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -1197,22 +1297,16 @@ __global__ void __launch_bounds__(64 * kGenMaxWaves)
   const uint32_t h = blockIdx.x * sh.SPB + hl;
   const bool valid = h < H4;
   const uint32_t o = h * LS + s;
-  cx<T> f[12], f2[12];
+  cx<T> f[12];
   if (valid) {
     load_site<S>(f, in, o);
   } else {
 #pragma unroll
     for (int k = 0; k < 12; k++) f[k] = {0, 0};
   }
-  if (OUT2)
-#pragma unroll
-    for (int k = 0; k < 12; k++) f2[k] = f[k];
   group_matrix<T>(f, lds, mats, sh, t, hl, s, epb);
-  if (OUT2) group_matrix<T>(f2, lds, mats2, sh, t, hl, s, epb);
   if (!valid) return;
-  if (PHI) axpy_site<S>(f, beta, phi, o);
   store_site<S>(out, f, o, false);
-  if (OUT2) store_site<S>(out2, f2, o, false);
 }
 
 // Waves per workgroup of the general kernels for extent LS (0: the templated kernels, -1: no
@@ -1286,12 +1380,12 @@ static GShape make_shape(int LS, int LB, int W) {
   M(1) M(2) M(3) M(4) M(5) M(6) M(7) M(8) M(9) M(10) M(11) M(12) M(13) M(14) M(15) M(16)
 #endif
 
-// epi: 0 out = hop; 1 out = alpha hop + beta phi; 2 out = alpha A(hop) [+ beta phi when phi is
-// given] (A: mat).  fz: reductions in the epilogue of the 4-wave whole-site kernel (HopFuse).
+// epi: 0 out = hop; 1 out = alpha hop + beta phi; 2 out = alpha A(hop); 3 out = alpha A(hop) + B(phi)
+// (HopEpi).  fz: reductions in the epilogue (HopFuse).
 template <typename S>
 int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int cb_out, int dag, const Gate *gate,
-                    hipStream_t st, int epi, const void *phi, const void *mat, double alpha, double beta, int lb,
-                    const void *coef, const HopFuse *fz) {
+                    hipStream_t st, int epi, const void *phi, const void *mat, double alpha, int lb, const void *coef,
+                    const HopFuse *fz) {
   typedef typename Sto<S>::C T;
   if (fz && fz->nparts) *fz->nparts = 0;
   if (lb <= 0) lb = g.Ls;
@@ -1299,15 +1393,15 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
     set_error("dhop: lattice too large for 32-bit site indexing");
     return GX_EINVAL;
   }
-  if (epi == 2 && g.Ls < 2) {
+  if (epi >= 2 && g.Ls < 2) {
     set_error("dhop: matrix epilogue needs Ls >= 2");
     return GX_EINVAL;
   }
-  if ((epi == 1 && (!phi || !coef)) || (epi == 2 && !mat)) {
+  if (((epi == 1 || epi == 3) && (!phi || !coef)) || ((epi == 1 || epi == 2 || (epi == 3 && dag)) && !mat)) {
     set_error("dhop: epilogue operand missing");
     return GX_EINVAL;
   }
-  const int kepi = (epi == 2 && phi) ? 3 : epi;
+  const int kepi = epi;
   int map = tune_get(GX_TUNE_DHOP_MAP, prec_of<S>());
   KGeom k = kgeom(g);
   if (map == 4) {
@@ -1329,7 +1423,7 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   const cx<S> *pin = (const cx<S> *)in;
   cx<S> *pout = (cx<S> *)out;
   const cx<S> *pU = (const cx<S> *)U;
-  HopEpi<S> ep{(const cx<S> *)phi, (const T *)mat, (T)alpha, (T)beta, (const T *)coef,
+  HopEpi<S> ep{(const cx<S> *)phi, (const T *)mat, (T)alpha, (const T *)coef,
                fz ? fz->npart : nullptr,  (cx<S> *)(fz ? fz->r : nullptr),  fz ? fz->a : nullptr,
                fz ? fz->astride : 1};
   if constexpr (std::is_same<S, float>::value) {
@@ -1359,7 +1453,7 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
     }
   }
   // row tiles: 2 x 2 rows of x in LDS (whole tiles only: Ly and Lz are even)
-  if (tune_get(GX_TUNE_DHOP_TILE, prec_of<S>()) && g.Ls % lb == 0) {
+  if (tune_get(GX_TUNE_DHOP_TILE, prec_of<S>()) && g.Ls % lb == 0 && kepi <= 2) {
     const uint32_t RW = (uint32_t)(k.Lxh * g.Ls), nthr = 4 * RW;
     const size_t lds = ((size_t)12 * nthr + (size_t)4 * k.Lxh * kLinkPad) * sizeof(cx<T>) +
                        (Sto<S>::H ? (size_t)nthr * sizeof(T) : 0);  // FP16: the entries' site scales
@@ -1425,8 +1519,7 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
       switch (kepi) {
         case 0: GX_ROWS_EPI(0); break;
         case 1: GX_ROWS_EPI(1); break;
-        case 2: GX_ROWS_EPI(2); break;
-        default: GX_ROWS_EPI(3); break;
+        default: GX_ROWS_EPI(2); break;
       }
 #undef GX_ROWS_EPI
 #undef GX_ROWS_GO
@@ -1454,13 +1547,14 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
                      ntiles, map, flags, ep, sh, blocks, persist)
 #define GX_DHOPG_EPI(EPI) \
   if (dag) GX_DHOPG_GO(true, EPI); else GX_DHOPG_GO(false, EPI)
-    // fused reductions: EPI 5 (kepi 1, dag 0), 6 (kepi 1, dag 1, r), 7 (kepi 3, dag 1, r); one
-    // workgroup per tile only (the persistent grid runs the separate passes)
-    const bool gnorm = !persist && fz && fz->npart && fz->nparts &&
-                       ((kepi == 1 && (fz->r ? (dag && fz->a) : !dag)) || (kepi == 3 && dag && fz->r && fz->a));
+    // fused reductions: EPI 5 (kepi 1, dag 0), 8 (kepi 3, dag 0), 6 (kepi 1, dag 1, r), 7 (kepi 3, dag
+    // 1, r); one workgroup per tile only (the persistent grid runs the separate passes)
+    const bool gnorm = !persist && fz && fz->npart && fz->nparts && (kepi == 1 || kepi == 3) &&
+                       (fz->r ? (dag && fz->a) : !dag);
     if (gnorm) {
       *fz->nparts = ntiles;
-      if (!dag) GX_DHOPG_GO(false, 5);
+      if (!dag && kepi == 3) GX_DHOPG_GO(false, 8);
+      else if (!dag) GX_DHOPG_GO(false, 5);
       else if (kepi == 3) GX_DHOPG_GO(true, 7);
       else GX_DHOPG_GO(true, 6);
     } else {
@@ -1480,9 +1574,9 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   const uint32_t ntiles = (uint32_t)((g.H4 + spb - 1) / spb);
   const uint32_t pad = (map == 1 || map == 4) ? 8 : (map == 2 ? 64 : (map == 3 ? 256 : 1));
   const uint32_t blocks = (ntiles + pad - 1) / pad * pad;
-  // EPI 5: kepi 1, dag 0; EPI 6: kepi 1, dag 1, r; EPI 7: kepi 3 (matrix and phi), dag 1, r
-  const bool norm = fz && fz->npart && fz->nparts && g.Ls >= 2 &&
-                    ((kepi == 1 && (fz->r ? (dag && fz->a) : !dag)) || (kepi == 3 && dag && fz->r && fz->a));
+  // EPI 5: kepi 1, dag 0; EPI 8: kepi 3, dag 0; EPI 6: kepi 1, dag 1, r; EPI 7: kepi 3, dag 1, r
+  const bool norm = fz && fz->npart && fz->nparts && g.Ls >= 2 && (kepi == 1 || kepi == 3) &&
+                    (fz->r ? (dag && fz->a) : !dag);
   if (norm) *fz->nparts = ntiles;
 #define GX_DHOP_GO(LS, DAG, PF, ORD, EPI)                                                                         \
   hipLaunchKernelGGL((k_dhop<S, LS, DAG, PF, ORD, EPI>), dim3(blocks), dim3(256), 0, st, pin, pout, pU, k, cb_out, \
@@ -1505,6 +1599,9 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
         } else if (dag) {                                        \
           if (pf) GX_DHOP_GO(LS, true, true, 0, 6);              \
           else GX_DHOP_GO(LS, true, false, 0, 6);                \
+        } else if (kepi == 3) {                                  \
+          if (pf) GX_DHOP_GO(LS, false, true, 0, 8);             \
+          else GX_DHOP_GO(LS, false, false, 0, 8);               \
         } else {                                                 \
           if (pf) GX_DHOP_GO(LS, false, true, 0, 5);             \
           else GX_DHOP_GO(LS, false, false, 0, 5);               \
@@ -1544,18 +1641,15 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
 template <typename S>
 int launch_dhop(const Geom &g, const void *in, void *out, const void *U, int cb_out, int dag, const Gate *gate,
                 hipStream_t st) {
-  return launch_dhop_epi<S>(g, in, out, U, cb_out, dag, gate, st, 0, nullptr, nullptr, 1.0, 0.0, 0, nullptr, nullptr);
+  return launch_dhop_epi<S>(g, in, out, U, cb_out, dag, gate, st, 0, nullptr, nullptr, 1.0, 0, nullptr, nullptr);
 }
 
-// out_s = sum_t A_chi[s][t] in_t (+ beta phi_s with PHI), and with OUT2 also
-// out2_s = sum_t C_chi[s][t] in_t from the same staged input.  mats: [2][LS][LS] in T,
-// chirality 0 = spins 0,1.  One lane per (h, s); the site's s-row is staged in LDS.
-template <typename S, int LS, bool OUT2, bool PHI>
-__global__ void __launch_bounds__(256) k_smat(const cx<S> *__restrict__ in, const cx<S> *__restrict__ phi,
-                                              typename Sto<S>::C beta, cx<S> *__restrict__ out,
-                                              const typename Sto<S>::C *__restrict__ mats, cx<S> *__restrict__ out2,
-                                              const typename Sto<S>::C *__restrict__ mats2, int64_t H4,
-                                              int64_t stride, const Gate *__restrict__ gate) {
+// out_s = sum_t A_chi[s][t] in_t.  mats: [2][LS][LS] in T, chirality 0 = spins 0,1.  One lane per
+// (h, s); the site's s-row is staged in LDS.
+template <typename S, int LS>
+__global__ void __launch_bounds__(256) k_smat(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
+                                              const typename Sto<S>::C *__restrict__ mats, int64_t H4,
+                                              const Gate *__restrict__ gate) {
   typedef typename Sto<S>::C T;
   if (gated(gate)) return;
   constexpr int SPW = 64 / LS;
@@ -1581,43 +1675,30 @@ __global__ void __launch_bounds__(256) k_smat(const cx<S> *__restrict__ in, cons
   }
   __syncthreads();
   if (!valid) return;
-  cx<T> acc[12], acc2[OUT2 ? 12 : 1];
+  cx<T> acc[12];
 #pragma unroll
   for (int k = 0; k < 12; k++) acc[k] = {0, 0};
-  if (OUT2)
-#pragma unroll
-    for (int k = 0; k < 12; k++) acc2[k] = {0, 0};
 #pragma unroll
   for (int t = 0; t < LS; t++) {
     const T ap = mats[s * LS + t], am = mats[LS * LS + s * LS + t];
-    T cp = 0, cm = 0;
-    if (OUT2) {
-      cp = mats2[s * LS + t];
-      cm = mats2[LS * LS + s * LS + t];
-    }
 #pragma unroll
     for (int k = 0; k < 12; k++) {
       const cx<T> v = lds[w][k][ls * LS + t];
       const T a = k < 6 ? ap : am;
       acc[k].r = fma(a, v.r, acc[k].r);
       acc[k].i = fma(a, v.i, acc[k].i);
-      if (OUT2) {
-        const T c = k < 6 ? cp : cm;
-        acc2[k].r = fma(c, v.r, acc2[k].r);
-        acc2[k].i = fma(c, v.i, acc2[k].i);
-      }
     }
   }
-  if (PHI) axpy_site<S>(acc, beta, phi, o);
   store_site<S>(out, acc, o, false);
-  if (OUT2) store_site<S>(out2, acc2, o, false);
 }
 
 template <typename S>
-int launch_smat2(const Geom &g, const void *in, const void *phi, double beta, void *out, const void *mats, void *out2,
-                 const void *mats2, const Gate *gate, hipStream_t st, int lb) {
+int launch_smat(const Geom &g, const void *in, void *out, const void *mats, const Gate *gate, hipStream_t st, int lb) {
   typedef typename Sto<S>::C T;
   if (lb <= 0) lb = g.Ls;
+  const cx<S> *pin = (const cx<S> *)in;
+  cx<S> *pout = (cx<S> *)out;
+  const T *pm = (const T *)mats;
   if (g.Ls > kMaxLs || lb != g.Ls) {
     const int W = general_waves(g.Ls, 0, sizeof(cx<T>), true, lb);
     if (W <= 0 || g.Ls % lb != 0) {
@@ -1627,43 +1708,16 @@ int launch_smat2(const Geom &g, const void *in, const void *phi, double beta, vo
     const GShape sh = make_shape(g.Ls, lb, W);
     const uint32_t blocks = (uint32_t)((g.H4 + sh.SPB - 1) / sh.SPB);
     const size_t lds = (size_t)6 * 64 * W * sizeof(cx<T>);
-    const cx<S> *pin = (const cx<S> *)in, *pphi = (const cx<S> *)phi;
-    cx<S> *pout = (cx<S> *)out, *pout2 = (cx<S> *)out2;
-    const T *pm = (const T *)mats, *pm2 = (const T *)mats2;
-#define GX_SMATG_GO(OUT2, PHI)                                                                                       \
-  hipLaunchKernelGGL((k_smat_g<S, OUT2, PHI>), dim3(blocks), dim3(64 * W), lds, st, pin, pphi, (T)beta, pout, pm,   \
-                     pout2, pm2, (uint32_t)g.H4, gate, sh)
-    if (out2) {
-      if (phi) GX_SMATG_GO(true, true);
-      else GX_SMATG_GO(true, false);
-    } else {
-      if (phi) GX_SMATG_GO(false, true);
-      else GX_SMATG_GO(false, false);
-    }
-#undef GX_SMATG_GO
+    hipLaunchKernelGGL((k_smat_g<S>), dim3(blocks), dim3(64 * W), lds, st, pin, pout, pm, (uint32_t)g.H4, gate, sh);
     GX_CHECK_HIP(hipGetLastError());
     return GX_OK;
   }
   const int spw = 64 / g.Ls;
   const int64_t waves = (g.H4 + spw - 1) / spw;
   const int64_t blocks = (waves * 64 + 255) / 256;
-  const int64_t stride = g.half_pad();
-  const cx<S> *pin = (const cx<S> *)in;
-  const cx<S> *pphi = (const cx<S> *)phi;
-  cx<S> *pout = (cx<S> *)out, *pout2 = (cx<S> *)out2;
-  const T *pm = (const T *)mats, *pm2 = (const T *)mats2;
-#define GX_SMAT_GO(LS, OUT2, PHI)                                                                           \
-  hipLaunchKernelGGL((k_smat<S, LS, OUT2, PHI>), dim3(blocks), dim3(256), 0, st, pin, pphi, (T)beta, pout, pm, \
-                     pout2, pm2, g.H4, stride, gate)
-#define GX_SMAT_CASE(LS)                    \
-  case LS:                                  \
-    if (out2) {                             \
-      if (phi) GX_SMAT_GO(LS, true, true);  \
-      else GX_SMAT_GO(LS, true, false);     \
-    } else {                                \
-      if (phi) GX_SMAT_GO(LS, false, true); \
-      else GX_SMAT_GO(LS, false, false);    \
-    }                                       \
+#define GX_SMAT_CASE(LS)                                                                                       \
+  case LS:                                                                                                     \
+    hipLaunchKernelGGL((k_smat<S, LS>), dim3(blocks), dim3(256), 0, st, pin, pout, pm, g.H4, gate);            \
     break;
   switch (g.Ls) {
     GX_LS_CASES(GX_SMAT_CASE)
@@ -1672,15 +1726,67 @@ int launch_smat2(const Geom &g, const void *in, const void *phi, double beta, vo
       return GX_EINVAL;
   }
 #undef GX_SMAT_CASE
-#undef GX_SMAT_GO
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
 
+// out = A(in) (+ phi with PHI) with A a two-band fifth-dimension matrix (slice_nbr; bands: [2][2][Ls]).
+// One thread per entry; its neighbour slices' halves are entries of the same or the next cache line that
+// the neighbouring lanes load as their own, so they come from the L1 and the pass moves what it must:
+// out may be phi, not in.
+template <typename S, bool PHI>
+__global__ void __launch_bounds__(256) k_band(const cx<S> *__restrict__ in, const cx<S> *phi, cx<S> *out,
+                                              const typename Sto<S>::C *__restrict__ bands, uint32_t nent, int dag,
+                                              const Gate *__restrict__ gate, FDiv fLS) {
+  typedef typename Sto<S>::C T;
+  constexpr int VW = Sto<S>::VW;
+  if (gated(gate)) return;
+  const uint32_t e = blockIdx.x * 256 + threadIdx.x, LS = fLS.d;
+  if (e >= nent) return;
+  const uint32_t s = e - fdiv(e, fLS) * LS;
+  cx<T> f[12], v[12];
+  load_site<S>(f, in, e);
+  T sc[2] = {(T)1, (T)1};
+#pragma unroll
+  for (int chi = 0; chi < 2; chi++) {
+    const uint32_t n = e - s + slice_nbr(s, chi, dag != 0, LS);
+    const cx<S> *q = in + bidx<S>(n, 0);
+    sc[chi] = site_scale<S>(in, n);
+    // groups that hold components of this chirality: 6 chi .. 6 chi + 5 (FP16's middle group holds both)
+#pragma unroll
+    for (int g = 6 * chi / VW; g <= (6 * chi + 5) / VW; g++) {
+      cx<T> w[VW];
+      load_group<S>(w, q, g);
+#pragma unroll
+      for (int c = 0; c < VW; c++)
+        if (g * VW + c >= 6 * chi && g * VW + c < 6 * chi + 6) v[g * VW + c] = w[c];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 12; k++) {
+    const int chi = k / 6;
+    const T d = bands[2 * chi * LS + s], b = bands[(2 * chi + 1) * LS + s] * sc[chi];
+    f[k] = {fma(b, v[k].r, d * f[k].r), fma(b, v[k].i, d * f[k].i)};
+  }
+  if (PHI) axpy_site<S>(f, (T)1, phi, e);
+  store_site<S>(out, f, e, false);
+}
+
 template <typename S>
-int launch_smat(const Geom &g, const void *in, const void *phi, void *out, const void *mats, const Gate *gate,
-                hipStream_t st, int lb) {
-  return launch_smat2<S>(g, in, phi, 1.0, out, mats, nullptr, nullptr, gate, st, lb);
+int launch_band(const Geom &g, const void *in, const void *phi, void *out, const void *bands, int dag, const Gate *gate,
+                hipStream_t st) {
+  typedef typename Sto<S>::C T;
+  const uint32_t nent = (uint32_t)(g.H4 * g.Ls), nb = (nent + 255) / 256;
+  const FDiv f = make_fdiv((uint32_t)g.Ls);
+  const cx<S> *pin = (const cx<S> *)in, *pphi = (const cx<S> *)phi;
+  cx<S> *pout = (cx<S> *)out;
+  const T *pb = (const T *)bands;
+  if (phi)
+    hipLaunchKernelGGL((k_band<S, true>), dim3(nb), dim3(256), 0, st, pin, pphi, pout, pb, nent, dag, gate, f);
+  else
+    hipLaunchKernelGGL((k_band<S, false>), dim3(nb), dim3(256), 0, st, pin, pphi, pout, pb, nent, dag, gate, f);
+  GX_CHECK_HIP(hipGetLastError());
+  return GX_OK;
 }
 
 // ---------------- BLAS1 ----------------
@@ -3202,14 +3308,13 @@ int launch_digest_slices(Ctx *ctx, const Geom &g, const void *full, int s0, int 
 
 #define GX_INST(S)                                                                                                 \
   template int launch_dhop_epi<S>(const Geom &, const void *, void *, const void *, int, int, const Gate *,       \
-                                  hipStream_t, int, const void *, const void *, double, double, int, const void *, \
+                                  hipStream_t, int, const void *, const void *, double, int, const void *,         \
                                   const HopFuse *);                                                                \
-  template int launch_smat2<S>(const Geom &, const void *, const void *, double, void *, const void *, void *,     \
-                               const void *, const Gate *, hipStream_t, int);                                    \
+  template int launch_band<S>(const Geom &, const void *, const void *, void *, const void *, int, const Gate *,   \
+                              hipStream_t);                                                                        \
   template int launch_dhop<S>(const Geom &, const void *, void *, const void *, int, int, const Gate *,           \
                               hipStream_t);                                                                        \
-  template int launch_smat<S>(const Geom &, const void *, const void *, void *, const void *, const Gate *,        \
-                              hipStream_t, int);                                                                   \
+  template int launch_smat<S>(const Geom &, const void *, void *, const void *, const Gate *, hipStream_t, int);   \
   template int launch_axpby<S>(int64_t, int64_t, double, const void *, double, const void *, void *, const Gate *, \
                                hipStream_t);                                                                       \
   template int launch_scale_slices<S>(const Geom &, const void *, void *, const void *, const Gate *, hipStream_t); \
