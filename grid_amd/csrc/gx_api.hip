@@ -30,9 +30,9 @@ static thread_local char g_err[1024] = "";
 
 // knob values per storage precision (GX_F64, GX_F32, GX_F16): a mixed-precision solve runs its
 // FP64 and its inner operators each with the launch shape tuned for that precision
-static int g_tune[3][GX_TUNE_COUNT] = {{1, 1, 1, 0, 1, 1, 0, 0, 0, 0},   // map pf nt order graph fused shape
-                                       {1, 1, 1, 0, 1, 1, 0, 0, 0, 0},   // persist mfma tile
-                                       {1, 1, 1, 0, 1, 1, 0, 0, 0, 0}};
+static int g_tune[3][GX_TUNE_COUNT] = {{4, 1, 1, 0, 1, 1, 0, 0, 0, 0},   // map pf nt order graph fused shape
+                                       {4, 1, 1, 0, 1, 1, 0, 0, 0, 0},   // persist mfma tile
+                                       {4, 1, 1, 0, 1, 1, 0, 0, 0, 0}};
 static int g_tune_version = 0;
 int tune_get(int knob, int prec) {
   if (knob < 0 || knob >= GX_TUNE_COUNT) return 0;

@@ -1402,7 +1402,14 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
     return GX_EINVAL;
   }
   const int kepi = epi;
+  // The blocked sweep (map 4, the default) keeps the t-neighbours' rows in the XCD's L2 between slices:
+  // FP64 16^4 x 16 53.6 us against 68.7 as plain slabs (map 1), FP32 32^3x64 x 12 893 against 1080, and
+  // the best or within 5% of the best map on every lattice tried with Ls > 1.  With one slice per site the
+  // links are three quarters of the traffic and streamed: runs of 8 tiles per XCD (map 2) take 326 us
+  // on 32^3 x 64 FP64, slabs 360, the sweep 416.  Such runs need thousands of tiles of 256 sites to
+  // spread evenly over the XCDs (8^4 would run on one); below that, slabs.
   int map = tune_get(GX_TUNE_DHOP_MAP, prec_of<S>());
+  if (map == 4 && g.Ls == 1) map = g.H4 >= (1 << 19) ? 2 : 1;
   KGeom k = kgeom(g);
   if (map == 4) {
     // blocks of Lxh x by x bz sites per t-slice with three t-slices of the input (and the links)
