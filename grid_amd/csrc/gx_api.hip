@@ -30,9 +30,9 @@ static thread_local char g_err[1024] = "";
 
 // knob values per storage precision (GX_F64, GX_F32, GX_F16): a mixed-precision solve runs its
 // FP64 and its inner operators each with the launch shape tuned for that precision
-static int g_tune[3][GX_TUNE_COUNT] = {{4, 1, 1, 0, 1, 1, 0, 0, 0, 0},   // map pf nt order graph fused shape
-                                       {4, 1, 1, 0, 1, 1, 0, 0, 0, 0},   // persist mfma tile
-                                       {4, 1, 1, 0, 1, 1, 0, 0, 0, 0}};
+static int g_tune[3][GX_TUNE_COUNT] = {{4, 1, 1, 0, 1, 1, 0, 0, 0, 0, 1},   // map pf nt order graph fused shape
+                                       {4, 1, 1, 0, 1, 1, 0, 0, 0, 0, 1},   // persist mfma tile split
+                                       {4, 1, 1, 0, 1, 1, 0, 0, 0, 0, 1}};
 static int g_tune_version = 0;
 int tune_get(int knob, int prec) {
   if (knob < 0 || knob >= GX_TUNE_COUNT) return 0;
@@ -760,6 +760,22 @@ static int full_m_fused(Op *op, Field *in, Field *out, int dag) {
     GX_TRY(op_band(op, prec, dag ? Op::S_MOOEEDAG : Op::S_MOOEE, &b_mooee));
     if (!dag && !(t = op_tmp(op, prec, 3))) return GX_ENOMEM;
   }
+  if (hop_split<T>(g)) {  // both checkerboards in one launch
+    const void *src[2] = {in->half(1), in->half(0)}, *same[2] = {in->half(0), in->half(1)}, *pu[2] = {U[0], U[1]};
+    void *po[2] = {out->half(0), out->half(1)};
+    if (t) {
+      Field *u = op_tmp(op, prec, 1);
+      if (!u) return GX_ENOMEM;
+      GX_TRY(launch_band<T>(g, src[0], nullptr, t->data, b_meo, 0, nullptr, st));
+      GX_TRY(launch_band<T>(g, src[1], nullptr, u->data, b_meo, 0, nullptr, st));
+      src[0] = t->data;
+      src[1] = u->data;
+    }
+    if (op->kind == GX_WILSON)
+      return launch_hop_split<T>(g, 0, 2, src, po, pu, same, dag, nullptr, st, 1, d, 0.0, one, nullptr);
+    return launch_hop_split<T>(g, 0, 2, src, po, pu, same, dag, nullptr, st, 3, dag ? b_meo : nullptr, 1.0, b_mooee,
+                               nullptr);
+  }
   for (int cb = 0; cb < 2; cb++) {
     const void *same = in->half(cb), *other = in->half(1 - cb);
     if (t) {
@@ -947,7 +963,8 @@ int gx_tune_set_prec(int knob, int prec, int value) {
   if (knob == GX_TUNE_DHOP_MAP) GX_REQUIRE(value >= 0 && value <= 4, GX_EINVAL, "tile map takes 0..4");
   else if (knob <= GX_TUNE_FUSED) GX_REQUIRE(value == 0 || value == 1, GX_EINVAL, "knob %d takes 0 or 1", knob);
   else if (knob == GX_TUNE_DHOP_SHAPE) GX_REQUIRE(value >= 0 && value <= 8, GX_EINVAL, "tile shape takes 0..8 waves");
-  else if (knob == GX_TUNE_DHOP_PERSIST || knob == GX_TUNE_DHOP_MFMA || knob == GX_TUNE_DHOP_TILE)
+  else if (knob == GX_TUNE_DHOP_PERSIST || knob == GX_TUNE_DHOP_MFMA || knob == GX_TUNE_DHOP_TILE ||
+           knob == GX_TUNE_DHOP_SPLIT)
     GX_REQUIRE(value == 0 || value == 1, GX_EINVAL, "knob %d takes 0 or 1", knob);
   g_tune[prec][knob] = value;
   g_tune_version++;
@@ -1545,6 +1562,17 @@ int gx_MooeeInvDag(gx_op op, gx_field in, gx_field out) {
 }
 int gx_Dhop(gx_op op, gx_field in, gx_field out, int dag) {
   GX_TRY(check_io(O(op), F(in), F(out), true));
+  void *U[2];
+  GX_TRY(op_gauge(O(op), in->prec, &U[0], &U[1]));
+  const int split = by_prec(in->prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g); });
+  if (split) {  // both checkerboards in one launch
+    const void *src[2] = {in->half(1), in->half(0)}, *pu[2] = {U[0], U[1]};
+    void *po[2] = {out->half(0), out->half(1)};
+    return by_prec(in->prec, [&](auto t) {
+      return launch_hop_split<decltype(t)>(op->g, 0, 2, src, po, pu, nullptr, dag, nullptr, op->ctx->stream, 0, nullptr,
+                                           1.0, nullptr, nullptr);
+    });
+  }
   for (int cb = 0; cb < 2; cb++) {
     Field i = half_view(F(in), 1 - cb), o = half_view(F(out), cb);
     GX_TRY(apply_dhop_half(O(op), &i, &o, cb, dag));

@@ -244,7 +244,25 @@ struct HopFuse {
   void *r = nullptr;
   const double *a = nullptr;
   int astride = 1;
+  // leg-per-wave kernel, single-RHS CG: a = c / d from the state cur and the nd partials of d (in place of
+  // *a, which has to be given all the same), left in nxt
+  const CGState *cur = nullptr;
+  CGState *nxt = nullptr;
+  const double *dpart = nullptr;
+  int nd = 0;
 };
+// Small lattices (hop_split) run the hop with one leg per wave, which launch_dhop_epi then does by
+// itself; ncb = 2 does both checkerboards cb and cb ^ 1 in one launch (operand j of each list).
+// Up to 32768 entries (H4 Ls) it is the faster in every precision (FP64 8^4: 8.6 -> 4.3 us, 8^4 x 8: 7.2 ->
+// 4.6, 8^4 x 16: 7.7 -> 6.5, 16^4: 13.6 -> 12.1); at 65536 the LDS round trip costs more than the latency it
+// hides (8^3 x 16 x 16: 9.5 -> 11.9).
+constexpr int64_t kSplitMax = 40960;
+template <typename S>
+bool hop_split(const Geom &g);
+template <typename S>
+int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], void *const out[2], const void *const U[2],
+                     const void *const phi[2], int dag, const Gate *gate, hipStream_t st, int epi, const void *mat,
+                     double alpha, const void *coef, const HopFuse *fz);
 template <typename T>
 int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int cb_out, int dag, const Gate *gate,
                     hipStream_t st, int epi, const void *phi, const void *mat, double alpha, int lb = 0,

@@ -129,6 +129,14 @@ __device__ __forceinline__ float mul_rounded(float a, float b) {
   return a * b;
 }
 
+// a * b as an FP32 product, then rounded to binary16: opaque in between, as the compiler takes one
+// v_fma_mix*_f16, which rounds once, in some kernels and not in others (every kernel stores the same bits)
+__device__ __forceinline__ half_t to_half(float a, float b) {
+  float p = a * b;
+  asm("" : "+v"(p));
+  return (half_t)p;
+}
+
 // The 12 components of entry i (FP16: multiplied by the site's scale), 12 / VW loads of 16 bytes.
 template <typename S, typename I>
 __device__ __forceinline__ void load_site(cx<typename Sto<S>::C> *f, const cx<S> *__restrict__ p, I i) {
@@ -197,8 +205,8 @@ __device__ __forceinline__ void store_site(cx<S> *__restrict__ p, const cx<typen
       f16x8 v;
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        v[2 * c] = (half_t)((a[4 * g + c].r * up) * inv);
-        v[2 * c + 1] = (half_t)((a[4 * g + c].i * up) * inv);
+        v[2 * c] = to_half(a[4 * g + c].r * up, inv);
+        v[2 * c + 1] = to_half(a[4 * g + c].i * up, inv);
       }
       *reinterpret_cast<f16x8 *>(q + g * kBlk * VW) = v;
     }
@@ -981,6 +989,283 @@ __global__ void __launch_bounds__(64 * kGenMaxWaves)
   }
 }
 
+// ---------------- hop with one leg per wave, for small lattices ----------------
+// What bounds a small lattice's hop is the serial chain of one lane: eight neighbours and eight links one
+// or two legs at a time, each a round trip to the L2 or beyond, on a handful of CUs.  Here a workgroup of 8
+// waves takes 64 / LS whole sites and wave w runs leg w of them, so all loads of a site are in flight at once
+// and eight times as many waves share them; the products meet in LDS, where waves 0..2 reconstruct one
+// colour each, in leg order, and run the epilogue on that colour's four spins.  The arithmetic and its
+// order are k_dhop's: the same bits.  Grid: tiles x 1 checkerboard, or x 2 for both in one launch
+// (checkerboard cb ^ blockIdx.y).
+template <typename S>
+struct SplitArgs {
+  const cx<S> *in[2], *U[2], *phi[2];
+  cx<S> *out[2];
+  int cb;
+  uint32_t LS, SPW;
+  FDiv fLS;
+  // RUPD in a single-RHS CG: a = c / d with c of the state cur and d the sum of nd partials, left in nxt
+  const CGState *cur;
+  CGState *nxt;
+  const double *dpart;
+  int nd;
+};
+
+// component k of entry e, without and with the FP16 site scale
+template <typename S>
+__device__ __forceinline__ cx<typename Sto<S>::C> load_comp_raw(const cx<S> *__restrict__ p, uint32_t e, int k) {
+  const cx<S> v = p[bidx<S>(e, 0) + (uint32_t)((k / Sto<S>::VW) * kBlk * Sto<S>::VW + k % Sto<S>::VW)];
+  return {(typename Sto<S>::C)v.r, (typename Sto<S>::C)v.i};
+}
+template <typename S>
+__device__ __forceinline__ cx<typename Sto<S>::C> load_comp(const cx<S> *__restrict__ p, uint32_t e, int k) {
+  const cx<typename Sto<S>::C> v = load_comp_raw<S>(p, e, k);
+  if constexpr (Sto<S>::H) {
+    const float sc = site_scale<S>(p, e);
+    return {mul_rounded(v.r, sc), mul_rounded(v.i, sc)};
+  }
+  return v;
+}
+
+// half-lattice index of neighbour P of half-site h (site_neighbours, one of the eight)
+template <int P>
+__device__ __forceinline__ uint32_t site_neighbour(const KGeom &g, uint32_t h, int cb_out) {
+  const uint32_t r1 = fdiv(h, g.fLxh), r2 = fdiv(r1, g.fL1), r3 = fdiv(r2, g.fL2);
+  const int xh = (int)(h - r1 * (uint32_t)g.Lxh), y = (int)(r1 - r2 * (uint32_t)g.L[1]);
+  const int z = (int)(r2 - r3 * (uint32_t)g.L[2]), t = (int)r3;
+  constexpr int MU = P & 3;
+  constexpr bool FWD = P < 4;
+  if (MU == 0) {
+    const int x = 2 * xh + ((cb_out + y + z + t) & 1);
+    const int xn = FWD ? (x + 1 == g.L[0] ? 0 : x + 1) : (x == 0 ? g.L[0] - 1 : x - 1);
+    return h - xh + (xn >> 1);
+  }
+  const int c = MU == 1 ? y : (MU == 2 ? z : t), L = g.L[MU];
+  const uint32_t st = (uint32_t)(MU == 1 ? g.sY : (MU == 2 ? g.sZ : g.sT));
+  if (FWD) return (c + 1 == L) ? h - (uint32_t)(L - 1) * st : h + st;
+  return (c == 0) ? h + (uint32_t)(L - 1) * st : h - st;
+}
+
+// leg LEG of one lane's site: the six link products (and FP16's site scale) into LDS
+template <typename S, bool DAG, int LEG>
+__device__ __forceinline__ void split_leg(const cx<S> *__restrict__ in, const cx<S> *__restrict__ U, const KGeom &g,
+                                          int cb_out, uint32_t h, uint32_t s, uint32_t LS, uint32_t lane,
+                                          cx<typename Sto<S>::C> *prod, typename Sto<S>::C *lsc) {
+  typedef typename Sto<S>::C T;
+  typedef LegSel<DAG, 0, LEG> L;
+  const uint32_t H4 = (uint32_t)g.H4;
+  cx<T> f[12], u[9], hs[6];
+  const T sc = load_site_raw<S>(f, in, site_neighbour<L::P>(g, h, cb_out) * LS + s);
+#pragma unroll
+  for (int k = 0; k < 9; k++) u[k] = ldc<S>(U, (uint32_t)(L::P * 9 + k) * H4 + h);
+  project<T, L::MU, L::PLUS>(f, hs);
+#pragma unroll
+  for (int r = 0; r < 3; r++) {
+    prod[((LEG * 2 + 0) * 3 + r) * 64 + lane] = su3_row<T>(u + 3 * r, hs);
+    prod[((LEG * 2 + 1) * 3 + r) * 64 + lane] = su3_row<T>(u + 3 * r, hs + 3);
+  }
+  if (Sto<S>::H) lsc[LEG * 64 + lane] = sc;
+}
+
+template <typename S, bool DAG, int LEG>
+__device__ __forceinline__ void split_recon(cx<typename Sto<S>::C> *a, const cx<typename Sto<S>::C> *prod,
+                                            const typename Sto<S>::C *lsc, uint32_t c, uint32_t lane) {
+  typedef LegSel<DAG, 0, LEG> L;
+  typedef typename Sto<S>::C T;
+  const cx<T> h0 = prod[((LEG * 2 + 0) * 3 + c) * 64 + lane], h1 = prod[((LEG * 2 + 1) * 3 + c) * 64 + lane];
+  if constexpr (Sto<S>::H) recon_colour_s<T, L::MU, L::PLUS>(a, 0, h0, h1, lsc[LEG * 64 + lane]);
+  else recon_colour<T, L::MU, L::PLUS>(a, 0, h0, h1);
+}
+
+__device__ __forceinline__ double wave_total(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+template <typename S, bool DAG, int EPI>
+__global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, const Gate *__restrict__ gate, HopEpi<S> ep) {
+  typedef typename Sto<S>::C T;
+  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || EPI == 7 || EPI == 8, PHI = EPI == 1 || EPI == 5 || EPI == 6;
+  constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7;
+  if (gated(gate)) return;
+  __shared__ cx<T> prod[8 * 6 * 64];
+  __shared__ T lsc[Sto<S>::H ? 8 * 64 : 1], smax[Sto<S>::H ? 3 * 64 : 1];
+  __shared__ double nsh[NORM ? 3 * 64 : 1], dsh[RUPD ? 8 : 1];
+  const uint32_t lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t LS = A.LS, ls = fdiv(lane, A.fLS), s = lane - ls * LS;
+  const uint32_t h0 = blockIdx.x * A.SPW, H4 = (uint32_t)g.H4, j = blockIdx.y;
+  const int cb = A.cb ^ (int)j;
+  const bool valid = ls < A.SPW && h0 + ls < H4;
+  const uint32_t h = valid ? h0 + ls : h0, o = h * LS + s;  // idle lanes: in-bounds addresses
+  double ds = 0;
+  if (RUPD && A.cur)
+    for (int i = threadIdx.x; i < A.nd; i += 512) ds += A.dpart[i];
+  switch (w) {
+#define GX_SPLIT_LEG(L)   case L: split_leg<S, DAG, L>(A.in[j], A.U[j], g, cb, h, s, LS, lane, prod, lsc); break;
+    GX_SPLIT_LEG(0) GX_SPLIT_LEG(1) GX_SPLIT_LEG(2) GX_SPLIT_LEG(3)
+    GX_SPLIT_LEG(4) GX_SPLIT_LEG(5) GX_SPLIT_LEG(6) GX_SPLIT_LEG(7)
+#undef GX_SPLIT_LEG
+  }
+  if (RUPD && A.cur) {
+    ds = wave_total(ds);
+    if (lane == 0) dsh[w] = ds;
+  }
+  // the epilogue's operands are loaded before the barrier: one colour c per wave
+  const uint32_t c = w;
+  const cx<S> *phi = A.phi[j];
+  cx<T> fv[4], rv[4];
+  T psc = (T)1;
+  if (c < 3) {
+    if (PHI) {
+      psc = site_scale<S>(phi, o);
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) fv[sp] = load_comp_raw<S>(phi, o, 3 * sp + c);
+    }
+    if (BAND)
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) fv[sp] = load_comp<S>(phi, o, 3 * sp + c);
+    if (RUPD)
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) rv[sp] = load_comp<S>(ep.rv, o, 3 * sp + c);
+  }
+  __syncthreads();
+  cx<T> a[12];  // a[3 sp]: spin sp
+#pragma unroll
+  for (int k = 0; k < 12; k++) a[k] = {0, 0};
+  double nv = 0;
+  if (c < 3) {
+    split_recon<S, DAG, 0>(a, prod, lsc, c, lane);
+    split_recon<S, DAG, 1>(a, prod, lsc, c, lane);
+    split_recon<S, DAG, 2>(a, prod, lsc, c, lane);
+    split_recon<S, DAG, 3>(a, prod, lsc, c, lane);
+    split_recon<S, DAG, 4>(a, prod, lsc, c, lane);
+    split_recon<S, DAG, 5>(a, prod, lsc, c, lane);
+    split_recon<S, DAG, 6>(a, prod, lsc, c, lane);
+    split_recon<S, DAG, 7>(a, prod, lsc, c, lane);
+    const uint32_t row = ls * LS;
+    // the four spins of this colour in the LDS slots that only this wave reads: stg(sp)[lane]
+    auto stg = [&](int sp) { return prod + (sp * 3 + c) * 64; };
+    if constexpr (MAT) {
+      wave_sync();
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) stg(sp)[lane] = a[3 * sp];
+      wave_sync();
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) a[3 * sp] = {0, 0};
+      const T *ap = ep.mat + s * LS, *am = ep.mat + LS * LS + s * LS;
+      for (uint32_t tt = 0; tt < LS; tt++) {
+        const T cp = ap[tt], cm = am[tt];
+#pragma unroll
+        for (int sp = 0; sp < 4; sp++) {
+          const cx<T> v = stg(sp)[(row + tt) & 63];
+          const T m = sp < 2 ? cp : cm;
+          a[3 * sp].r = fma(m, v.r, a[3 * sp].r);
+          a[3 * sp].i = fma(m, v.i, a[3 * sp].i);
+        }
+      }
+    }
+    if constexpr (BAND) {
+      uint32_t n[2];
+#pragma unroll
+      for (int chi = 0; chi < 2; chi++) n[chi] = (row + slice_nbr(s, chi, DAG, LS)) & 63;
+      if constexpr (DAG) {
+        wave_sync();
+#pragma unroll
+        for (int sp = 0; sp < 4; sp++) stg(sp)[lane] = a[3 * sp];
+        wave_sync();
+#pragma unroll
+        for (int sp = 0; sp < 4; sp++) {
+          const int chi = sp / 2;
+          const T d = ep.alpha * ep.mat[2 * chi * LS + s], f = ep.alpha * ep.mat[(2 * chi + 1) * LS + s];
+          const cx<T> v = stg(sp)[n[chi]];
+          a[3 * sp] = {fma(f, v.r, d * a[3 * sp].r), fma(f, v.i, d * a[3 * sp].i)};
+        }
+      } else {
+#pragma unroll
+        for (int sp = 0; sp < 4; sp++) a[3 * sp] = {ep.alpha * a[3 * sp].r, ep.alpha * a[3 * sp].i};
+      }
+      wave_sync();
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) stg(sp)[lane] = fv[sp];
+      wave_sync();
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) {
+        const int chi = sp / 2;
+        const T d = ep.coef[2 * chi * LS + s], f = ep.coef[(2 * chi + 1) * LS + s];
+        const cx<T> v = stg(sp)[n[chi]];
+        a[3 * sp].r = fma(f, v.r, fma(d, fv[sp].r, a[3 * sp].r));
+        a[3 * sp].i = fma(f, v.i, fma(d, fv[sp].i, a[3 * sp].i));
+      }
+    } else if constexpr (EPI != 0) {
+      const T al = PHI ? ep.coef[s] : ep.alpha;
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) a[3 * sp] = {al * a[3 * sp].r, al * a[3 * sp].i};
+      if (PHI) {
+        const T b = ep.mat[s] * psc;
+#pragma unroll
+        for (int sp = 0; sp < 4; sp++) {
+          a[3 * sp].r = fma(b, fv[sp].r, a[3 * sp].r);
+          a[3 * sp].i = fma(b, fv[sp].i, a[3 * sp].i);
+        }
+      }
+    }
+    if constexpr (RUPD) {
+      double av;
+      if (A.cur) {
+        double d = 0;
+        for (int i = 0; i < 8; i++) d += dsh[i];
+        av = A.cur->c / d;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          A.nxt->d = d;
+          A.nxt->a = av;
+        }
+      } else {
+        av = ep.acoef[ep.astride * s];
+      }
+      const T ra = (T)(-av);
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) a[3 * sp] = {fma(ra, a[3 * sp].r, rv[sp].r), fma(ra, a[3 * sp].i, rv[sp].i)};
+    }
+    if (NORM && valid)
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) nv += (double)fma(a[3 * sp].r, a[3 * sp].r, a[3 * sp].i * a[3 * sp].i);
+    if constexpr (Sto<S>::H) {
+      float m = 0.f;
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) m = fmaxf(m, fmaxf(fabsf(a[3 * sp].r), fabsf(a[3 * sp].i)));
+      smax[c * 64 + lane] = m;
+    }
+    if (NORM) nsh[c * 64 + lane] = nv;
+  }
+  if (NORM || Sto<S>::H) __syncthreads();
+  cx<S> *dst = RUPD ? ep.rv : A.out[j];
+  if (c < 3 && valid) {
+    T up = (T)1, inv = (T)1;
+    if constexpr (Sto<S>::H) {  // the site's scale, as store_site
+      const float m = fmaxf(smax[lane], fmaxf(smax[64 + lane], smax[128 + lane]));
+      const bool tiny = __builtin_expect(m > 0.f && m < FLT_MIN, 0);
+      up = tiny ? 0x1p64f : 1.f;
+      inv = m > 0.f ? 1.f / (m * up) : 0.f;
+      if (c == 0) *reinterpret_cast<float *>(dst + sidx<S>(o)) = m;
+    }
+#pragma unroll
+    for (int sp = 0; sp < 4; sp++) {
+      const int k = 3 * sp + c;
+      cx<S> v;
+      if constexpr (Sto<S>::H) v = {to_half(a[3 * sp].r * up, inv), to_half(a[3 * sp].i * up, inv)};
+      else v = a[3 * sp];
+      dst[bidx<S>(o, 0) + (uint32_t)((k / Sto<S>::VW) * kBlk * Sto<S>::VW + k % Sto<S>::VW)] = v;
+    }
+  }
+  if (NORM && threadIdx.x < LS) {
+    double v = 0;
+    for (uint32_t q = 0; q < A.SPW; q++)
+      for (int cc = 0; cc < 3; cc++) v += nsh[cc * 64 + q * LS + threadIdx.x];
+    ep.npart[(size_t)blockIdx.x * LS + threadIdx.x] = v;
+  }
+}
+
 // ---------------- hop with x, y and z legs from a tile of input rows in LDS ----------------
 // Tile = the 2 x 2 rows (y0, y0 + 1) x (z0, z0 + 1) of one t-slice, every x and every slice s:
 // RW = Lxh LS entries per row and 4 RW threads, thread t on row r = t / RW (y = y0 + (r & 1),
@@ -1380,6 +1665,72 @@ static GShape make_shape(int LS, int LB, int W) {
   M(1) M(2) M(3) M(4) M(5) M(6) M(7) M(8) M(9) M(10) M(11) M(12) M(13) M(14) M(15) M(16)
 #endif
 
+// The leg-per-wave kernel's range: up to kSplitMax entries per checkerboard
+template <typename S>
+bool hop_split(const Geom &g) {
+  const int p = prec_of<S>();
+  return tune_get(GX_TUNE_DHOP_SPLIT, p) && !tune_get(GX_TUNE_DHOP_SHAPE, p) && !tune_get(GX_TUNE_DHOP_MFMA, p) &&
+         !tune_get(GX_TUNE_DHOP_TILE, p) && g.Ls <= 64 && g.H4 * g.Ls <= kSplitMax;
+}
+
+template <typename S>
+int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], void *const out[2], const void *const U[2],
+                     const void *const phi[2], int dag, const Gate *gate, hipStream_t st, int epi, const void *mat,
+                     double alpha, const void *coef, const HopFuse *fz) {
+  typedef typename Sto<S>::C T;
+  SplitArgs<S> A{};
+  for (int j = 0; j < ncb; j++) {
+    A.in[j] = (const cx<S> *)in[j];
+    A.out[j] = (cx<S> *)out[j];
+    A.U[j] = (const cx<S> *)U[j];
+    A.phi[j] = (const cx<S> *)(phi ? phi[j] : nullptr);
+  }
+  A.cb = cb;
+  A.LS = (uint32_t)g.Ls;
+  A.SPW = 64u / A.LS;
+  A.fLS = make_fdiv(A.LS);
+  const uint32_t tiles = (uint32_t)((g.H4 + A.SPW - 1) / A.SPW);
+  const bool norm = fz && fz->npart && fz->nparts && (epi == 1 || epi == 3) && (fz->r ? (dag && fz->a) : !dag);
+  HopEpi<S> ep{nullptr, (const T *)mat, (T)alpha, (const T *)coef, nullptr, nullptr, nullptr, 1};
+  if (fz && fz->nparts) *fz->nparts = 0;
+  if (norm) {
+    ep.npart = fz->npart;
+    ep.rv = (cx<S> *)fz->r;
+    ep.acoef = fz->a;
+    ep.astride = fz->astride;
+    if (fz->r) {
+      A.cur = fz->cur;
+      A.nxt = fz->nxt;
+      A.dpart = fz->dpart;
+      A.nd = fz->nd;
+    }
+    *fz->nparts = tiles;
+  }
+  const KGeom k = kgeom(g);
+  const dim3 grid(tiles, ncb);
+#define GX_SPLIT_GO(DAG, EPI) hipLaunchKernelGGL((k_hop_split<S, DAG, EPI>), grid, dim3(512), 0, st, A, k, gate, ep)
+#define GX_SPLIT_EPI(EPI) \
+  if (dag) GX_SPLIT_GO(true, EPI); else GX_SPLIT_GO(false, EPI)
+  if (norm) {
+    if (!dag && epi == 3) GX_SPLIT_GO(false, 8);
+    else if (!dag) GX_SPLIT_GO(false, 5);
+    else if (!fz->r) return GX_EINVAL;
+    else if (epi == 3) GX_SPLIT_GO(true, 7);
+    else GX_SPLIT_GO(true, 6);
+  } else {
+    switch (epi) {
+      case 0: GX_SPLIT_EPI(0); break;
+      case 1: GX_SPLIT_EPI(1); break;
+      case 2: GX_SPLIT_EPI(2); break;
+      default: GX_SPLIT_EPI(3); break;
+    }
+  }
+#undef GX_SPLIT_EPI
+#undef GX_SPLIT_GO
+  GX_CHECK_HIP(hipGetLastError());
+  return GX_OK;
+}
+
 // epi: 0 out = hop; 1 out = alpha hop + beta phi; 2 out = alpha A(hop); 3 out = alpha A(hop) + B(phi)
 // (HopEpi).  fz: reductions in the epilogue (HopFuse).
 template <typename S>
@@ -1400,6 +1751,11 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   if (((epi == 1 || epi == 3) && (!phi || !coef)) || ((epi == 1 || epi == 2 || (epi == 3 && dag)) && !mat)) {
     set_error("dhop: epilogue operand missing");
     return GX_EINVAL;
+  }
+  if (lb == g.Ls && hop_split<S>(g)) {
+    const void *pi[2] = {in, nullptr}, *pu[2] = {U, nullptr}, *pp[2] = {phi, nullptr};
+    void *po[2] = {out, nullptr};
+    return launch_hop_split<S>(g, cb_out, 1, pi, po, pu, pp, dag, gate, st, epi, mat, alpha, coef, fz);
   }
   const int kepi = epi;
   // The blocked sweep (map 4, the default) keeps the t-neighbours' rows in the XCD's L2 between slices:
@@ -3317,6 +3673,10 @@ int launch_digest_slices(Ctx *ctx, const Geom &g, const void *full, int s0, int 
   template int launch_dhop_epi<S>(const Geom &, const void *, void *, const void *, int, int, const Gate *,       \
                                   hipStream_t, int, const void *, const void *, double, int, const void *,         \
                                   const HopFuse *);                                                                \
+  template bool hop_split<S>(const Geom &);                                                                        \
+  template int launch_hop_split<S>(const Geom &, int, int, const void *const[2], void *const[2],                   \
+                                   const void *const[2], const void *const[2], int, const Gate *, hipStream_t,    \
+                                   int, const void *, double, const void *, const HopFuse *);                      \
   template int launch_band<S>(const Geom &, const void *, const void *, void *, const void *, int, const Gate *,   \
                               hipStream_t);                                                                        \
   template int launch_dhop<S>(const Geom &, const void *, void *, const void *, int, int, const Gate *,           \

@@ -404,6 +404,7 @@ enum gx_tune_knob {
                                products on the matrix cores (v_mfma_f32_16x16x4f32) */
   GX_TUNE_DHOP_TILE = 9,    /* 1: hops in tiles of 2 x 2 rows of x staged in LDS (x, y and z legs from the tile;
                                when 4 Lx/2 Ls threads and the tile fit a workgroup) */
+  GX_TUNE_DHOP_SPLIT = 10,  /* 1 (default): hops of small lattices run one leg per wave (with SHAPE, MFMA and TILE at 0) */
   GX_TUNE_COUNT = 12
 };
 int gx_tune_set(int knob, int value);   /* every precision's value */
