@@ -230,7 +230,7 @@ int launch_dhop(const Geom &g, const void *in, void *out, const void *U, int cb_
 // and B two-band matrices (mat and coef hold their bands, 4*lb in T: op_band).  fz: reductions fused
 // into the epilogue (HopFuse).
 //
-// HopFuse, on Ls >= 2 where the tuned kernel is the 4-wave whole-site one or a general shape:
+// HopFuse, where the tuned kernel is the 4-wave whole-site one or a general shape:
 //   r == nullptr, epi 1 or 3, dag 0: out as without, and the per-tile slice sums of |out|^2 in npart;
 //   r != nullptr, epi 1 or 3, dag 1: r_s -= a[astride s] (the epilogue's result)_s and out
 //   is NOT written; per-tile slice sums of |r_s|^2 in npart (a on the device: astride 1, one value
@@ -244,6 +244,7 @@ struct HopFuse {
   void *r = nullptr;
   const double *a = nullptr;
   int astride = 1;
+  int total = 0;   // 1: npart holds one sum per tile, over its slices (single-RHS CG)
   // leg-per-wave kernel, single-RHS CG: a = c / d from the state cur and the nd partials of d (in place of
   // *a, which has to be given all the same), left in nxt
   const CGState *cur = nullptr;
@@ -279,9 +280,9 @@ size_t hop_norm_bytes(int64_t H4, int Ls);
 // multi-RHS CG state as the reduction of that mode: which 4 -> d_s, a_s; 2 -> cp_s, b_s,
 // convergence, k += 1
 int launch_fold_norms(Ctx *ctx, const double *npart, int64_t ntiles, int Ls, MrhsState *state, int which);
-// the same tile sums added over all slices into the single-RHS CG state: which 0 -> d, a; 1 -> cp, b,
+// tile sums over all slices (HopFuse total) into the single-RHS CG state: which 0 -> d, a; 1 -> cp, b,
 // stopping test, k += 1 (as the dot and axpy-norm finalisers)
-int launch_fold_cg(Ctx *ctx, const double *npart, int64_t ntiles, int Ls, CGState *state, int which);
+int launch_fold_cg(Ctx *ctx, const double *npart, int64_t ntiles, CGState *state, int which);
 // out_e = c[s] in_e on the (h, s) entries of half fields (c: Ls values in the arithmetic type)
 template <typename S>
 int launch_scale_slices(const Geom &g, const void *in, void *out, const void *c, const Gate *gate, hipStream_t st);
@@ -323,9 +324,13 @@ template <typename T>
 int launch_cg_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, void *r, const void *mmp, CGState *state);
 template <typename S>
 int launch_cg_update(Ctx *ctx, int64_t nsites, int64_t stride, void *psi, void *p, const void *r, CGState *state);
+// the update with the norm finaliser in it: np partials of |r|^2 and the state cur give the next state nxt
+template <typename S>
+int launch_cg_update_fin(Ctx *ctx, int64_t nsites, int64_t stride, void *psi, void *p, const void *r, const CGState *cur,
+                         CGState *nxt, const double *partial, int np);
 
 // Multi-RHS (slice) kernels; a half field is viewed as rows x Ls with s innermost.
-// mode 0: d_s = Re<x_s|y_s> -> a_s = c_s / d_s (state);   mode 4: d_s = |x_s|^2 -> a_s (state);
+// mode 4: d_s = |x_s|^2 -> a_s = c_s / d_s (state);
 // mode 2: x_s -= a_s y_s, cp_s = |x_s|^2 -> b_s, convergence, k += 1 (state);   mode 1: out_s = |x_s|^2;
 // mode 3: z_s = y_s - x_s, out_s = |z_s|^2
 template <typename T>

@@ -581,7 +581,24 @@ struct HopEpi {
   cx<S> *rv;
   const double *acoef;
   int astride;
+  int total;      // npart holds one sum per tile, over its slices
 };
+
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// a tile's slice sums v (thread s < LS <= 64 of the tile's first wave; zero on its other lanes) to npart
+__device__ __forceinline__ void write_norms(double *npart, uint32_t tile, uint32_t LS, double v, int total) {
+  if (total) {
+    v = wave_sum(v);
+    if (threadIdx.x == 0) npart[tile] = v;
+  } else if (threadIdx.x < LS) {
+    npart[(size_t)tile * LS + threadIdx.x] = v;
+  }
+}
 
 // The fifth-dimension operators but MooeeInv and its products have two bands per chirality: slice s
 // couples to itself and to one neighbour, s - 1 for chirality 0 and s + 1 for chirality 1 (the other
@@ -778,11 +795,12 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
     }
     nsh[threadIdx.x] = nv;
     __syncthreads();
-    if (threadIdx.x < LS) {
+    if (threadIdx.x < 64) {
       double v = 0;
-      for (int ww = 0; ww < 4; ww++)
-        for (int j = 0; j < SPW; j++) v += nsh[ww * 64 + j * LS + threadIdx.x];
-      ep.npart[(size_t)tile * LS + threadIdx.x] = v;
+      if (threadIdx.x < LS)
+        for (int ww = 0; ww < 4; ww++)
+          for (int j = 0; j < SPW; j++) v += nsh[ww * 64 + j * LS + threadIdx.x];
+      write_norms(ep.npart, tile, LS, v, ep.total);
     }
     return;
   }
@@ -954,10 +972,11 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
     __shared__ double nsh[64 * kGenMaxWaves];
     nsh[t] = nv;
     __syncthreads();
-    if (t < LS) {
+    if (t < 64) {
       double v = 0;
-      for (uint32_t j = 0; j < sh.SPB; j++) v += nsh[j * LS + t];
-      ep.npart[(size_t)tile * LS + t] = v;
+      if (t < LS)
+        for (uint32_t j = 0; j < sh.SPB; j++) v += nsh[j * LS + t];
+      write_norms(ep.npart, tile, LS, v, ep.total);
     }
   }
 }
@@ -1077,12 +1096,6 @@ __device__ __forceinline__ void split_recon(cx<typename Sto<S>::C> *a, const cx<
   else recon_colour<T, L::MU, L::PLUS>(a, 0, h0, h1);
 }
 
-__device__ __forceinline__ double wave_total(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
 template <typename S, bool DAG, int EPI>
 __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, const Gate *__restrict__ gate, HopEpi<S> ep) {
   typedef typename Sto<S>::C T;
@@ -1108,7 +1121,7 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
 #undef GX_SPLIT_LEG
   }
   if (RUPD && A.cur) {
-    ds = wave_total(ds);
+    ds = wave_sum(ds);
     if (lane == 0) dsh[w] = ds;
   }
   // the epilogue's operands are loaded before the barrier: one colour c per wave
@@ -1258,11 +1271,12 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
       dst[bidx<S>(o, 0) + (uint32_t)((k / Sto<S>::VW) * kBlk * Sto<S>::VW + k % Sto<S>::VW)] = v;
     }
   }
-  if (NORM && threadIdx.x < LS) {
+  if (NORM && threadIdx.x < 64) {
     double v = 0;
-    for (uint32_t q = 0; q < A.SPW; q++)
-      for (int cc = 0; cc < 3; cc++) v += nsh[cc * 64 + q * LS + threadIdx.x];
-    ep.npart[(size_t)blockIdx.x * LS + threadIdx.x] = v;
+    if (threadIdx.x < LS)
+      for (uint32_t q = 0; q < A.SPW; q++)
+        for (int cc = 0; cc < 3; cc++) v += nsh[cc * 64 + q * LS + threadIdx.x];
+    write_norms(ep.npart, blockIdx.x, LS, v, ep.total);
   }
 }
 
@@ -1691,7 +1705,7 @@ int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], vo
   A.fLS = make_fdiv(A.LS);
   const uint32_t tiles = (uint32_t)((g.H4 + A.SPW - 1) / A.SPW);
   const bool norm = fz && fz->npart && fz->nparts && (epi == 1 || epi == 3) && (fz->r ? (dag && fz->a) : !dag);
-  HopEpi<S> ep{nullptr, (const T *)mat, (T)alpha, (const T *)coef, nullptr, nullptr, nullptr, 1};
+  HopEpi<S> ep{nullptr, (const T *)mat, (T)alpha, (const T *)coef, nullptr, nullptr, nullptr, 1, fz ? fz->total : 0};
   if (fz && fz->nparts) *fz->nparts = 0;
   if (norm) {
     ep.npart = fz->npart;
@@ -1788,7 +1802,7 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   const cx<S> *pU = (const cx<S> *)U;
   HopEpi<S> ep{(const cx<S> *)phi, (const T *)mat, (T)alpha, (const T *)coef,
                fz ? fz->npart : nullptr,  (cx<S> *)(fz ? fz->r : nullptr),  fz ? fz->a : nullptr,
-               fz ? fz->astride : 1};
+               fz ? fz->astride : 1,  fz ? fz->total : 0};
   if constexpr (std::is_same<S, float>::value) {
     // the link products on the matrix cores: FP32 multi-RHS (Wilson, no matrix epilogue), Ls <= 16
     if (tune_get(GX_TUNE_DHOP_MFMA, prec_of<S>()) && kepi <= 1 && g.Ls >= 2 && g.Ls <= 16 && lb == g.Ls) {
@@ -1938,8 +1952,7 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   const uint32_t pad = (map == 1 || map == 4) ? 8 : (map == 2 ? 64 : (map == 3 ? 256 : 1));
   const uint32_t blocks = (ntiles + pad - 1) / pad * pad;
   // EPI 5: kepi 1, dag 0; EPI 8: kepi 3, dag 0; EPI 6: kepi 1, dag 1, r; EPI 7: kepi 3, dag 1, r
-  const bool norm = fz && fz->npart && fz->nparts && g.Ls >= 2 && (kepi == 1 || kepi == 3) &&
-                    (fz->r ? (dag && fz->a) : !dag);
+  const bool norm = fz && fz->npart && fz->nparts && (kepi == 1 || kepi == 3) && (fz->r ? (dag && fz->a) : !dag);
   if (norm) *fz->nparts = ntiles;
 #define GX_DHOP_GO(LS, DAG, PF, ORD, EPI)                                                                         \
   hipLaunchKernelGGL((k_dhop<S, LS, DAG, PF, ORD, EPI>), dim3(blocks), dim3(256), 0, st, pin, pout, pU, k, cb_out, \
@@ -1954,21 +1967,23 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   }
 #define GX_DHOP_CASE(LS)                                         \
   case LS:                                                       \
-    if (norm) {                                                  \
+    if (norm && kepi == 3) {                                     \
       if constexpr (LS >= 2) {                                   \
-        if (dag && kepi == 3) {                                  \
+        if (dag) {                                               \
           if (pf) GX_DHOP_GO(LS, true, true, 0, 7);              \
           else GX_DHOP_GO(LS, true, false, 0, 7);                \
-        } else if (dag) {                                        \
-          if (pf) GX_DHOP_GO(LS, true, true, 0, 6);              \
-          else GX_DHOP_GO(LS, true, false, 0, 6);                \
-        } else if (kepi == 3) {                                  \
+        } else {                                                 \
           if (pf) GX_DHOP_GO(LS, false, true, 0, 8);             \
           else GX_DHOP_GO(LS, false, false, 0, 8);               \
-        } else {                                                 \
-          if (pf) GX_DHOP_GO(LS, false, true, 0, 5);             \
-          else GX_DHOP_GO(LS, false, false, 0, 5);               \
         }                                                        \
+      }                                                          \
+    } else if (norm) {                                           \
+      if (dag) {                                                 \
+        if (pf) GX_DHOP_GO(LS, true, true, 0, 6);                \
+        else GX_DHOP_GO(LS, true, false, 0, 6);                  \
+      } else {                                                   \
+        if (pf) GX_DHOP_GO(LS, false, true, 0, 5);               \
+        else GX_DHOP_GO(LS, false, false, 0, 5);                 \
       }                                                          \
     } else if (kepi == 1) {                                      \
       GX_DHOP_CASE_O(LS, 0, 1)                                   \
@@ -2305,12 +2320,6 @@ int launch_convert_site(int64_t nsites, int64_t stride, const void *in, void *ou
 // boundary makes the partials visible to the second kernel, so no device-scope fence or atomic
 // is needed (on a multi-XCD part such a fence writes back the XCD's L2).  The grid size depends
 // only on the problem size, so results are bitwise reproducible.
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double (*sh)[4]) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -2488,37 +2497,50 @@ __global__ void __launch_bounds__(256) k_cg_axpy_norm(int64_t nsites, int64_t st
   write_partial<1>(v, partial);
 }
 
+// the scalars and stopping tests that follow from cp = |r|^2 of an iteration (all but k)
+__device__ __forceinline__ void cg_advance(CGState &st, double cp) {
+  st.cprev = st.c;
+  st.b = cp / st.c;
+  st.cp = cp;
+  st.c = cp;
+  if (st.delta > 0 && cp > st.maxres) st.maxres = cp;
+  if (st.k_conv != INT_MAX) return;
+  if (cp <= st.rsq) {
+    st.k_conv = st.k;
+  } else if (st.delta > 0 && cp < st.delta * st.maxres) {
+    st.ru = 1;
+    st.k_conv = st.k;
+  } else if (st.fbtol > 0 && cp < st.fbtol) {
+    st.ru = 2;
+    st.k_conv = st.k;
+  }
+}
+
 // which = 0: d = sum, a = c / d.   which = 1: cp = sum, b = cp / c, c = cp, convergence test.
 // The which = 1 finaliser advances k in every iteration, also once the solve has stopped, so the
 // gate of the following solution update (k-1) closes after the last real iteration.
-static __global__ void __launch_bounds__(256) k_cg_fin(const double *partial, int nparts, CGState *st, int which) {
+// One workgroup of 1024 threads takes the partials (up to a hop's tile sums) in a fixed order.
+static __global__ void __launch_bounds__(1024) k_cg_fin(const double *partial, int nparts, CGState *st, int which) {
   const bool skip = gated(st);
   if (skip && which == 0) return;
-  __shared__ double sh[1][4];
-  double v[1] = {0};
-  if (!skip) sum_partials<1>(v, partial, nparts, sh);
+  __shared__ double sh[16];
+  double v = 0;
+  if (!skip) {
+    for (int b = threadIdx.x; b < nparts; b += 1024) v += partial[b];
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+  }
   if (threadIdx.x == 0) {
+    if (!skip) {
+      v = 0;
+      for (int i = 0; i < 16; i++) v += sh[i];
+    }
     if (which == 0) {
-      st->d = v[0];
+      st->d = v;
       st->a = st->c / st->d;
     } else {
-      if (!skip) {
-        const double cp = v[0];
-        st->cprev = st->c;
-        st->b = cp / st->c;
-        st->cp = cp;
-        st->c = cp;
-        if (st->delta > 0 && cp > st->maxres) st->maxres = cp;
-        if (cp <= st->rsq && st->k_conv == INT_MAX) {
-          st->k_conv = st->k;
-        } else if (st->delta > 0 && cp < st->delta * st->maxres && st->k_conv == INT_MAX) {
-          st->ru = 1;
-          st->k_conv = st->k;
-        } else if (st->fbtol > 0 && cp < st->fbtol && st->k_conv == INT_MAX) {
-          st->ru = 2;
-          st->k_conv = st->k;
-        }
-      }
+      if (!skip) cg_advance(*st, v);
       st->k = st->k + 1;
     }
   }
@@ -2526,13 +2548,10 @@ static __global__ void __launch_bounds__(256) k_cg_fin(const double *partial, in
 
 // psi = a p + psi; p = b p + r  (FP64/FP32 per entry, FP16 per site)
 template <typename S>
-__global__ void __launch_bounds__(256) k_cg_update(int64_t nsites, int64_t stride, cx<S> *__restrict__ psi,
-                                                   cx<S> *__restrict__ p, const cx<S> *__restrict__ r,
-                                                   const CGState *st) {
+__device__ __forceinline__ void cg_update(int64_t nsites, int64_t stride, cx<S> *__restrict__ psi,
+                                          cx<S> *__restrict__ p, const cx<S> *__restrict__ r, typename Sto<S>::C a,
+                                          typename Sto<S>::C b, bool keep_p) {
   typedef typename Sto<S>::C T;
-  if (gated_prev(st)) return;
-  const T a = (T)st->a, b = (T)st->b;
-  const bool keep_p = st->ru == 1;  // reliable update pending: the host forms the new p
   if constexpr (!Sto<S>::H) {
     // one 16-byte group (VW complex numbers) per thread and step
     constexpr int VW = Sto<S>::VW;
@@ -2576,11 +2595,65 @@ __global__ void __launch_bounds__(256) k_cg_update(int64_t nsites, int64_t strid
 }
 
 template <typename S>
+__global__ void __launch_bounds__(256) k_cg_update(int64_t nsites, int64_t stride, cx<S> *__restrict__ psi,
+                                                   cx<S> *__restrict__ p, const cx<S> *__restrict__ r,
+                                                   const CGState *st) {
+  typedef typename Sto<S>::C T;
+  if (gated_prev(st)) return;
+  // ru: reliable update pending, the host forms the new p
+  cg_update<S>(nsites, stride, psi, p, r, (T)st->a, (T)st->b, st->ru == 1);
+}
+
+// The same with the norm finaliser folded in, for lattices whose iteration is launch latency: every
+// workgroup adds the np partials of |r|^2 in the same order and takes b and the stopping test from the state
+// cur (a and d of this iteration are in nxt already); the first one leaves the next state in nxt.
+template <typename S>
+__global__ void __launch_bounds__(256) k_cg_update_fin(int64_t nsites, int64_t stride, cx<S> *__restrict__ psi,
+                                                       cx<S> *__restrict__ p, const cx<S> *__restrict__ r,
+                                                       const CGState *cur, CGState *nxt, const double *partial, int np) {
+  typedef typename Sto<S>::C T;
+  const bool skip = gated(cur), first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (skip && !first) return;
+  CGState st = *cur;
+  if (skip) {
+    st.k++;
+    *nxt = st;
+    return;
+  }
+  __shared__ double sh[4];
+  double v = 0;
+  for (int b = threadIdx.x; b < np; b += 256) v += partial[b];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  st.a = nxt->a;
+  st.d = nxt->d;
+  cg_advance(st, (sh[0] + sh[1]) + (sh[2] + sh[3]));
+  const T a = (T)st.a, b = (T)st.b;
+  const bool keep_p = st.ru == 1;
+  if (first) {
+    st.k++;
+    *nxt = st;
+  }
+  cg_update<S>(nsites, stride, psi, p, r, a, b, keep_p);
+}
+
+template <typename S>
+int launch_cg_update_fin(Ctx *ctx, int64_t nsites, int64_t stride, void *psi, void *p, const void *r, const CGState *cur,
+                         CGState *nxt, const double *partial, int np) {
+  const int64_t work = Sto<S>::H ? nsites : 12 * nsites / Sto<S>::VW;
+  hipLaunchKernelGGL((k_cg_update_fin<S>), dim3(stream_blocks(work)), dim3(256), 0, ctx->stream, nsites, stride,
+                     (cx<S> *)psi, (cx<S> *)p, (const cx<S> *)r, cur, nxt, partial, np);
+  GX_CHECK_HIP(hipGetLastError());
+  return GX_OK;
+}
+
+template <typename S>
 int launch_cg_dot(Ctx *ctx, int64_t nsites, int64_t stride, const void *p, const void *mmp, CGState *state) {
   const int nb = red_blocks(nsites);
   hipLaunchKernelGGL((k_cg_dot<S>), dim3(nb), dim3(256), 0, ctx->stream, nsites, stride, (const cx<S> *)p,
                      (const cx<S> *)mmp, (const CGState *)state, ctx->red_partial);
-  hipLaunchKernelGGL(k_cg_fin, dim3(1), dim3(256), 0, ctx->stream, (const double *)ctx->red_partial, nb, state, 0);
+  hipLaunchKernelGGL(k_cg_fin, dim3(1), dim3(1024), 0, ctx->stream, (const double *)ctx->red_partial, nb, state, 0);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
@@ -2589,7 +2662,7 @@ int launch_cg_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, void *r, const
   const int nb = red_blocks(nsites);
   hipLaunchKernelGGL((k_cg_axpy_norm<S>), dim3(nb), dim3(256), 0, ctx->stream, nsites, stride, (cx<S> *)r,
                      (const cx<S> *)mmp, (const CGState *)state, ctx->red_partial);
-  hipLaunchKernelGGL(k_cg_fin, dim3(1), dim3(256), 0, ctx->stream, (const double *)ctx->red_partial, nb, state, 1);
+  hipLaunchKernelGGL(k_cg_fin, dim3(1), dim3(1024), 0, ctx->stream, (const double *)ctx->red_partial, nb, state, 1);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
@@ -2617,7 +2690,7 @@ __global__ void __launch_bounds__(256) k_mrhs_reduce(int64_t H4, int Ls, cx<S> *
                                                      const cx<S> *__restrict__ y, cx<S> *__restrict__ z,
                                                      const MrhsState *st, double *partial) {
   typedef typename Sto<S>::C T;
-  if ((MODE == 0 || MODE == 2 || MODE == 4) && mgated(st)) return;
+  if ((MODE == 2 || MODE == 4) && mgated(st)) return;
   __shared__ double sh[256];
   const int rpb = 256 / Ls;
   const int s = threadIdx.x % Ls;
@@ -2632,9 +2705,7 @@ __global__ void __launch_bounds__(256) k_mrhs_reduce(int64_t H4, int Ls, cx<S> *
       if (MODE != 1 && MODE != 4) load_site<S>(yv, y, e);
 #pragma unroll
       for (int k = 0; k < 12; k++) {
-        if (MODE == 0) {
-          acc += (double)fma(xv[k].r, yv[k].r, xv[k].i * yv[k].i);
-        } else if (MODE == 1 || MODE == 4) {
+        if (MODE == 1 || MODE == 4) {
           acc += (double)fma(xv[k].r, xv[k].r, xv[k].i * xv[k].i);
         } else if (MODE == 2) {
           xv[k] = {fma(a, yv[k].r, xv[k].r), fma(a, yv[k].i, xv[k].i)};
@@ -2657,14 +2728,13 @@ __global__ void __launch_bounds__(256) k_mrhs_reduce(int64_t H4, int Ls, cx<S> *
   }
 }
 
-// which: 0, 4 -> d_s, a_s;  2 -> cp_s, b_s, convergence, k += 1;  1, 3 -> out[s] = sum
+// which: 4 -> d_s, a_s;  2 -> cp_s, b_s, convergence, k += 1;  1, 3 -> out[s] = sum
 // 256 threads: thread t adds the partials b = t/Ls, t/Ls + 256/Ls, ... of slice t % Ls, and the
 // per-thread sums of each slice are then added in thread order (fixed order, so deterministic).
 static __global__ void __launch_bounds__(256) k_mrhs_fin(const double *partial, int nparts, int Ls, MrhsState *st,
                                                   double *out, int which) {
-  if (which == 4) which = 0;
-  const bool skip = (which == 0 || which == 2) && mgated(st);
-  if (skip && which == 0) return;
+  const bool skip = (which == 4 || which == 2) && mgated(st);
+  if (skip && which == 4) return;
   __shared__ double sh[256];
   const int per = 256 / Ls;
   const int ts = threadIdx.x % Ls, tp = threadIdx.x / Ls;
@@ -2683,7 +2753,7 @@ static __global__ void __launch_bounds__(256) k_mrhs_fin(const double *partial, 
     return;
   }
   __shared__ double rel[kMaxRhs];
-  if (which == 0) {
+  if (which == 4) {
     if (s < Ls) {
       st->d[s] = v;
       st->a[s] = (v != 0.0) ? st->c[s] / v : 0.0;
@@ -2746,7 +2816,6 @@ int launch_mrhs_reduce(Ctx *ctx, int mode, const Geom &g, void *x, const void *y
   hipLaunchKernelGGL((k_mrhs_reduce<T, M>), dim3(nb), dim3(256), 0, ctx->stream, g.H4, g.Ls, px, py, pz,           \
                      (const MrhsState *)state, ctx->red_partial)
   switch (mode) {
-    case 0: GX_MR(0); break;
     case 1: GX_MR(1); break;
     case 2: GX_MR(2); break;
     case 3: GX_MR(3); break;
@@ -3451,10 +3520,17 @@ static __global__ void __launch_bounds__(256) k_fold_tiles(const double *__restr
   }
 }
 
+// up to this many tile sums the finaliser takes them directly (32 per thread): one launch less
+constexpr int64_t kFoldDirect = 8192;
 int launch_fold_norms(Ctx *ctx, const double *npart, int64_t ntiles, int Ls, MrhsState *state, int which) {
   if (Ls < 1 || Ls > kMaxRhs || ntiles < 1 || (which != 2 && which != 4)) {
     set_error("fold norms: %lld tiles of %d slices (which %d)", (long long)ntiles, Ls, which);
     return GX_EINVAL;
+  }
+  if (ntiles * Ls <= kFoldDirect) {
+    hipLaunchKernelGGL(k_mrhs_fin, dim3(1), dim3(256), 0, ctx->stream, npart, (int)ntiles, Ls, state, nullptr, which);
+    GX_CHECK_HIP(hipGetLastError());
+    return GX_OK;
   }
   const int rpb = 256 / Ls;
   int64_t nb = (ntiles + rpb - 1) / rpb;
@@ -3467,29 +3543,12 @@ int launch_fold_norms(Ctx *ctx, const double *npart, int64_t ntiles, int Ls, Mrh
   return GX_OK;
 }
 
-// the same tile sums added over every tile and slice into block partials of the single-RHS CG
-// (fixed order: thread, wave, workgroup)
-static __global__ void __launch_bounds__(256) k_fold_all(const double *__restrict__ tp, int64_t n, const CGState *st,
-                                                         double *partial) {
-  if (gated(st)) return;
-  __shared__ double sh[1][4];
-  double v[1] = {0};
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    v[0] += tp[i];
-  block_sum<1>(v, sh);
-  write_partial<1>(v, partial);
-}
-
-int launch_fold_cg(Ctx *ctx, const double *npart, int64_t ntiles, int Ls, CGState *state, int which) {
-  if (Ls < 1 || ntiles < 1 || (which != 0 && which != 1)) {
-    set_error("fold cg: %lld tiles of %d slices (which %d)", (long long)ntiles, Ls, which);
+int launch_fold_cg(Ctx *ctx, const double *npart, int64_t ntiles, CGState *state, int which) {
+  if (ntiles < 1 || ntiles > INT_MAX || (which != 0 && which != 1)) {
+    set_error("fold cg: %lld tiles (which %d)", (long long)ntiles, which);
     return GX_EINVAL;
   }
-  const int64_t n = ntiles * Ls;
-  const int nb = red_blocks(n);
-  hipLaunchKernelGGL(k_fold_all, dim3(nb), dim3(256), 0, ctx->stream, npart, n, (const CGState *)state,
-                     ctx->red_partial);
-  hipLaunchKernelGGL(k_cg_fin, dim3(1), dim3(256), 0, ctx->stream, (const double *)ctx->red_partial, nb, state, which);
+  hipLaunchKernelGGL(k_cg_fin, dim3(1), dim3(1024), 0, ctx->stream, npart, (int)ntiles, state, which);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
@@ -3688,6 +3747,8 @@ int launch_digest_slices(Ctx *ctx, const Geom &g, const void *full, int s0, int 
   template int launch_reduce<S>(Ctx *, int, int64_t, int64_t, const void *, const void *, void *, double, int);   \
   template int launch_cg_dot<S>(Ctx *, int64_t, int64_t, const void *, const void *, CGState *);                   \
   template int launch_cg_axpy_norm<S>(Ctx *, int64_t, int64_t, void *, const void *, CGState *);                   \
+  template int launch_cg_update_fin<S>(Ctx *, int64_t, int64_t, void *, void *, const void *, const CGState *,     \
+                                       CGState *, const double *, int);                                            \
   template int launch_cg_update<S>(Ctx *, int64_t, int64_t, void *, void *, const void *, CGState *);
 #define GX_INST_REAL(T)                                                                                            \
   template int launch_slice_proj<T>(const Geom &, const void *, int, int, void *, int, int, int, int, hipStream_t, \

@@ -66,7 +66,7 @@ static int run_batch(Ctx *ctx, BatchGraph &g, const void *const key[8], int batc
 }
 
 struct CGWork {
-  CGState *dev = nullptr;
+  CGState *dev = nullptr;   // 2: the state, and its successor (cg_iteration_small)
   CGState *host = nullptr;  // pinned, 2 slots
   hipEvent_t ev[2] = {};
   BatchGraph graph[3];  // per precision
@@ -131,7 +131,7 @@ static int solver_work(Op *op, SolverWork **out) {
     SolverWork *w = new SolverWork();
     CGWork &c = w->cg;
     MrhsWork &m = w->mrhs;
-    hipError_t e = hipMalloc(&c.dev, sizeof(CGState));
+    hipError_t e = hipMalloc(&c.dev, 2 * sizeof(CGState));
     if (e == hipSuccess) e = hipHostMalloc(&c.host, 2 * sizeof(CGState), hipHostMallocDefault);
     if (e == hipSuccess) e = hipMalloc(&m.dev, sizeof(MrhsState));
     if (e == hipSuccess) e = hipHostMalloc(&m.host, 2 * sizeof(MrhsState), hipHostMallocDefault);
@@ -161,42 +161,73 @@ size_t solver_work_bytes(const SolverWork *w) { return w ? w->mrhs.npart_bytes :
 
 size_t hop_norm_bytes(int64_t H4, int Ls) { return sizeof(double) * (size_t)hop_norm_tiles(H4, Ls) * Ls; }
 
-// FP64 follows Grid (d = <p, MpcDag Mpc p>, then r -= a MpcDag Mpc p with its norm).  In FP32 and
-// FP16 storage, where the tuned hop kernel has the fused epilogues (HopFuse, Ls >= 2), the Mpc
-// hop sums |t|^2 (t = Mpc p) per tile, folded to d = |t|^2 and a, and the last MpcDag hop updates
-// r -= a MpcDag t and sums |r|^2 per tile without storing MpcDag t, as in the multi-RHS CG.
+// Where the tuned hop kernel has the fused epilogues (HopFuse), the Mpc hop sums |t|^2 (t = Mpc p) per
+// tile, folded to d = |t|^2 (equal to Grid's <p, MpcDag Mpc p> in exact arithmetic) and a, and the last
+// MpcDag hop updates r -= a MpcDag t and sums |r|^2 per tile without storing MpcDag t, as in the multi-RHS
+// CG: two passes over the fields less.  npart: room for the tile sums (null: none).
 template <typename T>
 static int cg_iteration(Op *op, Field *psi, Field *p, Field *mmp, Field *r, CGState *st, double *npart) {
   Ctx *ctx = op->ctx;
   const int64_t nsites = p->g.half_pad();
   int64_t n1 = 0, n2 = 0;
-  Field *t = nullptr;
-  if (!std::is_same<T, double>::value && npart) {
-    t = op_tmp(op, p->prec, 2);
-    if (!t) return GX_ENOMEM;
-    HopFuse f1;
-    f1.npart = npart;
-    f1.nparts = &n1;
-    GX_TRY(apply_mpc(op, p, t, 0, st, &f1));
-  }
+  Field *t = op_tmp(op, p->prec, 2);
+  if (!t) return GX_ENOMEM;
+  HopFuse f1;
+  f1.npart = npart;
+  f1.nparts = &n1;
+  f1.total = 1;
+  GX_TRY(apply_mpc(op, p, t, 0, st, npart ? &f1 : nullptr));
   if (n1 == 0) {
-    if (t) GX_TRY(apply_mpc(op, t, mmp, 1, st));
-    else GX_TRY(apply_mpcdagmpc(op, p, mmp, st));
+    GX_TRY(apply_mpc(op, t, mmp, 1, st));
     GX_TRY(launch_cg_dot<T>(ctx, nsites, nsites, p->data, mmp->data, st));
   } else {
-    GX_TRY(launch_fold_cg(ctx, npart, n1, op->g.Ls, st, 0));
-    HopFuse f2;
-    f2.npart = npart;
+    GX_TRY(launch_fold_cg(ctx, npart, n1, st, 0));
+    HopFuse f2 = f1;
     f2.nparts = &n2;
     f2.r = r->data;
     f2.a = &st->a;  // device address of the state's a (not dereferenced here)
     f2.astride = 0;
     GX_TRY(apply_mpc(op, t, mmp, 1, st, &f2));
   }
-  if (n2 > 0) GX_TRY(launch_fold_cg(ctx, npart, n2, op->g.Ls, st, 1));
+  if (n2 > 0) GX_TRY(launch_fold_cg(ctx, npart, n2, st, 1));
   else GX_TRY(launch_cg_axpy_norm<T>(ctx, nsites, nsites, r->data, mmp->data, st));
   GX_TRY(launch_cg_update<T>(ctx, nsites, nsites, psi->data, p->data, r->data, st));
   return GX_OK;
+}
+
+// The same iteration on small lattices (hop_split), where launches are what it costs: the finalisers run
+// inside the kernels that need their results, every workgroup adding the few hundred tile sums for itself in the
+// same order.  The state alternates between cur and nxt, so no kernel writes what another workgroup of it
+// reads.  Wilson: 5 launches instead of 9 (a red-black solve on 8^4 in FP64 2.40 -> 1.50 ms).
+template <typename T>
+static int cg_iteration_small(Op *op, Field *psi, Field *p, Field *mmp, Field *r, CGState *cur, CGState *nxt) {
+  Ctx *ctx = op->ctx;
+  const int64_t nsites = p->g.half_pad();
+  double *dpart = ctx->red_partial, *rpart = dpart + kRedBlocks * kMaxRhs / 2;
+  int64_t n1 = 0, n2 = 0;
+  Field *t = op_tmp(op, p->prec, 2);
+  if (!t) return GX_ENOMEM;
+  HopFuse f1;
+  f1.npart = dpart;
+  f1.nparts = &n1;
+  f1.total = 1;
+  GX_TRY(apply_mpc(op, p, t, 0, cur, &f1));
+  HopFuse f2 = f1;
+  f2.npart = rpart;
+  f2.nparts = &n2;
+  f2.r = r->data;
+  f2.a = &cur->a;
+  f2.astride = 0;
+  f2.cur = cur;
+  f2.nxt = nxt;
+  f2.dpart = dpart;
+  f2.nd = (int)n1;
+  GX_TRY(apply_mpc(op, t, mmp, 1, cur, &f2));
+  if (n1 < 1 || n2 < 1) {
+    set_error("CG: the small-lattice hop left no tile sums");
+    return GX_EINVAL;
+  }
+  return launch_cg_update_fin<T>(ctx, nsites, nsites, psi->data, p->data, r->data, cur, nxt, rpart, (int)n2);
 }
 
 // Device-resident CG iterations on (psi, p, mmp, r) of precision prec, from the state in w.dev,
@@ -206,15 +237,28 @@ static int cg_iteration(Op *op, Field *psi, Field *p, Field *mmp, Field *r, CGSt
 static int cg_device_loop(Op *op, int prec, Field *psi, Field *p, Field *mmp, Field *r, CGWork &w, int maxit,
                           int &enqueued, CGState *out) {
   Ctx *ctx = op->ctx;
-  const int64_t vol = op->g.half_elems();
-  const int batch = vol >= (1 << 20) ? 8 : (vol >= (1 << 16) ? 16 : 32);
+  // 8 iterations per batch: two batches ahead keep the device fed, and at most 16 run gated past the end
+  // (a gated iteration of 8^4 still costs 7 us)
+  const int batch = 8;
   const bool use_graph = tune_get(GX_TUNE_CG_GRAPH, prec) != 0;
   for (int i = 0; i < 4; i++)
     if (!op_tmp(op, prec, i)) return GX_ENOMEM;  // no allocation inside a capture
-  auto one_batch = [&]() -> int {
-    for (int i = 0; i < batch; i++) {
-      GX_TRY(by_prec(prec, [&](auto t) { return cg_iteration<decltype(t)>(op, psi, p, mmp, r, w.dev, w.npart); }));
-    }
+  const bool small = tune_get(GX_TUNE_FUSED, prec) &&
+                     by_prec(prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g); }) != 0;
+  // tile sums: the operator's own buffer, or with Ls = 1 the context's reduction buffer where it holds them
+  double *npart = w.npart;
+  if (!npart && op->g.Ls == 1 && hop_norm_tiles(op->g.H4, 1) <= kRedBlocks * kMaxRhs) npart = ctx->red_partial;
+  int par = 0;  // which of the two states the next iteration reads (small)
+  auto iterate = [&]() -> int {
+    return by_prec(prec, [&](auto t) -> int {
+      if (!small) return cg_iteration<decltype(t)>(op, psi, p, mmp, r, w.dev, npart);
+      CGState *cur = w.dev + par, *nxt = w.dev + (par ^ 1);
+      par ^= 1;
+      return cg_iteration_small<decltype(t)>(op, psi, p, mmp, r, cur, nxt);
+    });
+  };
+  auto one_batch = [&]() -> int {  // an even number of iterations: the state is back where it was
+    for (int i = 0; i < batch; i++) GX_TRY(iterate());
     return GX_OK;
   };
   auto enqueue = [&](int s) -> int {
@@ -224,11 +268,9 @@ static int cg_device_loop(Op *op, int prec, Field *psi, Field *p, Field *mmp, Fi
       GX_TRY(run_batch(ctx, w.graph[prec], key, batch, one_batch));
       enqueued += batch;
     } else {
-      for (int i = 0; i < batch && enqueued < maxit; i++, enqueued++) {
-        GX_TRY(by_prec(prec, [&](auto t) { return cg_iteration<decltype(t)>(op, psi, p, mmp, r, w.dev, w.npart); }));
-      }
+      for (int i = 0; i < batch && enqueued < maxit; i++, enqueued++) GX_TRY(iterate());
     }
-    GX_CHECK_HIP(hipMemcpyAsync(&w.host[s], w.dev, sizeof(CGState), hipMemcpyDeviceToHost, ctx->stream));
+    GX_CHECK_HIP(hipMemcpyAsync(&w.host[s], w.dev + par, sizeof(CGState), hipMemcpyDeviceToHost, ctx->stream));
     GX_CHECK_HIP(hipEventRecord(w.ev[s], ctx->stream));
     return GX_OK;
   };
@@ -597,9 +639,8 @@ static int slice_reduce(Op *op, int mode, Field *x, Field *y, Field *z, double *
   return GX_OK;
 }
 
-// One CGmultiRHS iteration.  d_s = Re<p_s, MpcDag Mpc p_s> as in Grid (BlockConjugateGradient.h:474-478)
-// for FP64; the FP32 / FP16-storage inner solves of defect correction take the same quantity as
-// |Mpc p_s|^2 from the intermediate t = Mpc p (equal in exact arithmetic since MpcDag is the adjoint
+// One CGmultiRHS iteration.  d_s = Re<p_s, MpcDag Mpc p_s> of Grid (BlockConjugateGradient.h:474-478) is taken
+// as |Mpc p_s|^2 from the intermediate t = Mpc p (equal in exact arithmetic since MpcDag is the adjoint
 // of Mpc).  There, where the tuned hop kernel has the fused epilogues (HopFuse), the Mpc hop sums
 // |t_s|^2 per tile (folded to d_s, a_s), and the last MpcDag hop updates r_s -= a_s (MpcDag t)_s
 // and sums |r_s|^2 per tile without storing MpcDag t: the iteration reads and writes no field
@@ -607,19 +648,13 @@ static int slice_reduce(Op *op, int mode, Field *x, Field *y, Field *z, double *
 template <typename T>
 static int mrhs_iteration(Op *op, Field *psi, Field *p, Field *mmp, Field *r, MrhsState *st, double *npart) {
   Ctx *ctx = op->ctx;
-  if (std::is_same<T, double>::value || !npart) {
-    GX_TRY(apply_mpcdagmpc(op, p, mmp, st));
-    if (std::is_same<T, double>::value) {
-      GX_TRY(launch_mrhs_reduce<T>(ctx, 0, op->g, p->data, mmp->data, nullptr, st, nullptr));
-    } else {
-      Field *t = op_tmp(op, p->prec, 2);
-      if (!t) return GX_ENOMEM;
-      GX_TRY(launch_mrhs_reduce<T>(ctx, 4, op->g, t->data, nullptr, nullptr, st, nullptr));
-    }
+  Field *t = op_tmp(op, p->prec, 2);
+  if (!t) return GX_ENOMEM;
+  if (!npart) {
+    GX_TRY(apply_mpcdagmpc(op, p, mmp, st));  // leaves Mpc p in t
+    GX_TRY(launch_mrhs_reduce<T>(ctx, 4, op->g, t->data, nullptr, nullptr, st, nullptr));
     GX_TRY(launch_mrhs_reduce<T>(ctx, 2, op->g, r->data, mmp->data, nullptr, st, nullptr));
   } else {
-    Field *t = op_tmp(op, p->prec, 2);
-    if (!t) return GX_ENOMEM;
     int64_t n1 = 0, n2 = 0;
     HopFuse f1;
     f1.npart = npart;
@@ -720,7 +755,7 @@ int mrhs_cg_run(Op *op, Field *src, Field *psi, double tol, int maxit, gx_solver
     GX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     const int64_t vol = op->g.half_elems();
     // iterations per enqueued batch: one batch at most runs gated past convergence
-    const int batch = vol >= (1 << 24) ? 4 : (vol >= (1 << 20) ? 8 : (vol >= (1 << 16) ? 16 : 32));
+    const int batch = vol >= (1 << 24) ? 4 : 8;
     int enqueued = 0, slot = 0;
     const bool use_graph = tune_get(GX_TUNE_CG_GRAPH, prec) != 0;
     for (int i = 0; i < 4; i++)
