@@ -998,6 +998,7 @@ int gx_ctx_create(int device, gx_ctx *out) {
 int gx_ctx_destroy(gx_ctx c) {
   if (!c) return GX_OK;
   (void)hipStreamSynchronize(c->stream);
+  block_work_free(c->block);
   for (int i = 0; i < 16; i++) (void)hipEventDestroy(c->ev[i]);
   (void)hipFree(c->red_partial);
   (void)hipFree(c->digest);

@@ -119,6 +119,9 @@ struct MrhsState : Gate {
   double tol2;
 };
 
+struct BlockWork;  // workspace of the block algebra (gx_solver.hip)
+void block_work_free(BlockWork *w);
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -128,6 +131,7 @@ struct Ctx {
   double *red_result = nullptr;      // [kRedSlots]
   double *pinned = nullptr;          // host mirror of red_result
   int next_slot = 0;
+  BlockWork *block = nullptr;        // created by the first block-algebra call, released with the context
 };
 
 struct Field {

@@ -3322,69 +3322,83 @@ static __device__ __forceinline__ int64_t slice_idx(int64_t gs, int s, int k, in
   return hf * hstride + ((e / kBlk) * 12 + k) * kBlk + (e & (kBlk - 1));
 }
 
-// sliceInnerProductMatrix: m(s, t) = sum conj(x_s) y_t.  A workgroup stages kIpmSites sites (every
-// slice and component) of x and y in LDS; thread s * Ls + t accumulates m(s, t) over them and
-// writes its workgroup's partial sum; k_slice_ipm_fin adds the partials in a fixed order.
-constexpr int kIpmSites = 8;
-static __global__ void __launch_bounds__(256) k_slice_ipm(int64_t nsite, int64_t H4, int Ls, int64_t hstride,
-                                                          const cx<double> *__restrict__ x,
-                                                          const cx<double> *__restrict__ y, double2 *partial) {
-  __shared__ double2 sx[kIpmSites * kMaxLs * 12], sy[kIpmSites * kMaxLs * 12];
-  const int t = threadIdx.x, ls2 = Ls * Ls;
-  const int si = t / Ls, ti = t - si * Ls;
-  const int per = kIpmSites * Ls;
-  double ar = 0, ai = 0;
-  for (int64_t g0 = (int64_t)blockIdx.x * kIpmSites; g0 < nsite; g0 += (int64_t)gridDim.x * kIpmSites) {
-    const int ns = (int)min((int64_t)kIpmSites, nsite - g0);
-    __syncthreads();
-    for (int q = t; q < 12 * per; q += 256) {
-      const int k = q / per, j = q - k * per;  // component k, staged entry j = site * Ls + s
-      double2 vx = {0, 0}, vy = {0, 0};
-      if (j < ns * Ls) {
-        const int hs = j / Ls;
-        const int64_t i = slice_idx(g0 + hs, j - hs * Ls, k, H4, Ls, hstride);
-        vx = {x[i].r, x[i].i};
-        vy = {y[i].r, y[i].i};
-      }
-      sx[j * 12 + k] = vx;
-      sy[j * 12 + k] = vy;
-    }
-    __syncthreads();
-    if (t < ls2)
-      for (int hs = 0; hs < ns; hs++) {
-        const double2 *px = sx + (hs * Ls + si) * 12, *py = sy + (hs * Ls + ti) * 12;
-#pragma unroll
-        for (int k = 0; k < 12; k++) {
-          ar = fma(px[k].x, py[k].x, fma(px[k].y, py[k].y, ar));
-          ai = fma(px[k].x, py[k].y, fma(-px[k].y, py[k].x, ai));
-        }
-      }
+// ---- inner-product matrices on the matrix cores ----
+// m(i, j) = sum over rows of conj(x_i) y_j is a contraction over the rows (4D site, component): v_mfma_f64_
+// 16x16x4f64 adds four rows of it, lane l holding x and y of column l % 16 at row l / 16 (A and B alike), as
+// loaded: no staging.  Fewer than 16 columns: the 16 lanes hold G = 16 / n row groups of n columns, whose
+// products are the diagonal n x n blocks.  Result register v of lane l: (4 v + l / 16, l % 16).
+// Bound by the two fields' reads: 12 columns of 16^3 x 32 / 2 sites, 2 x 151 MB, 94 us as dot products
+// from LDS, 66 us so; with x = y (one read) 94 -> 36.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+constexpr int kIpmWaves = 8;
+
+struct IpmAcc {
+  f64x4 re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+  __device__ __forceinline__ void add(cx<double> x, cx<double> y) {
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(x.r, y.r, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(x.r, y.i, im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(x.i, y.i, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.i, y.r, im, 0, 0, 0);
   }
-  if (t < ls2) partial[(int64_t)blockIdx.x * ls2 + t] = {ar, ai};
+};
+
+// the waves' and row groups' matrices added in a fixed order into partial[entry][workgroup]
+__device__ __forceinline__ void ipm_finish(const IpmAcc &a, int n, double2 *partial) {
+  __shared__ double2 sm[kIpmWaves][256];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int v = 0; v < 4; v++) sm[w][(4 * v + (lane >> 4)) * 16 + (lane & 15)] = {a.re[v], a.im[v]};
+  __syncthreads();
+  if (threadIdx.x >= n * n) return;
+  const int i = threadIdx.x / n, j = threadIdx.x - i * n;
+  double2 t = {0, 0};
+  for (int ww = 0; ww < kIpmWaves; ww++)
+    for (int q = 0; q < 16 / n; q++) {
+      const double2 v = sm[ww][(q * n + i) * 16 + q * n + j];
+      t.x += v.x;
+      t.y += v.y;
+    }
+  partial[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
+}
+
+// sliceInnerProductMatrix: columns = the Ls slices; a wave step takes 4 G sites, their 12 components one
+// after another
+template <bool SAME>
+static __global__ void __launch_bounds__(64 * kIpmWaves) k_slice_ipm(int64_t nsite, int64_t H4, int Ls, int64_t hstride,
+                                                                     const cx<double> *__restrict__ x,
+                                                                     const cx<double> *__restrict__ y, double2 *partial) {
+  const int lane = threadIdx.x & 63, G = 16 / Ls, q = (lane & 15) / Ls, s = (lane & 15) - q * Ls;
+  const int64_t step = 4 * G, first = (int64_t)blockIdx.x * kIpmWaves + (threadIdx.x >> 6);
+  IpmAcc acc;
+  for (int64_t g0 = first * step; g0 < nsite; g0 += (int64_t)gridDim.x * kIpmWaves * step) {
+    const int64_t gs = g0 + (lane >> 4) * G + q;
+    const bool on = q < G && gs < nsite;
+    const int64_t i = slice_idx(on ? gs : 0, on ? s : 0, 0, H4, Ls, hstride);
+    cx<double> xv[12], yv[12];
+#pragma unroll
+    for (int k = 0; k < 12; k++) {
+      xv[k] = on ? x[i + k * kBlk] : cx<double>{0, 0};
+      yv[k] = SAME ? xv[k] : on ? y[i + k * kBlk] : cx<double>{0, 0};
+    }
+#pragma unroll
+    for (int k = 0; k < 12; k++) acc.add(xv[k], yv[k]);
+  }
+  ipm_finish(acc, Ls, partial);
 }
 
 // workgroup p adds the partials of matrix entry p: thread t the partials t, t + 256, ... in order,
 // then a fixed tree over the threads (bitwise reproducible)
-static __global__ void __launch_bounds__(256) k_slice_ipm_fin(const double2 *partial, int nparts, int ls2,
-                                                              double2 *out) {
+static __global__ void __launch_bounds__(256) k_ipm_fin(const double2 *partial, int nparts, double2 *out) {
   const int t = threadIdx.x, p = blockIdx.x;
-  double ar = 0, ai = 0;
+  double v[2] = {0, 0};
   for (int b = t; b < nparts; b += 256) {
-    ar += partial[(int64_t)b * ls2 + p].x;
-    ai += partial[(int64_t)b * ls2 + p].y;
+    const double2 w = partial[(int64_t)p * nparts + b];
+    v[0] += w.x;
+    v[1] += w.y;
   }
-  __shared__ double sh[2][256];
-  sh[0][t] = ar;
-  sh[1][t] = ai;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (t < off) {
-      sh[0][t] += sh[0][t + off];
-      sh[1][t] += sh[1][t + off];
-    }
-    __syncthreads();
-  }
-  if (t == 0) out[p] = {sh[0][0], sh[1][0]};
+  __shared__ double sh[2][4];
+  block_sum<2>(v, sh);
+  if (t == 0) out[p] = {v[0], v[1]};
 }
 
 // sliceMaddMatrix: r_t = y_t + scale sum_s x_s a(s, t), a row-major (a[s * Ls + t]); y = null reads
@@ -3437,38 +3451,34 @@ static __global__ void __launch_bounds__(256) k_slice_madd(int64_t nsite, int64_
 
 // ---------------- matrices over lists of fields (BlockConjugateGradient.h:35-74) ----------------
 // InnerProductMatrix: m(b, bp) = <X_b, Y_bp> over n FP64 fields of nelem stored complex numbers
-// each (padding entries are zero).  A workgroup stages kVecChunk elements of every X_b and Y_b in
-// LDS; thread b * n + bp accumulates m(b, bp) over them and writes its workgroup's partial sum,
-// which k_slice_ipm_fin adds in a fixed order.
-constexpr int kVecChunk = 64;
-static __global__ void __launch_bounds__(256) k_vec_ipm(int64_t nelem, int n, VecPtrs x, VecPtrs y, double2 *partial) {
-  __shared__ double2 sx[kMaxLs * kVecChunk], sy[kMaxLs * kVecChunk];
-  const int t = threadIdx.x, n2 = n * n;
-  const int bi = t / n, bj = t - bi * n;
-  double ar = 0, ai = 0;
-  for (int64_t i0 = (int64_t)blockIdx.x * kVecChunk; i0 < nelem; i0 += (int64_t)gridDim.x * kVecChunk) {
-    const int ne = (int)min((int64_t)kVecChunk, nelem - i0);
-    __syncthreads();
-    for (int q = t; q < n * kVecChunk; q += 256) {
-      const int f = q / kVecChunk, j = q - f * kVecChunk;  // field f, element i0 + j (coalesced in j)
-      double2 vx = {0, 0}, vy = {0, 0};
-      if (j < ne) {
-        vx = reinterpret_cast<const double2 *>(x.p[f])[i0 + j];
-        vy = reinterpret_cast<const double2 *>(y.p[f])[i0 + j];
-      }
-      sx[q] = vx;
-      sy[q] = vy;
+// each (padding entries are zero): columns = the fields, a wave step takes 8 G runs of 4 elements
+static __global__ void __launch_bounds__(64 * kIpmWaves) k_vec_ipm(int64_t nelem, int n, VecPtrs x, VecPtrs y,
+                                                                   double2 *partial) {
+  __shared__ const cx<double> *px[kMaxLs], *py[kMaxLs];
+#pragma unroll
+  for (int b = 0; b < kMaxLs; b++)
+    if (threadIdx.x == b) {
+      px[b] = (const cx<double> *)x.p[b];
+      py[b] = (const cx<double> *)y.p[b];
     }
-    __syncthreads();
-    if (t < n2) {
-      const double2 *px = sx + bi * kVecChunk, *py = sy + bj * kVecChunk;
-      for (int j = 0; j < ne; j++) {
-        ar = fma(px[j].x, py[j].x, fma(px[j].y, py[j].y, ar));
-        ai = fma(px[j].x, py[j].y, fma(-px[j].y, py[j].x, ai));
-      }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, G = 16 / n, q = (lane & 15) / n, b = (lane & 15) - q * n;
+  const int64_t step = 32 * G, first = (int64_t)blockIdx.x * kIpmWaves + (threadIdx.x >> 6);
+  const cx<double> *xb = px[b], *yb = py[b];
+  IpmAcc acc;
+  for (int64_t i0 = first * step; i0 < nelem; i0 += (int64_t)gridDim.x * kIpmWaves * step) {
+    cx<double> xv[8], yv[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int64_t i = i0 + (q * 8 + k) * 4 + (lane >> 4);
+      const bool on = q < G && i < nelem;
+      xv[k] = on ? xb[i] : cx<double>{0, 0};
+      yv[k] = on ? yb[i] : cx<double>{0, 0};
     }
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc.add(xv[k], yv[k]);
   }
-  if (t < n2) partial[(int64_t)blockIdx.x * n2 + t] = {ar, ai};
+  ipm_finish(acc, n, partial);
 }
 
 // MaddMatrix: R_b = Y_b + scale sum_bp X_bp a(bp, b) (Y null reads as zero: MulMatrix), one thread per
@@ -3553,16 +3563,22 @@ int launch_fold_cg(Ctx *ctx, const double *npart, int64_t ntiles, CGState *state
   return GX_OK;
 }
 
+// workgroups of the inner-product matrices over `steps` wave steps: at most two of 8 waves per CU
+static int ipm_blocks(int64_t steps, int nparts) {
+  int64_t nb = (steps + kIpmWaves - 1) / kIpmWaves;
+  if (nb > 512) nb = 512;
+  return (int)(nb > nparts ? nparts : nb);
+}
+
 int launch_vec_ipm(Ctx *ctx, int64_t nelem, int n, const VecPtrs &x, const VecPtrs &y, void *partial, int nparts,
                    void *out_dev) {
   if (n < 1 || n > kMaxLs || nparts < 1) {
     set_error("inner product matrix: %d fields (1..%d)", n, kMaxLs);
     return GX_EINVAL;
   }
-  int64_t nb = (nelem + kVecChunk - 1) / kVecChunk;
-  if (nb > nparts) nb = nparts;
-  hipLaunchKernelGGL(k_vec_ipm, dim3(nb), dim3(256), 0, ctx->stream, nelem, n, x, y, (double2 *)partial);
-  hipLaunchKernelGGL(k_slice_ipm_fin, dim3(n * n), dim3(256), 0, ctx->stream, (const double2 *)partial, (int)nb, n * n,
+  const int nb = ipm_blocks((nelem + 32 * (16 / n) - 1) / (32 * (16 / n)), nparts);
+  hipLaunchKernelGGL(k_vec_ipm, dim3(nb), dim3(64 * kIpmWaves), 0, ctx->stream, nelem, n, x, y, (double2 *)partial);
+  hipLaunchKernelGGL(k_ipm_fin, dim3(n * n), dim3(256), 0, ctx->stream, (const double2 *)partial, nb,
                      (double2 *)out_dev);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
@@ -3586,13 +3602,16 @@ int launch_slice_ipm(Ctx *ctx, const Geom &g, int nhalf, const void *x, const vo
     set_error("slice inner product matrix: Ls %d > %d or no partials", g.Ls, kMaxLs);
     return GX_EINVAL;
   }
-  const int64_t nsite = nhalf * g.H4, hstride = 12 * g.half_pad();
-  int64_t nb = (nsite + kIpmSites - 1) / kIpmSites;
-  if (nb > nparts) nb = nparts;
-  hipLaunchKernelGGL(k_slice_ipm, dim3(nb), dim3(256), 0, ctx->stream, nsite, g.H4, g.Ls, hstride,
-                     (const cx<double> *)x, (const cx<double> *)y, (double2 *)partial);
-  hipLaunchKernelGGL(k_slice_ipm_fin, dim3(g.Ls * g.Ls), dim3(256), 0, ctx->stream, (const double2 *)partial,
-                     (int)nb, g.Ls * g.Ls, (double2 *)out_dev);
+  const int64_t nsite = nhalf * g.H4, hstride = 12 * g.half_pad(), step = 4 * (16 / g.Ls);
+  const int nb = ipm_blocks((nsite + step - 1) / step, nparts);
+  if (x == y)
+    hipLaunchKernelGGL((k_slice_ipm<true>), dim3(nb), dim3(64 * kIpmWaves), 0, ctx->stream, nsite, g.H4, g.Ls, hstride,
+                       (const cx<double> *)x, (const cx<double> *)y, (double2 *)partial);
+  else
+    hipLaunchKernelGGL((k_slice_ipm<false>), dim3(nb), dim3(64 * kIpmWaves), 0, ctx->stream, nsite, g.H4, g.Ls, hstride,
+                       (const cx<double> *)x, (const cx<double> *)y, (double2 *)partial);
+  hipLaunchKernelGGL(k_ipm_fin, dim3(g.Ls * g.Ls), dim3(256), 0, ctx->stream, (const double2 *)partial, nb,
+                     (double2 *)out_dev);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }

@@ -1041,71 +1041,110 @@ static bool cm_chol(const CMat &m, CMat &L) {
   return true;
 }
 
-constexpr int kIpmParts = 2048;  // workgroups of the slice inner products (8 per CU)
+constexpr int kIpmParts = 2048;  // room for the workgroup partials of the inner-product matrices
 
+// Workspace of the block algebra, kept by its context from the first call on (9 MB; allocating and freeing
+// it in every slice-matrix call took 65 us of each, and the frees synchronised the device).
 struct BlockWork {
+  static constexpr int kRing = 8;
   Ctx *ctx = nullptr;
-  void *partial = nullptr;   // workgroup partials of the slice inner products
-  double2 *mat_dev = nullptr;   // result matrix + 4 coefficient matrices, kMaxLs^2 each
+  void *partial = nullptr;      // workgroup partials of the inner products
+  double2 *mat_dev = nullptr;   // result matrix + kRing coefficient matrices, kMaxLs^2 each
   double2 *mat_host = nullptr;  // pinned mirror
+  hipEvent_t ev[kRing] = {};    // last use of a coefficient matrix
+  bool used[kRing] = {};
+  int next = 0;
   int nparts = kIpmParts;
   ~BlockWork() {
     if (partial) (void)hipFree(partial);
     if (mat_dev) (void)hipFree(mat_dev);
     if (mat_host) (void)hipHostFree(mat_host);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
   }
   int init(Ctx *c) {
     ctx = c;
     const size_t m = (size_t)kMaxLs * kMaxLs * sizeof(double2);
     hipError_t e = hipMalloc(&partial, (size_t)nparts * m);
-    if (e == hipSuccess) e = hipMalloc(&mat_dev, 5 * m);
-    if (e == hipSuccess) e = hipHostMalloc(&mat_host, 5 * m, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMalloc(&mat_dev, (1 + kRing) * m);
+    if (e == hipSuccess) e = hipHostMalloc(&mat_host, (1 + kRing) * m, hipHostMallocDefault);
+    for (int i = 0; i < kRing && e == hipSuccess; i++) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
     if (e != hipSuccess) {
       set_error("block solver workspace: %s", hipGetErrorString(e));
       return GX_ENOMEM;
     }
     return GX_OK;
   }
-  // m(s, t) = <x_s, y_t> (sliceInnerProductMatrix); synchronises the stream
-  int ipm(const Geom &g, int nhalf, Field *x, Field *y, CMat &m) {
-    const int n = g.Ls;
-    GX_TRY(launch_slice_ipm(ctx, g, nhalf, x->data, y->data, partial, nparts, mat_dev));
+  // the result matrix; synchronises the stream
+  int read(int n, CMat &m) {
     GX_CHECK_HIP(hipMemcpyAsync(mat_host, mat_dev, sizeof(double2) * n * n, hipMemcpyDeviceToHost, ctx->stream));
     GX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     m = CMat(n);
     for (int i = 0; i < n * n; i++) m.a[i] = cd(mat_host[i].x, mat_host[i].y);
     return GX_OK;
+  }
+  // m(s, t) = <x_s, y_t> (sliceInnerProductMatrix); synchronises the stream
+  int ipm(const Geom &g, int nhalf, Field *x, Field *y, CMat &m) {
+    GX_TRY(launch_slice_ipm(ctx, g, nhalf, x->data, y->data, partial, nparts, mat_dev));
+    return read(g.Ls, m);
   }
   // InnerProductMatrix over n fields of nelem stored complex numbers; synchronises the stream
   int ipm_vec(int n, int64_t nelem, const VecPtrs &x, const VecPtrs &y, CMat &m) {
     GX_TRY(launch_vec_ipm(ctx, nelem, n, x, y, partial, nparts, mat_dev));
-    GX_CHECK_HIP(hipMemcpyAsync(mat_host, mat_dev, sizeof(double2) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    GX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    m = CMat(n);
-    for (int i = 0; i < n * n; i++) m.a[i] = cd(mat_host[i].x, mat_host[i].y);
+    return read(n, m);
+  }
+  // A coefficient matrix on the device, in the next slot of the ring once its last use has ended; done()
+  // marks the use that has just been enqueued.
+  int coefficients(const CMat &a, double2 **dev) {
+    if (a.n > kMaxLs) {
+      set_error("slice madd matrix: Ls %d > %d", a.n, kMaxLs);
+      return GX_EINVAL;
+    }
+    if (used[next]) GX_CHECK_HIP(hipEventSynchronize(ev[next]));
+    double2 *h = mat_host + (size_t)(1 + next) * kMaxLs * kMaxLs;
+    *dev = mat_dev + (size_t)(1 + next) * kMaxLs * kMaxLs;
+    for (int i = 0; i < a.n * a.n; i++) h[i] = make_double2(a.a[i].real(), a.a[i].imag());
+    GX_CHECK_HIP(hipMemcpyAsync(*dev, h, sizeof(double2) * a.n * a.n, hipMemcpyHostToDevice, ctx->stream));
     return GX_OK;
   }
-  // MaddMatrix over n fields (coefficient slots as in madd)
-  int madd_vec(int n, int64_t nelem, const VecPtrs &r, const CMat &a, const VecPtrs &x, const VecPtrs &y, double scale,
-               int slot) {
-    double2 *h = mat_host + (size_t)slot * kMaxLs * kMaxLs, *d = mat_dev + (size_t)slot * kMaxLs * kMaxLs;
-    for (int i = 0; i < n * n; i++) h[i] = make_double2(a.a[i].real(), a.a[i].imag());
-    GX_CHECK_HIP(hipMemcpyAsync(d, h, sizeof(double2) * n * n, hipMemcpyHostToDevice, ctx->stream));
-    return launch_vec_madd(ctx, nelem, n, d, scale, x, y, r);
+  int done() {
+    GX_CHECK_HIP(hipEventRecord(ev[next], ctx->stream));
+    used[next] = true;
+    next = (next + 1) % kRing;
+    return GX_OK;
   }
-  // r_t = y_t + scale sum_s x_s a(s, t) (sliceMaddMatrix; y = null: sliceMulMatrix) with coefficient
-  // slot 1..4: a slot's pinned copy is rewritten only after a later ipm() has synchronised the
-  // stream past its use.
-  int madd(const Geom &g, int nhalf, Field *r, const CMat &a, Field *x, Field *y, double scale, int slot) {
-    const int n = g.Ls;
-    double2 *h = mat_host + (size_t)slot * kMaxLs * kMaxLs, *d = mat_dev + (size_t)slot * kMaxLs * kMaxLs;
-    for (int i = 0; i < n * n; i++) h[i] = make_double2(a.a[i].real(), a.a[i].imag());
-    GX_CHECK_HIP(hipMemcpyAsync(d, h, sizeof(double2) * n * n, hipMemcpyHostToDevice, ctx->stream));
+  // MaddMatrix over n fields
+  int madd_vec(int n, int64_t nelem, const VecPtrs &r, const CMat &a, const VecPtrs &x, const VecPtrs &y, double scale) {
+    double2 *d;
+    GX_TRY(coefficients(a, &d));
+    GX_TRY(launch_vec_madd(ctx, nelem, n, d, scale, x, y, r));
+    return done();
+  }
+  // r_t = y_t + scale sum_s x_s a(s, t) (sliceMaddMatrix; y = null: sliceMulMatrix)
+  int madd(const Geom &g, int nhalf, Field *r, const CMat &a, Field *x, Field *y, double scale) {
+    double2 *d;
+    GX_TRY(coefficients(a, &d));
     GX_TRY(launch_slice_madd(ctx, g, nhalf, d, scale, x->data, y ? y->data : nullptr, r->data));
     r->cb = x->cb;
-    return GX_OK;
+    return done();
   }
 };
+
+static int block_work(Ctx *ctx, BlockWork **out) {
+  if (!ctx->block) {
+    BlockWork *w = new BlockWork();
+    const int rc = w->init(ctx);
+    if (rc != GX_OK) {
+      delete w;
+      return rc;
+    }
+    ctx->block = w;
+  }
+  *out = ctx->block;
+  return GX_OK;
+}
+
+void block_work_free(BlockWork *w) { delete w; }
 
 // The block of Nblock right-hand sides BlockCGrQ works on, in one of two forms:
 //   SliceBlock  the fifth-dimension slices of one field (Orthog = 0, BlockCGrQsolve,
@@ -1129,8 +1168,8 @@ struct SliceBlock {
     return GX_OK;
   }
   int ipm(int x, int y, CMat &m) { return bw->ipm(op->g, 1, v[x], v[y], m); }
-  int madd(int r, const CMat &a, int x, int y, double scale, int slot) {
-    return bw->madd(op->g, 1, v[r], a, v[x], y < 0 ? nullptr : v[y], scale, slot);
+  int madd(int r, const CMat &a, int x, int y, double scale) {
+    return bw->madd(op->g, 1, v[r], a, v[x], y < 0 ? nullptr : v[y], scale);
   }
   // res[b] = |A X_b - B_b|^2 (R is overwritten)
   int residuals(double *res) {
@@ -1179,8 +1218,8 @@ struct VecBlock {
     return p;
   }
   int ipm(int x, int y, CMat &m) { return bw->ipm_vec(nb, v[x][0]->stored(), ptrs(x), ptrs(y), m); }
-  int madd(int r, const CMat &a, int x, int y, double scale, int slot) {
-    GX_TRY(bw->madd_vec(nb, v[x][0]->stored(), ptrs(r), a, ptrs(x), ptrs(y), scale, slot));
+  int madd(int r, const CMat &a, int x, int y, double scale) {
+    GX_TRY(bw->madd_vec(nb, v[x][0]->stored(), ptrs(r), a, ptrs(x), ptrs(y), scale));
     for (int b = 0; b < nb; b++) v[r][b]->cb = v[x][b]->cb;
     return GX_OK;
   }
@@ -1196,7 +1235,7 @@ struct VecBlock {
 // ThinQRfact (BlockConjugateGradient.h:132-190): m_rr = R^dag R (made manifestly Hermitian),
 // L = chol(m_rr), C = L^dag, Q = R C^-1.
 template <class Blk>
-static int thin_qr(Blk &blk, int Q, int R, CMat &C, int slot) {
+static int thin_qr(Blk &blk, int Q, int R, CMat &C) {
   CMat m, L, Cinv;
   GX_TRY(blk.ipm(R, R, m));
   CMat h = m;
@@ -1211,7 +1250,7 @@ static int thin_qr(Blk &blk, int Q, int R, CMat &C, int slot) {
     set_error("BlockCGrQ: singular triangular factor");
     return GX_ENOCONV;
   }
-  return blk.madd(Q, Cinv, R, -1, 1.0, slot);  // MulMatrix(Q, Cinv, R)
+  return blk.madd(Q, Cinv, R, -1, 1.0);  // MulMatrix(Q, Cinv, R)
 }
 
 // BlockCGrQ (Birk's thesis after Dubrulle 2001; BlockConjugateGradient.h:223-410 and the Vec form
@@ -1239,7 +1278,7 @@ static int block_cgrq_core(Blk &blk, double tol, int maxit, gx_solver_stats *st)
   GX_TRY(blk.apply(BV_X, BV_Z));
   GX_TRY(blk.sub(BV_R, BV_B, BV_Z));  // R = B - A X
   CMat C, S, M, DZ, rr;
-  GX_TRY(thin_qr(blk, BV_Q, BV_R, C, 3));
+  GX_TRY(thin_qr(blk, BV_Q, BV_R, C));
   GX_TRY(blk.copy(BV_D, BV_Q));
   int rc = GX_ENOCONV, k;
   for (k = 1; k <= maxit; k++) {
@@ -1249,12 +1288,12 @@ static int block_cgrq_core(Blk &blk, double tol, int maxit, gx_solver_stats *st)
       set_error("BlockCGrQ: D^dag A D is singular at iteration %d", k);
       break;
     }
-    GX_TRY(blk.madd(BV_X, cm_mul(M, C), BV_D, BV_X, 1.0, 1));  // X = X + D M C
-    GX_TRY(blk.madd(BV_R, M, BV_Z, BV_Q, -1.0, 2));            // R = Q - Z M
-    const int qr = thin_qr(blk, BV_Q, BV_R, S, 3);             // Q S = R
+    GX_TRY(blk.madd(BV_X, cm_mul(M, C), BV_D, BV_X, 1.0));  // X = X + D M C
+    GX_TRY(blk.madd(BV_R, M, BV_Z, BV_Q, -1.0));            // R = Q - Z M
+    const int qr = thin_qr(blk, BV_Q, BV_R, S);             // Q S = R
     if (qr == GX_ENOCONV) break;
     GX_TRY(qr);
-    GX_TRY(blk.madd(BV_D, cm_adj(S), BV_D, BV_Q, 1.0, 4));     // D = Q + D S^dag
+    GX_TRY(blk.madd(BV_D, cm_adj(S), BV_D, BV_Q, 1.0));     // D = Q + D S^dag
     C = cm_mul(S, C);
     rr = cm_mul(cm_adj(C), C);
     double mx = 0;
@@ -1285,9 +1324,9 @@ static int block_cgrq_run(Op *op, Field *B, Field *X, double tol, int maxit, gx_
   Field *R = op_tmp(op, GX_F64, 4), *Q = op_tmp(op, GX_F64, 5), *D = op_tmp(op, GX_F64, 6), *Z = op_tmp(op, GX_F64, 9);
   if (!R || !Q || !D || !Z) return GX_ENOMEM;
   X->cb = R->cb = Q->cb = D->cb = Z->cb = B->cb;
-  BlockWork bw;
-  GX_TRY(bw.init(op->ctx));
-  SliceBlock blk{op, &bw};
+  BlockWork *bw;
+  GX_TRY(block_work(op->ctx, &bw));
+  SliceBlock blk{op, bw};
   blk.v[BV_B] = B, blk.v[BV_X] = X, blk.v[BV_R] = R, blk.v[BV_Q] = Q, blk.v[BV_D] = D, blk.v[BV_Z] = Z;
   return block_cgrq_core(blk, tol, maxit, st);
 }
@@ -1297,9 +1336,9 @@ static int block_cgrq_run(Op *op, Field *B, Field *X, double tol, int maxit, gx_
 static int block_cgrq_vec_run(Op *op, int herm, int n, Field **B, Field **X, double tol, int maxit,
                               gx_solver_stats *st) {
   GX_TRY(op_prepare(op, GX_F64));
-  BlockWork bw;
-  GX_TRY(bw.init(op->ctx));
-  VecBlock blk{op, &bw, herm, n};
+  BlockWork *bw;
+  GX_TRY(block_work(op->ctx, &bw));
+  VecBlock blk{op, bw, herm, n};
   struct Owned {
     std::vector<Field *> list;
     ~Owned() {
@@ -1770,10 +1809,10 @@ int gx_slice_inner_product_matrix(gx_field lhs, gx_field rhs, double *mat) {
     set_error("slice_inner_product_matrix: needs two F64 fields of one lattice and subset");
     return GX_EINVAL;
   }
-  BlockWork bw;
-  GX_TRY(bw.init(lhs->ctx));
+  BlockWork *bw;
+  GX_TRY(block_work(lhs->ctx, &bw));
   CMat m;
-  GX_TRY(bw.ipm(lhs->g, lhs->subset == GX_FULL ? 2 : 1, lhs, rhs, m));
+  GX_TRY(bw->ipm(lhs->g, lhs->subset == GX_FULL ? 2 : 1, lhs, rhs, m));
   for (int i = 0; i < m.n * m.n; i++) {
     mat[2 * i] = m.a[i].real();
     mat[2 * i + 1] = m.a[i].imag();
@@ -1806,11 +1845,9 @@ int gx_slice_madd_matrix(gx_field R, const double *aa, gx_field X, gx_field Y, d
   const int n = X->g.Ls;
   CMat a(n);
   for (int i = 0; i < n * n; i++) a.a[i] = cd(aa[2 * i], aa[2 * i + 1]);
-  BlockWork bw;
-  GX_TRY(bw.init(X->ctx));
-  GX_TRY(bw.madd(X->g, X->subset == GX_FULL ? 2 : 1, R, a, X, Y, scale, 1));
-  GX_CHECK_HIP(hipStreamSynchronize(X->ctx->stream));  // the workspace is freed on return
-  return GX_OK;
+  BlockWork *bw;
+  GX_TRY(block_work(X->ctx, &bw));
+  return bw->madd(X->g, X->subset == GX_FULL ? 2 : 1, R, a, X, Y, scale);
 }
 
 // n fields of one lattice, subset and precision (F64) as a pointer list; false if they are not
@@ -1835,10 +1872,10 @@ int gx_inner_product_matrix(int n, gx_field *X, gx_field *Y, double *mat) {
     set_error("inner_product_matrix: needs 1..%d F64 fields of one lattice and subset on each side", kMaxLs);
     return GX_EINVAL;
   }
-  BlockWork bw;
-  GX_TRY(bw.init(fx->ctx));
+  BlockWork *bw;
+  GX_TRY(block_work(fx->ctx, &bw));
   CMat m;
-  GX_TRY(bw.ipm_vec(n, fx->stored(), px, py, m));
+  GX_TRY(bw->ipm_vec(n, fx->stored(), px, py, m));
   for (int i = 0; i < n * n; i++) {
     mat[2 * i] = m.a[i].real();
     mat[2 * i + 1] = m.a[i].imag();
@@ -1858,11 +1895,10 @@ int gx_madd_matrix(int n, gx_field *R, const double *aa, gx_field *X, gx_field *
   }
   CMat a(n);
   for (int i = 0; i < n * n; i++) a.a[i] = cd(aa[2 * i], aa[2 * i + 1]);
-  BlockWork bw;
-  GX_TRY(bw.init(fx->ctx));
-  GX_TRY(bw.madd_vec(n, fx->stored(), pr, a, px, py, scale, 1));
+  BlockWork *bw;
+  GX_TRY(block_work(fx->ctx, &bw));
+  GX_TRY(bw->madd_vec(n, fx->stored(), pr, a, px, py, scale));
   for (int b = 0; b < n; b++) R[b]->cb = X[b]->cb;
-  GX_CHECK_HIP(hipStreamSynchronize(fx->ctx->stream));  // the workspace is freed on return
   return GX_OK;
 }
 
