@@ -15,11 +15,13 @@
 #include <cfloat>
 #include <climits>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <new>
 #include <thread>
 
 #include "gx_internal.h"
@@ -64,6 +66,155 @@ static void parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> 
     th.emplace_back([=, &f]() { f(b, e); });
   }
   for (auto &x : th) x.join();
+}
+
+// ---------------- host transfers ----------------
+// A few threads for the length of one call: run(f) has each of them do its share f(i, n) and waits.
+class Team {
+  std::vector<std::thread> th;
+  std::mutex mu;
+  std::condition_variable go, done;
+  const std::function<void(int, int)> *job = nullptr;
+  int gen = 0, left = 0;
+  bool stop = false;
+  void work(int i, int n) {
+    int seen = 0;
+    for (;;) {
+      const std::function<void(int, int)> *f;
+      {
+        std::unique_lock<std::mutex> lk(mu);
+        go.wait(lk, [&] { return stop || gen != seen; });
+        if (stop) return;
+        seen = gen;
+        f = job;
+      }
+      (*f)(i, n);
+      std::lock_guard<std::mutex> lk(mu);
+      if (--left == 0) done.notify_one();
+    }
+  }
+
+ public:
+  explicit Team(int n) {
+    for (int i = 1; i < n; i++) {
+      try {
+        th.emplace_back([this, i, n] { work(i, n); });
+      } catch (...) {  // no thread to be had: run() refuses below
+        break;
+      }
+    }
+    if ((int)th.size() != n - 1) end();
+  }
+  ~Team() { end(); }
+  void end() {
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      stop = true;
+    }
+    go.notify_all();
+    for (auto &t : th) t.join();
+    th.clear();
+  }
+  void run(const std::function<void(int, int)> &f) {
+    const int n = (int)th.size() + 1;
+    if (n == 1) {
+      f(0, 1);
+      return;
+    }
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      job = &f;
+      left = n - 1;
+      gen++;
+    }
+    go.notify_all();
+    f(0, n);
+    std::unique_lock<std::mutex> lk(mu);
+    done.wait(lk, [&] { return left == 0; });
+  }
+};
+
+// Pinned chunks, kept by the context: one of 256 KB for small transfers, kChunks of kChunk bytes for the
+// others (16 MB in all), allocated by the first call that needs them.
+struct HostPipe {
+  static constexpr size_t kSmall = 256 << 10, kChunk = 4 << 20;
+  static constexpr int kChunks = 4;
+  char *small = nullptr, *big = nullptr;
+  hipEvent_t ev[kChunks] = {};
+  ~HostPipe() {
+    if (small) (void)hipHostFree(small);
+    if (big) (void)hipHostFree(big);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+  }
+  int reserve(size_t bytes) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < kChunks && e == hipSuccess; i++)
+      if (!ev[i]) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
+    char *&p = bytes <= kSmall ? small : big;
+    if (e == hipSuccess && !p)
+      e = hipHostMalloc((void **)&p, bytes <= kSmall ? kSmall : kChunks * kChunk, hipHostMallocDefault);
+    if (e != hipSuccess) {
+      set_error("host transfer: %s", hipGetErrorString(e));
+      return GX_ENOMEM;
+    }
+    return GX_OK;
+  }
+};
+
+// Eight threads at most: a transfer of n MB takes n of them (below that a thread costs what it saves).
+// Moves `units` units of `unit` bytes between the user's memory and the GPU in pinned chunks, in order.
+// launch(chunk, u0, u1) enqueues the kernel that fills (to_host) or reads the chunk of units u0 .. u1 - 1;
+// copy(chunk, b, e, u0) copies units b .. e - 1 of it from or to the user's memory.  Done on return.
+template <class Launch, class Copy>
+static int host_pipe(Ctx *ctx, int64_t units, size_t unit, bool to_host, Launch launch, Copy copy) {
+  if (!ctx->pipe && !(ctx->pipe = new (std::nothrow) HostPipe())) return GX_ENOMEM;
+  HostPipe &hp = *ctx->pipe;
+  const size_t bytes = units * unit;
+  GX_TRY(hp.reserve(bytes));
+  if (bytes <= HostPipe::kSmall) {
+    if (!to_host) copy(hp.small, 0, units, 0);
+    GX_TRY(launch(hp.small, 0, units));
+    GX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    if (to_host) copy(hp.small, 0, units, 0);
+    return GX_OK;
+  }
+  const int64_t per = std::max<int64_t>(1, HostPipe::kChunk / unit), nchunk = (units + per - 1) / per;
+  const int hw = (int)std::thread::hardware_concurrency();
+  Team team((int)std::max<int64_t>(1, std::min<int64_t>({8, hw > 0 ? hw : 1, (int64_t)(bytes >> 20)})));
+  auto chunk = [&](int64_t c) { return hp.big + (c % HostPipe::kChunks) * HostPipe::kChunk; };
+  auto copy_chunk = [&](int64_t c) {
+    const int64_t u0 = c * per, n = std::min(per, units - u0);
+    team.run([&](int i, int nt) {
+      const int64_t b = u0 + n * i / nt, e = u0 + n * (i + 1) / nt;
+      if (b < e) copy(chunk(c), b, e, u0);
+    });
+  };
+  auto start = [&](int64_t c) -> int {
+    GX_TRY(launch(chunk(c), c * per, std::min(units, (c + 1) * per)));
+    GX_CHECK_HIP(hipEventRecord(hp.ev[c % HostPipe::kChunks], ctx->stream));
+    return GX_OK;
+  };
+  int rc = GX_OK;
+  for (int64_t c = 0; c < nchunk && rc == GX_OK; c++) {
+    if (to_host) {
+      for (int64_t d = c == 0 ? 0 : c + HostPipe::kChunks - 1; d < std::min(nchunk, c + HostPipe::kChunks) && rc == GX_OK; d++)
+        rc = start(d);
+      if (rc != GX_OK) break;
+      if (hipEventSynchronize(hp.ev[c % HostPipe::kChunks]) != hipSuccess) rc = GX_EHIP;
+      else copy_chunk(c);
+    } else {
+      if (c >= HostPipe::kChunks && hipEventSynchronize(hp.ev[c % HostPipe::kChunks]) != hipSuccess) rc = GX_EHIP;
+      if (rc == GX_OK) copy_chunk(c);
+      if (rc == GX_OK) rc = start(c);
+    }
+  }
+  const hipError_t e = hipStreamSynchronize(ctx->stream);  // also after an error: the chunks are free again
+  if (rc == GX_EHIP || (rc == GX_OK && e != hipSuccess)) {
+    set_error("host transfer: %s", hipGetErrorString(e == hipSuccess ? hipGetLastError() : e));
+    return GX_EHIP;
+  }
+  return rc;
 }
 
 static bool geom_ok(const int dims[4], int Ls) {
@@ -813,86 +964,6 @@ int apply_mpcdagmpc(Op *op, Field *in, Field *out, const Gate *gate) {
   return apply_mpc(op, t, out, 1, gate);
 }
 
-// host (lexicographic, s innermost, AoS) <-> device (EO split, 64-entry blocks) index maps; the
-// stage holds 12 columns per half (half_pad entries each, padding zero) in the grouping of the
-// storage precision with the stage's type (FP64: 1 component per 16 bytes, FP32: 2); the FP16
-// packing reads an FP32-grouped stage
-template <typename T>
-static int vw_of() {
-  return 16 / (int)(2 * sizeof(T));
-}
-template <typename T>
-static void gather_to_device_layout(const Field *f, const double *host, T *stage) {
-  const int vw = vw_of<T>();
-  const Geom &g = f->g;
-  const int Ls = g.Ls;
-  const int64_t hp = 12 * g.half_pad();
-  if (f->subset == GX_FULL) {
-    parallel_for(g.V4, [&](int64_t b, int64_t e) {
-      for (int64_t s4 = b; s4 < e; s4++) {
-        int x[4];
-        coor_lex(g, s4, x);
-        const int cb = (x[0] + x[1] + x[2] + x[3]) & 1;
-        const int64_t h = half_index(g, x);
-        for (int s = 0; s < Ls; s++)
-          for (int k = 0; k < 12; k++) {
-            const double *src = host + ((s4 * Ls + s) * 12 + k) * 2;
-            T *dst = stage + (cb * hp + blk_index(h * Ls + s, k, 12, vw)) * 2;
-            dst[0] = (T)src[0];
-            dst[1] = (T)src[1];
-          }
-      }
-    });
-  } else {
-    parallel_for(g.H4, [&](int64_t b, int64_t e) {
-      for (int64_t h = b; h < e; h++)
-        for (int s = 0; s < Ls; s++)
-          for (int k = 0; k < 12; k++) {
-            const double *src = host + ((h * Ls + s) * 12 + k) * 2;
-            T *dst = stage + blk_index(h * Ls + s, k, 12, vw) * 2;
-            dst[0] = (T)src[0];
-            dst[1] = (T)src[1];
-          }
-    });
-  }
-}
-
-template <typename T>
-static void scatter_from_device_layout(const Field *f, const T *stage, double *host) {
-  const int vw = vw_of<T>();
-  const Geom &g = f->g;
-  const int Ls = g.Ls;
-  const int64_t hp = 12 * g.half_pad();
-  if (f->subset == GX_FULL) {
-    parallel_for(g.V4, [&](int64_t b, int64_t e) {
-      for (int64_t s4 = b; s4 < e; s4++) {
-        int x[4];
-        coor_lex(g, s4, x);
-        const int cb = (x[0] + x[1] + x[2] + x[3]) & 1;
-        const int64_t h = half_index(g, x);
-        for (int s = 0; s < Ls; s++)
-          for (int k = 0; k < 12; k++) {
-            double *dst = host + ((s4 * Ls + s) * 12 + k) * 2;
-            const T *src = stage + (cb * hp + blk_index(h * Ls + s, k, 12, vw)) * 2;
-            dst[0] = (double)src[0];
-            dst[1] = (double)src[1];
-          }
-      }
-    });
-  } else {
-    parallel_for(g.H4, [&](int64_t b, int64_t e) {
-      for (int64_t h = b; h < e; h++)
-        for (int s = 0; s < Ls; s++)
-          for (int k = 0; k < 12; k++) {
-            double *dst = host + ((h * Ls + s) * 12 + k) * 2;
-            const T *src = stage + blk_index(h * Ls + s, k, 12, vw) * 2;
-            dst[0] = (double)src[0];
-            dst[1] = (double)src[1];
-          }
-    });
-  }
-}
-
 int apply_full_m(Op *op, Field *in, Field *out, int dag) {
   if (tune_get(GX_TUNE_FUSED, in->prec))
     return by_prec(in->prec, [&](auto t) { return full_m_fused<decltype(t)>(op, in, out, dag); });
@@ -999,6 +1070,7 @@ int gx_ctx_destroy(gx_ctx c) {
   if (!c) return GX_OK;
   (void)hipStreamSynchronize(c->stream);
   block_work_free(c->block);
+  delete c->pipe;
   for (int i = 0; i < 16; i++) (void)hipEventDestroy(c->ev[i]);
   (void)hipFree(c->red_partial);
   (void)hipFree(c->digest);
@@ -1082,74 +1154,22 @@ int gx_field_destroy(gx_field f) {
   return GX_OK;
 }
 
-// FP16 storage <-> FP32 device layout on the host: per half block, 12 columns of binary16 pairs
-// scaled by each site's largest |component| (column 12, float).
-static void pack_f16(const Field *f, const float *in, uint32_t *out) {
-  const int64_t P = f->g.half_pad(), nh = f->halves();
-  for (int64_t hf = 0; hf < nh; hf++)
-    parallel_for(P, [&](int64_t b, int64_t e) {
-      const float *ih = in + hf * 12 * P * 2;
-      uint32_t *oh = out + hf * 13 * P;
-      for (int64_t i = b; i < e; i++) {
-        float m = 0.f;
-        for (int k = 0; k < 12; k++) {
-          const float *v = ih + blk_index(i, k, 12, 2) * 2;
-          m = std::max(m, std::max(std::fabs(v[0]), std::fabs(v[1])));
-        }
-        // a subnormal maximum is scaled by 2^64 (exact) first, as 1/m would overflow
-        const float up = (m > 0.f && m < FLT_MIN) ? 0x1p64f : 1.f;
-        const float inv = m > 0.f ? 1.f / (m * up) : 0.f;
-        for (int k = 0; k < 12; k++) {
-          const float *v = ih + blk_index(i, k, 12, 2) * 2;
-          const half_t pr[2] = {(half_t)((v[0] * up) * inv), (half_t)((v[1] * up) * inv)};
-          std::memcpy(&oh[blk_index(i, k, 13, 4)], pr, 4);
-        }
-        std::memcpy(&oh[blk_index(i, 12, 13, 4)], &m, 4);
-      }
-    });
-}
-
-static void unpack_f16(const Field *f, const uint32_t *in, float *out) {
-  const int64_t P = f->g.half_pad(), nh = f->halves();
-  for (int64_t hf = 0; hf < nh; hf++)
-    parallel_for(P, [&](int64_t b, int64_t e) {
-      const uint32_t *ih = in + hf * 13 * P;
-      float *oh = out + hf * 12 * P * 2;
-      for (int64_t i = b; i < e; i++) {
-        float m;
-        std::memcpy(&m, &ih[blk_index(i, 12, 13, 4)], 4);
-        for (int k = 0; k < 12; k++) {
-          half_t pr[2];
-          std::memcpy(pr, &ih[blk_index(i, k, 13, 4)], 4);
-          float *v = oh + blk_index(i, k, 12, 2) * 2;
-          v[0] = (float)pr[0] * m;
-          v[1] = (float)pr[1] * m;
-        }
-      }
-    });
-}
-
+// Host transfers move chunks of whole sites: the caller's threads copy a chunk between the user's memory and
+// pinned memory while the GPU writes or reads the neighbouring chunks, changing the layout on the way.
 int gx_field_import(gx_field f, const double *host) {
   GX_REQUIRE(f && host, GX_EINVAL, "null argument");
-  if (f->prec == GX_F16) {
-    std::vector<float> stage((size_t)f->stored() * 2, 0.f);
-    gather_to_device_layout<float>(f, host, stage.data());
-    std::vector<uint32_t> packed(f->bytes / 4);
-    pack_f16(f, stage.data(), packed.data());
-    GX_CHECK_HIP(hipMemcpyAsync(f->data, packed.data(), f->bytes, hipMemcpyHostToDevice, f->ctx->stream));
-    GX_CHECK_HIP(hipStreamSynchronize(f->ctx->stream));
-  } else if (f->prec == GX_F64) {
-    std::vector<double> stage((size_t)f->stored() * 2, 0.0);
-    gather_to_device_layout<double>(f, host, stage.data());
-    GX_CHECK_HIP(hipMemcpyAsync(f->data, stage.data(), f->bytes, hipMemcpyHostToDevice, f->ctx->stream));
-    GX_CHECK_HIP(hipStreamSynchronize(f->ctx->stream));
-  } else {
-    std::vector<float> stage((size_t)f->stored() * 2, 0.f);
-    gather_to_device_layout<float>(f, host, stage.data());
-    GX_CHECK_HIP(hipMemcpyAsync(f->data, stage.data(), f->bytes, hipMemcpyHostToDevice, f->ctx->stream));
-    GX_CHECK_HIP(hipStreamSynchronize(f->ctx->stream));
-  }
-  return GX_OK;
+  const size_t unit = (size_t)f->g.Ls * 12 * 16;
+  const int full = f->subset == GX_FULL;
+  return host_pipe(f->ctx, full ? f->g.V4 : f->g.H4, unit, false,
+                   [&](void *chunk, int64_t u0, int64_t u1) {
+                     return by_prec(f->prec, [&](auto t) {
+                       return launch_host_layout<decltype(t)>(f->g, full, 1, u0, u1 - u0, chunk, f->data,
+                                                              f->ctx->stream);
+                     });
+                   },
+                   [&](char *chunk, int64_t b, int64_t e, int64_t base) {
+                     std::memcpy(chunk + (b - base) * unit, (const char *)host + b * unit, (e - b) * unit);
+                   });
 }
 
 int gx_field_gaussian_slices(gx_field f, uint64_t seed, int s0, int ns) {
@@ -1214,25 +1234,18 @@ int gx_field_digest_slices(gx_field f, int s0, int ns, uint64_t *digest) {
 
 int gx_field_export(gx_field f, double *host) {
   GX_REQUIRE(f && host, GX_EINVAL, "null argument");
-  if (f->prec == GX_F16) {
-    std::vector<uint32_t> packed(f->bytes / 4);
-    GX_CHECK_HIP(hipMemcpyAsync(packed.data(), f->data, f->bytes, hipMemcpyDeviceToHost, f->ctx->stream));
-    GX_CHECK_HIP(hipStreamSynchronize(f->ctx->stream));
-    std::vector<float> stage((size_t)f->stored() * 2);
-    unpack_f16(f, packed.data(), stage.data());
-    scatter_from_device_layout<float>(f, stage.data(), host);
-  } else if (f->prec == GX_F64) {
-    std::vector<double> stage((size_t)f->stored() * 2);
-    GX_CHECK_HIP(hipMemcpyAsync(stage.data(), f->data, f->bytes, hipMemcpyDeviceToHost, f->ctx->stream));
-    GX_CHECK_HIP(hipStreamSynchronize(f->ctx->stream));
-    scatter_from_device_layout<double>(f, stage.data(), host);
-  } else {
-    std::vector<float> stage((size_t)f->stored() * 2);
-    GX_CHECK_HIP(hipMemcpyAsync(stage.data(), f->data, f->bytes, hipMemcpyDeviceToHost, f->ctx->stream));
-    GX_CHECK_HIP(hipStreamSynchronize(f->ctx->stream));
-    scatter_from_device_layout<float>(f, stage.data(), host);
-  }
-  return GX_OK;
+  const size_t unit = (size_t)f->g.Ls * 12 * 16;
+  const int full = f->subset == GX_FULL;
+  return host_pipe(f->ctx, full ? f->g.V4 : f->g.H4, unit, true,
+                   [&](void *chunk, int64_t u0, int64_t u1) {
+                     return by_prec(f->prec, [&](auto t) {
+                       return launch_host_layout<decltype(t)>(f->g, full, 0, u0, u1 - u0, chunk, f->data,
+                                                              f->ctx->stream);
+                     });
+                   },
+                   [&](char *chunk, int64_t b, int64_t e, int64_t base) {
+                     std::memcpy((char *)host + b * unit, chunk + (b - base) * unit, (e - b) * unit);
+                   });
 }
 
 int gx_field_checkerboard(gx_field f, int *cb) {
@@ -1603,8 +1616,7 @@ int gx_DhopDir(gx_op op, gx_field in, gx_field out, int dir, int disp) {
   const bool fwd = disp == 1;
   for (int cb = 0; cb < 2; cb++) {
     Field i = half_view(F(in), 1 - cb), o = half_view(F(out), cb);
-    GX_TRY(launch_hop_leg(op->g, dir, fwd, !fwd, 0, cb, i.data, cb == 0 ? Ue : Uo, nullptr, o.data, nullptr,
-                          op->ctx->stream));
+    GX_TRY(launch_hop_leg(op->g, dir, fwd, !fwd, cb, i.data, cb == 0 ? Ue : Uo, o.data, op->ctx->stream));
   }
   return GX_OK;
 }
@@ -1618,40 +1630,27 @@ static int dhop_deriv(Op *op, double *mat, Field *A, Field *B, int dag, int cb_f
   void *Ue, *Uo;
   GX_TRY(op_gauge(op, GX_F64, &Ue, &Uo));
   const Geom &g = op->g;
-  const size_t per = (size_t)g.H4 * 9 * 2 * sizeof(double);
-  double *dev = nullptr;
-  GX_CHECK_HIP(hipMalloc((void **)&dev, 4 * per));
-  std::vector<double> host(4 * per / sizeof(double));
-  int rc = GX_OK;
-  for (int cb = cb_first; cb <= cb_last && rc == GX_OK; cb++) {
-    const Field a = A->subset == GX_FULL ? half_view(A, cb) : *A;
-    const Field b = B->subset == GX_FULL ? half_view(B, 1 - cb) : *B;
-    for (int mu = 0; mu < 4 && rc == GX_OK; mu++)
-      rc = launch_hop_leg(g, mu, 1, dag ? 1 : 0, 1, cb, b.data, cb == 0 ? Ue : Uo, a.data, nullptr,
-                          dev + (size_t)mu * g.H4 * 18, op->ctx->stream);
-    hipError_t e = rc == GX_OK ? hipMemcpyAsync(host.data(), dev, 4 * per, hipMemcpyDeviceToHost, op->ctx->stream)
-                               : hipSuccess;
-    if (e == hipSuccess && rc == GX_OK) e = hipStreamSynchronize(op->ctx->stream);
-    if (e != hipSuccess) {
-      set_error("DhopDeriv: %s", hipGetErrorString(e));
-      rc = GX_EHIP;
-      break;
-    }
-    if (rc != GX_OK) break;
-    const int Lx = g.L[0], Ly = g.L[1], Lz = g.L[2], Lxh = Lx / 2;
-    for (int64_t h = 0; h < g.H4; h++) {
-      int64_t r = h / Lxh;
-      const int xh = (int)(h - r * Lxh), y = (int)(r % Ly);
-      r /= Ly;
-      const int z = (int)(r % Lz), t = (int)(r / Lz);
-      const int x = 2 * xh + ((cb + y + z + t) & 1);
-      const int64_t site = (((int64_t)t * Lz + z) * Ly + y) * Lx + x;
-      for (int mu = 0; mu < 4; mu++)
-        std::memcpy(mat + (site * 4 + mu) * 18, host.data() + ((size_t)mu * g.H4 + h) * 18, 18 * sizeof(double));
-    }
-  }
-  (void)hipFree(dev);
-  return rc;
+  const int mask = (cb_first == 0 ? 1 : 0) | (cb_last == 1 ? 2 : 0);
+  // half fields: only the one in mask is read
+  const void *pa[2] = {A->half(0), A->half(1)}, *pb[2] = {B->half(1), B->half(0)}, *pu[2] = {Ue, Uo};
+  constexpr size_t unit = 4 * 18 * sizeof(double);
+  return host_pipe(op->ctx, g.V4, unit, true,
+                   [&](void *chunk, int64_t u0, int64_t u1) {
+                     return launch_force(g, dag ? 1 : 0, mask, (uint32_t)u0, (uint32_t)(u1 - u0), pa, pb, pu, chunk,
+                                         op->ctx->stream);
+                   },
+                   [&](char *chunk, int64_t b, int64_t e, int64_t base) {
+                     if (mask == 3) {
+                       std::memcpy((char *)mat + b * unit, chunk + (b - base) * unit, (e - b) * unit);
+                       return;
+                     }
+                     for (int64_t s = b; s < e; s++) {
+                       int x[4];
+                       coor_lex(g, s, x);
+                       if ((mask >> ((x[0] + x[1] + x[2] + x[3]) & 1)) & 1)
+                         std::memcpy((char *)mat + s * unit, chunk + (s - base) * unit, unit);
+                     }
+                   });
 }
 
 static int deriv_args(Op *op, double *mat, Field *A, Field *B, bool full) {

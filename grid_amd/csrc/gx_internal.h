@@ -119,6 +119,7 @@ struct MrhsState : Gate {
   double tol2;
 };
 
+struct HostPipe;   // pinned chunks of host transfers (gx_api.hip)
 struct BlockWork;  // workspace of the block algebra (gx_solver.hip)
 void block_work_free(BlockWork *w);
 
@@ -131,6 +132,7 @@ struct Ctx {
   double *red_result = nullptr;      // [kRedSlots]
   double *pinned = nullptr;          // host mirror of red_result
   int next_slot = 0;
+  HostPipe *pipe = nullptr;          // pinned chunks of host transfers, from the first one on
   BlockWork *block = nullptr;        // created by the first block-algebra call, released with the context
 };
 
@@ -384,10 +386,18 @@ int launch_ms_update(Ctx *ctx, int64_t n, const void *r, void *p, const MsPtrs &
 int launch_gauge_stats(Ctx *ctx, const int dims[4], const void *U_dev, double *partial_dev, int nparts,
                        double *out_host);
 // One leg of the FP64 hop on the half fields of checkerboard cb_out (links U of cb_out): direction
-// mu, forward (fwd) or backward neighbour, projector (1 + gamma) (plus) or (1 - gamma).  mode 0:
-// out = the leg (half field of cb_out);  mode 1: mat[h][3][3] = sum over s and spin of leg (x) A^dag.
-int launch_hop_leg(const Geom &g, int mu, int fwd, int plus, int mode, int cb_out, const void *in, const void *U,
-                   const void *A, void *out, void *mat, hipStream_t st);
+// mu, forward (fwd) or backward neighbour, projector (1 + gamma) (plus) or (1 - gamma).
+int launch_hop_leg(const Geom &g, int mu, int fwd, int plus, int cb_out, const void *in, const void *U, void *out,
+                   hipStream_t st);
+// Force matrices mat[site][mu][3][3] of nsite lexicographic sites from site0 on (mat: the first one's), of the
+// checkerboards in mask: A[cb], U[cb] of the site's checkerboard, B[cb] the other one's half field.
+int launch_force(const Geom &g, int plus, int mask, uint32_t site0, uint32_t nsite, const void *const A[2],
+                 const void *const B[2], const void *const U[2], void *mat, hipStream_t st);
+// sites site0 .. site0 + nsite - 1 in the host's order and layout at host (pinned host memory) from or into
+// (import) a full or half field
+template <typename S>
+int launch_host_layout(const Geom &g, int full, int import, int64_t site0, int64_t nsite, void *host, void *field,
+                       hipStream_t st);
 
 // Slice matrices of FP64 fields with nhalf (1 or 2) checkerboard halves (sliceInnerProductMatrix,
 // sliceMaddMatrix).  ipm: out_dev[s * Ls + t] = sum conj(x_s) y_t (double2), through nparts

@@ -2979,74 +2979,190 @@ static __global__ void __launch_bounds__(256) k_digest(const uint64_t *__restric
   if (threadIdx.x == 0) atomicAdd(out, (unsigned long long)(part[0] + part[1] + part[2] + part[3]));
 }
 
-// ---------------- single-direction hop and force legs (WilsonKernels DhopDirKernel,
-// WilsonKernelsImplementation.h:375-410; WilsonImpl::InsertForce5D, WilsonImpl.h:193-238) ----------
-// One thread per output half-site h of checkerboard cb_out, all Ls slices: the leg of direction MU
-// at the forward (FWD: point MU, link Uds[MU](x)) or backward (point MU + 4, link Uds[MU + 4](x))
-// neighbour with projector (1 + gamma_MU) (PLUS) or (1 - gamma_MU):
-//   chi(h, s) = Uds[P](h) recon(project(in(nb_P(h), s))).
-// MODE 0 writes out(h, s) = chi (DhopDir); MODE 1 writes mat[h][a][b] = sum_{s, spin} chi_a conj(A_b)
-// (the colour outer product of InsertForce5D).  FP64.
-template <int MU, bool FWD, bool PLUS, int MODE>
-static __global__ void __launch_bounds__(256) k_hop_leg(KGeom g, int Ls, int cb_out, const cx<double> *__restrict__ in,
-                                                        const cx<double> *__restrict__ U,
-                                                        const cx<double> *__restrict__ A, cx<double> *__restrict__ out,
-                                                        cx<double> *__restrict__ mat) {
-  const uint32_t H4 = (uint32_t)g.H4;
-  for (uint32_t h = blockIdx.x * blockDim.x + threadIdx.x; h < H4; h += gridDim.x * blockDim.x) {
-    const uint32_t r1 = fdiv(h, g.fLxh), r2 = fdiv(r1, g.fL1), r3 = fdiv(r2, g.fL2);
-    const int xh = (int)(h - r1 * (uint32_t)g.Lxh);
-    const int y = (int)(r1 - r2 * (uint32_t)g.L[1]);
-    const int z = (int)(r2 - r3 * (uint32_t)g.L[2]);
-    const int t = (int)r3;
-    const int x = 2 * xh + ((cb_out + y + z + t) & 1);
-    uint32_t n;
-    if (MU == 0) {
-      const int xn = FWD ? (x + 1 == g.L[0] ? 0 : x + 1) : (x == 0 ? g.L[0] - 1 : x - 1);
-      n = h - xh + (xn >> 1);
-    } else {
-      const int c = MU == 1 ? y : (MU == 2 ? z : t), L = g.L[MU];
-      const uint32_t st = (uint32_t)(MU == 1 ? g.sY : (MU == 2 ? g.sZ : g.sT));
-      if (FWD) n = (c + 1 == L) ? h - (uint32_t)(L - 1) * st : h + st;
-      else n = (c == 0) ? h + (uint32_t)(L - 1) * st : h - st;
+// ---------------- host layout <-> device layout ----------------
+// The entries of sites site0 .. of the host order (full fields: lexicographic site, then slice; half fields:
+// half site, then slice; 12 complex doubles each), n of them, at host, which is pinned host memory written and read in place:
+// whole wave rows of consecutive doubles on that side, through LDS, the field's blocks on the other.  What
+// bounds the pass is PCIe (57 GB/s pinned) and the threads that copy between the chunks and the user's memory:
+// 46 MB up and down 26.8 ms with the layout changed on the host and pageable copies, 3.4 ms so.
+constexpr int kHostEnt = 128;  // entries per workgroup, one per thread
+struct HostGeom {
+  KGeom g;
+  FDiv fLs, fL0;
+  int full;
+};
+
+// the checkerboard (half fields: 0) and half-lattice index of host site `site`
+__device__ __forceinline__ uint32_t host_site(const HostGeom &hg, uint32_t site, int &cb) {
+  cb = 0;
+  if (!hg.full) return site;
+  const uint32_t r1 = fdiv(site, hg.fL0), x = site - r1 * hg.fL0.d;
+  const uint32_t r2 = fdiv(r1, hg.g.fL1), r3 = fdiv(r2, hg.g.fL2);
+  const uint32_t y = r1 - r2 * hg.g.fL1.d, z = r2 - r3 * hg.g.fL2.d, t = r3;
+  cb = (int)((x + y + z + t) & 1);
+  return (x >> 1) + (uint32_t)hg.g.Lxh * r1;
+}
+
+template <typename S, bool IMPORT>
+__global__ void __launch_bounds__(kHostEnt) k_host_layout(HostGeom hg, uint32_t site0, uint32_t n, double2 *__restrict__ host,
+                                                          cx<S> *__restrict__ field) {
+  typedef typename Sto<S>::C T;
+  __shared__ double2 sh[12 * kHostEnt];
+  const uint32_t t = threadIdx.x, b0 = blockIdx.x * kHostEnt, m = min((uint32_t)kHostEnt, n - b0);
+  double2 *row = host + (size_t)b0 * 12;
+  int cb;
+  const uint32_t l = b0 + min(t, m - 1), ls = fdiv(l, hg.fLs);
+  const int64_t e = (int64_t)host_site(hg, site0 + ls, cb) * hg.fLs.d + (l - ls * hg.fLs.d);
+  cx<S> *half = field + (size_t)cb * Sto<S>::NCOL * hg.g.stride;
+  cx<T> v[12];
+  if (IMPORT) {
+    for (uint32_t i = t; i < 12 * m; i += kHostEnt) sh[i] = row[i];
+    __syncthreads();
+    if (t >= m) return;
+#pragma unroll
+    for (int k = 0; k < 12; k++) v[k] = {(T)sh[12 * t + k].x, (T)sh[12 * t + k].y};
+    store_site<S>(half, v, e, false);
+  } else {
+    if (t < m) {
+      load_site<S>(v, half, e);
+#pragma unroll
+      for (int k = 0; k < 12; k++) sh[12 * t + k] = {(double)v[k].r, (double)v[k].i};
     }
-    constexpr int P = FWD ? MU : MU + 4;
-    cx<double> u[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++) u[k] = U[(int64_t)(P * 9 + k) * H4 + h];
-    cx<double> m[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++) m[k] = {0, 0};
-    for (int s = 0; s < Ls; s++) {
-      cx<double> f[12], hs[6], acc[12];
-      load_site<double>(f, in, (int64_t)n * Ls + s);
-      project<double, MU, PLUS>(f, hs);
-#pragma unroll
-      for (int k = 0; k < 12; k++) acc[k] = {0, 0};
-#pragma unroll
-      for (int r = 0; r < 3; r++)
-        recon_colour<double, MU, PLUS>(acc, r, su3_row<double>(u + 3 * r, hs), su3_row<double>(u + 3 * r, hs + 3));
-      if (MODE == 0) {
-        store_site<double>(out, acc, (int64_t)h * Ls + s, false);
-      } else {
-        cx<double> a[12];
-        load_site<double>(a, A, (int64_t)h * Ls + s);
-#pragma unroll
-        for (int sp = 0; sp < 4; sp++)
-#pragma unroll
-          for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = 0; j < 3; j++) {
-              const cx<double> c = acc[sp * 3 + i], d = a[sp * 3 + j];  // c conj(d)
-              m[i * 3 + j].r = fma(c.r, d.r, fma(c.i, d.i, m[i * 3 + j].r));
-              m[i * 3 + j].i = fma(c.i, d.r, fma(-c.r, d.i, m[i * 3 + j].i));
-            }
-      }
-    }
-    if (MODE == 1)
-#pragma unroll
-      for (int k = 0; k < 9; k++) mat[(int64_t)h * 9 + k] = m[k];
+    __syncthreads();
+    for (uint32_t i = t; i < 12 * m; i += kHostEnt) row[i] = sh[i];
   }
+}
+
+template <typename S>
+int launch_host_layout(const Geom &g, int full, int import, int64_t site0, int64_t nsite, void *host, void *field,
+                       hipStream_t st) {
+  if (site0 + nsite >= (int64_t)1 << 31 || nsite * g.Ls >= (int64_t)1 << 31) {
+    set_error("host transfer: lattice too large for 32-bit site indexing");
+    return GX_EINVAL;
+  }
+  const uint32_t n = (uint32_t)(nsite * g.Ls);
+  HostGeom hg{kgeom(g), make_fdiv((uint32_t)g.Ls), make_fdiv((uint32_t)g.L[0]), full};
+  const uint32_t nb = (n + kHostEnt - 1) / kHostEnt;
+  if (import)
+    hipLaunchKernelGGL((k_host_layout<S, true>), dim3(nb), dim3(kHostEnt), 0, st, hg, (uint32_t)site0, n, (double2 *)host,
+                       (cx<S> *)field);
+  else
+    hipLaunchKernelGGL((k_host_layout<S, false>), dim3(nb), dim3(kHostEnt), 0, st, hg, (uint32_t)site0, n, (double2 *)host,
+                       (cx<S> *)field);
+  GX_CHECK_HIP(hipGetLastError());
+  return GX_OK;
+}
+
+// ---------------- single-direction hop (WilsonKernels DhopDirKernel,
+// WilsonKernelsImplementation.h:375-410) ----------------
+// One thread per output entry (h, s) of checkerboard cb_out: the leg of direction MU at the forward (FWD:
+// point MU, link Uds[MU](x)) or backward (point MU + 4, link Uds[MU + 4](x)) neighbour with projector (1 +
+// gamma_MU) (PLUS) or (1 - gamma_MU): out(h, s) = Uds[P](h) recon(project(in(nb_P(h), s))).  FP64.
+template <int MU, bool FWD, bool PLUS>
+static __global__ void __launch_bounds__(256) k_hop_leg(KGeom g, FDiv fLS, int cb_out, uint32_t nent,
+                                                        const cx<double> *__restrict__ in,
+                                                        const cx<double> *__restrict__ U, cx<double> *__restrict__ out) {
+  const uint32_t H4 = (uint32_t)g.H4, e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= nent) return;
+  const uint32_t h = fdiv(e, fLS), s = e - h * fLS.d;
+  constexpr int P = FWD ? MU : MU + 4;
+  cx<double> f[12], hs[6], acc[12];
+  load_site<double>(f, in, (int64_t)site_neighbour<P>(g, h, cb_out) * fLS.d + s);
+  project<double, MU, PLUS>(f, hs);
+#pragma unroll
+  for (int k = 0; k < 12; k++) acc[k] = {0, 0};
+#pragma unroll
+  for (int r = 0; r < 3; r++) {
+    cx<double> u[3];
+#pragma unroll
+    for (int b = 0; b < 3; b++) u[b] = U[(int64_t)(P * 9 + 3 * r + b) * H4 + h];
+    recon_colour<double, MU, PLUS>(acc, r, su3_row<double>(u, hs), su3_row<double>(u, hs + 3));
+  }
+  store_site<double>(out, acc, (int64_t)e, false);
+}
+
+// ---------------- fermion force (WilsonImpl::InsertForce5D, WilsonImpl.h:193-238) ----------------
+// mat[site][mu] = sum over s and spin of Btilde_mu (x) A^dag with Btilde_mu = Uds[mu](x) P B(x + mu) and P the
+// projector (1 +- gamma_mu), for sites site0 .. site0 + nsite - 1 in lexicographic order whose checkerboard is
+// in mask (the others' places are left alone).  The projector acts on A as well and the link factors out of the
+// sum: mat = Uds[mu] sum_s sum_j (P B)_j (x) (P A)_j^dag over the two projected spins, half the products and one
+// link multiplication per site and direction.  One wave takes 64 / LP whole sites, LP = min(Ls, 64) lanes each;
+// A is read once for the four directions, the lanes' matrices are added in LDS, and the result goes to pinned
+// host memory in the user's order: 16^3 x 32 x 8, both checkerboards, 1.9 ms of kernels (one thread per site,
+// every slice after another, a launch per direction) and 20.4 ms a call before, 3.3 ms a call now, which is the
+// 75 MB over PCIe and into the user's array.
+template <bool PLUS, int MU>
+__device__ __forceinline__ void force_dir(const KGeom &g, uint32_t h, int cb, uint32_t s, uint32_t LP, uint32_t LS,
+                                          bool on, const cx<double> *__restrict__ A, const cx<double> *__restrict__ B,
+                                          cx<double> *m) {
+#pragma unroll
+  for (int k = 0; k < 9; k++) m[k] = {0, 0};
+  if (!on) return;
+  const uint32_t n = site_neighbour<MU>(g, h, cb);
+  for (; s < LS; s += LP) {
+    cx<double> f[12], hb[6], ha[6];
+    load_site<double>(f, B, (int64_t)n * LS + s);
+    project<double, MU, PLUS>(f, hb);
+    load_site<double>(f, A, (int64_t)h * LS + s);
+    project<double, MU, PLUS>(f, ha);
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+          const cx<double> c = hb[j * 3 + a], d = ha[j * 3 + b];  // c conj(d)
+          m[a * 3 + b].r = fma(c.r, d.r, fma(c.i, d.i, m[a * 3 + b].r));
+          m[a * 3 + b].i = fma(c.i, d.r, fma(-c.r, d.i, m[a * 3 + b].i));
+        }
+  }
+}
+
+struct ForceArgs {
+  const cx<double> *A[2], *B[2], *U[2];  // B[cb]: B's other checkerboard
+  uint32_t LS, LP, SPW, site0, nsite;
+  int mask;
+};
+
+template <bool PLUS>
+static __global__ void __launch_bounds__(64) k_force(ForceArgs F, HostGeom hg, FDiv fLP, double2 *__restrict__ mat) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  cx<double> *sm = reinterpret_cast<cx<double> *>(lds_raw);        // [9][64] the lanes' matrices
+  cx<double> *sums = sm + 9 * 64;                                  // [SPW][9]
+  cx<double> *res = sums + 9 * F.SPW;                              // [SPW][4][9]
+  uint32_t *where = reinterpret_cast<uint32_t *>(res + 36 * F.SPW);  // [SPW] half index, bit 31 = cb
+  const uint32_t lane = threadIdx.x, ls = fdiv(lane, fLP), s = lane - ls * F.LP;
+  const uint32_t l0 = blockIdx.x * F.SPW, m = min(F.SPW, F.nsite - l0), H4 = (uint32_t)hg.g.H4;
+  const bool mine = ls < m;
+  int cb = 0;
+  const uint32_t h = host_site(hg, F.site0 + l0 + (mine ? ls : 0), cb);
+  const bool on = mine && ((F.mask >> cb) & 1);
+  if (mine && s == 0) where[ls] = h | (uint32_t)cb << 31;
+  cx<double> v[9];
+#define GX_FORCE_DIR(MU)                                                                                         \
+  force_dir<PLUS, MU>(hg.g, h, cb, s, F.LP, F.LS, on, F.A[cb], F.B[cb], v);                                      \
+  wave_sync();                                                                                                   \
+  _Pragma("unroll") for (int k = 0; k < 9; k++) sm[k * 64 + lane] = v[k];                                        \
+  wave_sync();                                                                                                   \
+  for (uint32_t i = lane; i < 9 * m; i += 64) {                                                                  \
+    const uint32_t site = i / 9, k = i - site * 9;                                                               \
+    cx<double> t = {0, 0};                                                                                       \
+    for (uint32_t q = 0; q < F.LP; q++) t = cadd(t, sm[k * 64 + site * F.LP + q]);                               \
+    sums[i] = t;                                                                                                 \
+  }                                                                                                              \
+  wave_sync();                                                                                                   \
+  for (uint32_t i = lane; i < 9 * m; i += 64) {                                                                  \
+    const uint32_t site = i / 9, k = i - site * 9, a = k / 3, b = k - 3 * a, w = where[site];                    \
+    const cx<double> *u = F.U[w >> 31] + (size_t)(MU * 9 + 3 * a) * H4 + (w & 0x7fffffffu);                      \
+    cx<double> ur[3] = {u[0], u[H4], u[2 * (size_t)H4]}, hc[3];                                                  \
+    _Pragma("unroll") for (int c = 0; c < 3; c++) hc[c] = sums[site * 9 + 3 * c + b];                            \
+    res[(site * 4 + MU) * 9 + k] = su3_row<double>(ur, hc);                                                      \
+  }
+  GX_FORCE_DIR(0) GX_FORCE_DIR(1) GX_FORCE_DIR(2) GX_FORCE_DIR(3)
+#undef GX_FORCE_DIR
+  wave_sync();
+  for (uint32_t i = lane; i < 36 * m; i += 64)
+    if ((F.mask >> (where[i / 36] >> 31)) & 1) mat[(size_t)l0 * 36 + i] = {res[i].r, res[i].i};
 }
 
 // ---------------- gauge statistics (WilsonLoops.h:102-126,203-219) ----------------
@@ -3616,23 +3732,22 @@ int launch_slice_ipm(Ctx *ctx, const Geom &g, int nhalf, const void *x, const vo
   return GX_OK;
 }
 
-int launch_hop_leg(const Geom &g, int mu, int fwd, int plus, int mode, int cb_out, const void *in, const void *U,
-                   const void *A, void *out, void *mat, hipStream_t st) {
+int launch_hop_leg(const Geom &g, int mu, int fwd, int plus, int cb_out, const void *in, const void *U, void *out,
+                   hipStream_t st) {
   if (mu < 0 || mu > 3) {
     set_error("hop leg: direction %d", mu);
     return GX_EINVAL;
   }
   const KGeom k = kgeom(g);
-  const uint32_t nb = (uint32_t)((g.H4 + 255) / 256);
-  const cx<double> *pin = (const cx<double> *)in, *pU = (const cx<double> *)U, *pA = (const cx<double> *)A;
-  cx<double> *pout = (cx<double> *)out, *pmat = (cx<double> *)mat;
-#define GX_LEG(M, F, P, MODE)                                                                                    \
-  hipLaunchKernelGGL((k_hop_leg<M, F, P, MODE>), dim3(nb), dim3(256), 0, st, k, g.Ls, cb_out, pin, pU, pA, pout, pmat)
-#define GX_LEG_MODE(M, F, P) \
-  if (mode == 0) GX_LEG(M, F, P, 0); else GX_LEG(M, F, P, 1)
+  const uint32_t nent = (uint32_t)(g.H4 * g.Ls), nb = (nent + 255) / 256;
+  const FDiv f = make_fdiv((uint32_t)g.Ls);
+  const cx<double> *pin = (const cx<double> *)in, *pU = (const cx<double> *)U;
+  cx<double> *pout = (cx<double> *)out;
+#define GX_LEG(M, F, P) \
+  hipLaunchKernelGGL((k_hop_leg<M, F, P>), dim3(nb), dim3(256), 0, st, k, f, cb_out, nent, pin, pU, pout)
 #define GX_LEG_FP(M)                                              \
-  if (fwd) { if (plus) GX_LEG_MODE(M, true, true); else GX_LEG_MODE(M, true, false); } \
-  else { if (plus) GX_LEG_MODE(M, false, true); else GX_LEG_MODE(M, false, false); }
+  if (fwd) { if (plus) GX_LEG(M, true, true); else GX_LEG(M, true, false); } \
+  else { if (plus) GX_LEG(M, false, true); else GX_LEG(M, false, false); }
   switch (mu) {
     case 0: GX_LEG_FP(0); break;
     case 1: GX_LEG_FP(1); break;
@@ -3640,8 +3755,32 @@ int launch_hop_leg(const Geom &g, int mu, int fwd, int plus, int mode, int cb_ou
     default: GX_LEG_FP(3); break;
   }
 #undef GX_LEG_FP
-#undef GX_LEG_MODE
 #undef GX_LEG
+  GX_CHECK_HIP(hipGetLastError());
+  return GX_OK;
+}
+
+int launch_force(const Geom &g, int plus, int mask, uint32_t site0, uint32_t nsite, const void *const A[2],
+                 const void *const B[2], const void *const U[2], void *mat, hipStream_t st) {
+  ForceArgs F{};
+  for (int cb = 0; cb < 2; cb++) {
+    F.A[cb] = (const cx<double> *)A[cb];
+    F.B[cb] = (const cx<double> *)B[cb];
+    F.U[cb] = (const cx<double> *)U[cb];
+  }
+  F.LS = (uint32_t)g.Ls;
+  F.LP = F.LS < 64 ? F.LS : 64;
+  F.SPW = 64 / F.LP;
+  F.site0 = site0;
+  F.nsite = nsite;
+  F.mask = mask;
+  HostGeom hg{kgeom(g), make_fdiv(1), make_fdiv((uint32_t)g.L[0]), 1};
+  const uint32_t nb = (nsite + F.SPW - 1) / F.SPW;
+  const size_t lds = (9 * 64 + 45 * (size_t)F.SPW) * 16 + 4 * (size_t)F.SPW;
+  if (plus)
+    hipLaunchKernelGGL((k_force<true>), dim3(nb), dim3(64), lds, st, F, hg, make_fdiv(F.LP), (double2 *)mat);
+  else
+    hipLaunchKernelGGL((k_force<false>), dim3(nb), dim3(64), lds, st, F, hg, make_fdiv(F.LP), (double2 *)mat);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
@@ -3751,6 +3890,7 @@ int launch_digest_slices(Ctx *ctx, const Geom &g, const void *full, int s0, int 
   template int launch_dhop_epi<S>(const Geom &, const void *, void *, const void *, int, int, const Gate *,       \
                                   hipStream_t, int, const void *, const void *, double, int, const void *,         \
                                   const HopFuse *);                                                                \
+  template int launch_host_layout<S>(const Geom &, int, int, int64_t, int64_t, void *, void *, hipStream_t);       \
   template bool hop_split<S>(const Geom &);                                                                        \
   template int launch_hop_split<S>(const Geom &, int, int, const void *const[2], void *const[2],                   \
                                    const void *const[2], const void *const[2], int, const Gate *, hipStream_t,    \
