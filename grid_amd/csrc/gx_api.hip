@@ -855,7 +855,7 @@ int apply_mooee(Op *op, Field *in, Field *out, int which, const Gate *gate) {
 // in for the second hop costs more than the epilogue's few LDS reads: MpcDagMpc FP32 on 20 x 12 x 18 x 28
 // x 10 265 us with it, 223 us without.
 template <typename T>
-static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, const HopFuse *fz) {
+static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, const HopFuse *fz, const void *first) {
   const int prec = in->prec, cb_in = in->cb, cb_mid = 1 - cb_in;
   void *Ue, *Uo;
   GX_TRY(op_gauge(op, prec, &Ue, &Uo));
@@ -876,8 +876,9 @@ static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, c
     GX_TRY(op_smat(op, prec, dag ? Op::S_INVDAG_MEODAG5D : Op::S_MEO5D_INV, &m_p));
     GX_TRY(op_band(op, prec, dag ? Op::S_MEOOEDAG5D : Op::S_MEOOE5D, &b_meo));
     GX_TRY(op_band(op, prec, dag ? Op::S_MOOEEDAG : Op::S_MOOEE, &b_mooee));
-    const void *first = in->data;
-    if (!dag) {
+    if (dag) {
+      first = in->data;
+    } else if (!first) {
       GX_TRY(launch_band<T>(g, in->data, nullptr, t0->data, b_meo, 0, gate, st));
       first = t0->data;
     }
@@ -942,10 +943,10 @@ static int full_m_fused(Op *op, Field *in, Field *out, int dag) {
   return GX_OK;
 }
 
-int apply_mpc(Op *op, Field *in, Field *out, int dag, const Gate *gate, const HopFuse *fz) {
+int apply_mpc(Op *op, Field *in, Field *out, int dag, const Gate *gate, const HopFuse *fz, const void *first) {
   if (fz && fz->nparts) *fz->nparts = 0;
   if (tune_get(GX_TUNE_FUSED, in->prec))
-    return by_prec(in->prec, [&](auto t) { return mpc_fused<decltype(t)>(op, in, out, dag, gate, fz); });
+    return by_prec(in->prec, [&](auto t) { return mpc_fused<decltype(t)>(op, in, out, dag, gate, fz, first); });
   Field *t1 = op_tmp(op, in->prec, 0), *t2 = op_tmp(op, in->prec, 1);
   if (!t1 || !t2) return GX_ENOMEM;
   GX_TRY(apply_meooe(op, in, t1, dag, gate));
@@ -965,8 +966,11 @@ int apply_mpcdagmpc(Op *op, Field *in, Field *out, const Gate *gate) {
 }
 
 int apply_full_m(Op *op, Field *in, Field *out, int dag) {
-  if (tune_get(GX_TUNE_FUSED, in->prec))
-    return by_prec(in->prec, [&](auto t) { return full_m_fused<decltype(t)>(op, in, out, dag); });
+  // FP16 storage keeps the separate passes: each of them rounds, and the fused sum would differ by that
+  if (tune_get(GX_TUNE_FUSED, in->prec) && in->prec != GX_F16) {
+    if (in->prec == GX_F64) return full_m_fused<double>(op, in, out, dag);
+    return full_m_fused<float>(op, in, out, dag);
+  }
   for (int cb = 0; cb < 2; cb++) {
     Field in_other = half_view(in, 1 - cb), in_same = half_view(in, cb), o = half_view(out, cb);
     GX_TRY(apply_meooe(op, &in_other, &o, dag));

@@ -251,8 +251,8 @@ struct HopFuse {
   const double *a = nullptr;
   int astride = 1;
   int total = 0;   // 1: npart holds one sum per tile, over its slices (single-RHS CG)
-  // leg-per-wave kernel, single-RHS CG: a = c / d from the state cur and the nd partials of d (in place of
-  // *a, which has to be given all the same), left in nxt
+  // single-RHS CG, r given: a = c / d from the state cur and the nd partials of d, left in nxt (in place of
+  // *a, which has to be given all the same)
   const CGState *cur = nullptr;
   CGState *nxt = nullptr;
   const double *dpart = nullptr;
@@ -330,6 +330,10 @@ template <typename T>
 int launch_cg_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, void *r, const void *mmp, CGState *state);
 template <typename S>
 int launch_cg_update(Ctx *ctx, int64_t nsites, int64_t stride, void *psi, void *p, const void *r, CGState *state);
+// the same that also leaves q = A(p) of the new p, A's bands as of launch_band (dag 0); FP64 and FP32 half fields
+template <typename S>
+int launch_cg_update_band(Ctx *ctx, const Geom &g, void *psi, void *p, const void *r, void *q, const void *bands,
+                          const CGState *cur, CGState *nxt, const double *partial, int np);
 // the update with the norm finaliser in it: np partials of |r|^2 and the state cur give the next state nxt
 template <typename S>
 int launch_cg_update_fin(Ctx *ctx, int64_t nsites, int64_t stride, void *psi, void *p, const void *r, const CGState *cur,
@@ -443,7 +447,9 @@ int apply_dhop_half(Op *op, Field *in, Field *out, int cb_out, int dag, const Ga
 int apply_meooe(Op *op, Field *in, Field *out, int dag, const Gate *gate = nullptr);
 int apply_mooee(Op *op, Field *in, Field *out, int which, const Gate *gate = nullptr);
 // fz: HopFuse for the second hop (Wilson, fused Mpc path; *fz->nparts = 0 otherwise)
-int apply_mpc(Op *op, Field *in, Field *out, int dag, const Gate *gate = nullptr, const HopFuse *fz = nullptr);
+// first: Meooe5D in when the caller has it already (Cayley, dag 0, fused)
+int apply_mpc(Op *op, Field *in, Field *out, int dag, const Gate *gate = nullptr, const HopFuse *fz = nullptr,
+              const void *first = nullptr);
 // out = MpcDag Mpc in through temporary 2 (left holding Mpc in)
 int apply_mpcdagmpc(Op *op, Field *in, Field *out, const Gate *gate = nullptr);
 int apply_full_m(Op *op, Field *in, Field *out, int dag);

@@ -582,7 +582,35 @@ struct HopEpi {
   const double *acoef;
   int astride;
   int total;      // npart holds one sum per tile, over its slices
+  // RUPD in a single-RHS CG: with cur set, a = c / d with c of the state cur and d the sum of nd partials
+  // (every workgroup adds them for itself, in the same order), left in nxt; *acoef otherwise
+  const CGState *cur;
+  CGState *nxt;
+  const double *dpart;
+  int nd;
 };
+
+// this thread's share of the partials of d, and its wave's sum in dsh (one per wave)
+template <typename S>
+__device__ __forceinline__ double d_share(const HopEpi<S> &ep) {
+  double ds = 0;
+  if (ep.cur)
+    for (int i = threadIdx.x; i < ep.nd; i += blockDim.x) ds += ep.dpart[i];
+  return ds;
+}
+// a of slice s from the wave sums of d (after a barrier); `first`: the thread that leaves them in nxt
+template <typename S>
+__device__ __forceinline__ double rupd_coef(const HopEpi<S> &ep, const double *dsh, uint32_t s, bool first) {
+  if (!ep.cur) return ep.acoef[ep.astride * s];
+  double d = 0;
+  for (uint32_t i = 0; i < blockDim.x / 64; i++) d += dsh[i];
+  const double a = ep.cur->c / d;
+  if (first) {
+    ep.nxt->d = d;
+    ep.nxt->a = a;
+  }
+  return a;
+}
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -606,6 +634,34 @@ __device__ __forceinline__ void write_norms(double *npart, uint32_t tile, uint32
 // the diagonal, then the coefficient of the neighbour slice_nbr(s, chi, dag).
 __host__ __device__ __forceinline__ uint32_t slice_nbr(uint32_t s, int chi, bool dag, uint32_t LB) {
   return ((chi == 0) == dag) ? (s + 1 == LB ? 0 : s + 1) : (s == 0 ? LB - 1 : s - 1);
+}
+
+// The two bands' sum d own + f w (w the neighbour's value).  FP16 storage adds in slice order (`low`: the
+// neighbour is the lower slice), as a sum over the whole row would, and add_rounded adds B(phi) as a field of
+// FP16 storage would hold it: what its operators return does not depend on which passes are fused.
+template <typename S>
+__device__ __forceinline__ cx<typename Sto<S>::C> band_sum(typename Sto<S>::C d, cx<typename Sto<S>::C> own,
+                                                           typename Sto<S>::C f, cx<typename Sto<S>::C> w, bool low) {
+  if (Sto<S>::H && low) return {fma(d, own.r, mul_rounded(f, w.r)), fma(d, own.i, mul_rounded(f, w.i))};
+  return {fma(f, w.r, d * own.r), fma(f, w.i, d * own.i)};
+}
+// acc[0 .. N) += v as stored in FP16 under the site maximum m
+template <int N>
+__device__ __forceinline__ void add_rounded(cx<float> *acc, const cx<float> *v, float m) {
+  const bool tiny = __builtin_expect(m > 0.f && m < FLT_MIN, 0);
+  const float up = tiny ? 0x1p64f : 1.f, inv = m > 0.f ? 1.f / (m * up) : 0.f;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    acc[k].r = fma(m, (float)to_half(v[k].r * up, inv), acc[k].r);
+    acc[k].i = fma(m, (float)to_half(v[k].i * up, inv), acc[k].i);
+  }
+}
+template <int N>
+__device__ __forceinline__ float max_part(const cx<float> *v) {
+  float m = 0.f;
+#pragma unroll
+  for (int k = 0; k < N; k++) m = fmaxf(m, fmaxf(fabsf(v[k].r), fabsf(v[k].i)));
+  return m;
 }
 
 // LDS written by a wave and read by other lanes of the same wave
@@ -668,6 +724,8 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   const uint32_t ugrp = threadIdx.x / SPB, usite = threadIdx.x - ugrp * SPB;
   const bool ustage = LDSU && ugrp < (uint32_t)G && h0 + usite < H4;
   cx<T> ureg[NU];
+  double ds = 0;  // loaded first: loads return in order, and this one is waited for first
+  if (RUPD) ds = d_share(ep);
   if (LDSU) {
     const uint32_t hs = sweep && ustage ? sweep_site(g, h0 + usite) : h0 + usite;
 #pragma unroll
@@ -679,6 +737,11 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   cx<T> fa[12], fb[12];
   T sa = load_site_raw<S>(fa, in, leg_idx<DAG, ORD, 0>(nb, LS, s)), sb = (T)1;
   if (PF) sb = load_site_raw<S>(fb, in, leg_idx<DAG, ORD, 1>(nb, LS, s));
+  __shared__ double dsh[RUPD ? 4 : 1];
+  if (RUPD && ep.cur) {
+    ds = wave_sum(ds);
+    if (lane == 0) dsh[w] = ds;
+  }
   if (LDSU) {
     if (ugrp < (uint32_t)G) {
 #pragma unroll
@@ -688,6 +751,12 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  // the update's coefficient while the first neighbours are on their way
+  double ra = 0;
+  if constexpr (RUPD) {
+    if (!LDSU) __syncthreads();
+    ra = rupd_coef(ep, dsh, s, tile == 0 && threadIdx.x == 0);
   }
   if (!MAT && !BAND && !NORM && !valid) return;
   const cx<T> *ul = lds + (LDSU ? lsb * kLinkPad : 0);
@@ -734,13 +803,11 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
       wave_sync();
 #pragma unroll
       for (int chi = 0; chi < 2; chi++) {
-        const int n = row + (int)slice_nbr(s, chi, true, LS);
+        const int sn = (int)slice_nbr(s, chi, true, LS), n = row + sn;
         const T d = ep.alpha * ep.mat[2 * chi * LS + s], f = ep.alpha * ep.mat[(2 * chi + 1) * LS + s];
 #pragma unroll
-        for (int k = 6 * chi; k < 6 * chi + 6; k++) {
-          const cx<T> v = stg[k * 64 + (n & 63)];
-          acc[k] = {fma(f, v.r, d * acc[k].r), fma(f, v.i, d * acc[k].i)};
-        }
+        for (int k = 6 * chi; k < 6 * chi + 6; k++)
+          acc[k] = band_sum<S>(d, acc[k], f, stg[k * 64 + (n & 63)], sn < s);
       }
       wave_sync();
     } else {
@@ -754,15 +821,20 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
     wave_sync();
 #pragma unroll
     for (int chi = 0; chi < 2; chi++) {
-      const int n = row + (int)slice_nbr(s, chi, DAG, LS);
+      const int sn = (int)slice_nbr(s, chi, DAG, LS), n = row + sn;
       const T d = ep.coef[2 * chi * LS + s], f = ep.coef[(2 * chi + 1) * LS + s];
 #pragma unroll
       for (int k = 6 * chi; k < 6 * chi + 6; k++) {
         const cx<T> v = stg[k * 64 + (n & 63)];
-        acc[k].r = fma(f, v.r, fma(d, fv[k].r, acc[k].r));
-        acc[k].i = fma(f, v.i, fma(d, fv[k].i, acc[k].i));
+        if constexpr (Sto<S>::H) {
+          fv[k] = band_sum<S>(d, fv[k], f, v, sn < s);
+        } else {
+          acc[k].r = fma(f, v.r, fma(d, fv[k].r, acc[k].r));
+          acc[k].i = fma(f, v.i, fma(d, fv[k].i, acc[k].i));
+        }
       }
     }
+    if constexpr (Sto<S>::H) add_rounded<12>(acc, fv, max_part<12>(fv));
     if (!NORM && !valid) return;
   }
   if (EPI != 0 && !BAND && valid) {
@@ -780,7 +852,7 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
       if (RUPD) {
         cx<T> rv[12];
         load_site<S>(rv, ep.rv, o);
-        const T a = (T)(-ep.acoef[ep.astride * s]);
+        const T a = (T)(-ra);
 #pragma unroll
         for (int k = 0; k < 12; k++) {
           rv[k] = {fma(a, acc[k].r, rv[k].r), fma(a, acc[k].i, rv[k].i)};
@@ -867,7 +939,7 @@ __device__ __forceinline__ void group_band(cx<typename Sto<S>::C> *acc, cx<typen
   load_site<S>(fv, ep.phi, o);
 #pragma unroll
   for (int chi = 0; chi < 2; chi++) {
-    const uint32_t n = row + slice_nbr(sg, chi, DAG, LB);
+    const uint32_t sn = slice_nbr(sg, chi, DAG, LB), n = row + sn;
     if constexpr (DAG) {
       __syncthreads();
 #pragma unroll
@@ -875,10 +947,7 @@ __device__ __forceinline__ void group_band(cx<typename Sto<S>::C> *acc, cx<typen
       __syncthreads();
       const T d = ep.alpha * ep.mat[2 * chi * LB + sg], f = ep.alpha * ep.mat[(2 * chi + 1) * LB + sg];
 #pragma unroll
-      for (int k = 0; k < 6; k++) {
-        const cx<T> v = stg[k * epb + n];
-        acc[6 * chi + k] = {fma(f, v.r, d * acc[6 * chi + k].r), fma(f, v.i, d * acc[6 * chi + k].i)};
-      }
+      for (int k = 0; k < 6; k++) acc[6 * chi + k] = band_sum<S>(d, acc[6 * chi + k], f, stg[k * epb + n], sn < sg);
     } else {
 #pragma unroll
       for (int k = 6 * chi; k < 6 * chi + 6; k++) acc[k] = {ep.alpha * acc[k].r, ep.alpha * acc[k].i};
@@ -891,10 +960,15 @@ __device__ __forceinline__ void group_band(cx<typename Sto<S>::C> *acc, cx<typen
 #pragma unroll
     for (int k = 0; k < 6; k++) {
       const cx<T> v = stg[k * epb + n];
-      acc[6 * chi + k].r = fma(f, v.r, fma(d, fv[6 * chi + k].r, acc[6 * chi + k].r));
-      acc[6 * chi + k].i = fma(f, v.i, fma(d, fv[6 * chi + k].i, acc[6 * chi + k].i));
+      if constexpr (Sto<S>::H) {
+        fv[6 * chi + k] = band_sum<S>(d, fv[6 * chi + k], f, v, sn < sg);
+      } else {
+        acc[6 * chi + k].r = fma(f, v.r, fma(d, fv[6 * chi + k].r, acc[6 * chi + k].r));
+        acc[6 * chi + k].i = fma(f, v.i, fma(d, fv[6 * chi + k].i, acc[6 * chi + k].i));
+      }
     }
   }
+  if constexpr (Sto<S>::H) add_rounded<12>(acc, fv, max_part<12>(fv));
 }
 
 // The hop of k_dhop (same legs, projectors, link staging and epilogues) in the general tile shape,
@@ -917,6 +991,8 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
   const uint32_t h = sweep ? sweep_site(g, pos) : pos;
   uint32_t nb[8];
   site_neighbours(g, h, cb_out, nb);
+  double ds = 0;
+  if (RUPD) ds = d_share(ep);
   // links of tile site hl: thread (hl, s) loads entries s, s + LS, ... (< 72)
   cx<T> ureg[kGenLinkPerThread];
 #pragma unroll
@@ -927,12 +1003,19 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
   cx<T> fa[12], fb[12];
   T sa = load_site_raw<S>(fa, in, leg_idx<DAG, 0, 0>(nb, LS, s));
   T sb = load_site_raw<S>(fb, in, leg_idx<DAG, 0, 1>(nb, LS, s));
+  __shared__ double dsh[RUPD ? kGenMaxWaves : 1];
+  if (RUPD && ep.cur) {
+    ds = wave_sum(ds);
+    if ((t & 63) == 0) dsh[t >> 6] = ds;
+  }
 #pragma unroll
   for (int j = 0; j < kGenLinkPerThread; j++) {
     const uint32_t pk = s + LS * j;
     if (pk < 72) lds[hl * kLinkPad + pk] = ureg[j];
   }
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  double ra = 0;
+  if (RUPD) ra = rupd_coef(ep, dsh, s, tile == 0 && t == 0);
   cx<T> acc[12];
 #pragma unroll
   for (int k = 0; k < 12; k++) acc[k] = {0, 0};
@@ -952,7 +1035,7 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
       // the residual update in place of storing the result (k_dhop's EPI 6 / 7)
       cx<T> rv[12];
       load_site<S>(rv, ep.rv, o);
-      const T a = (T)(-ep.acoef[ep.astride * s]);
+      const T a = (T)(-ra);
 #pragma unroll
       for (int k = 0; k < 12; k++) {
         rv[k] = {fma(a, acc[k].r, rv[k].r), fma(a, acc[k].i, rv[k].i)};
@@ -1023,11 +1106,6 @@ struct SplitArgs {
   int cb;
   uint32_t LS, SPW;
   FDiv fLS;
-  // RUPD in a single-RHS CG: a = c / d with c of the state cur and d the sum of nd partials, left in nxt
-  const CGState *cur;
-  CGState *nxt;
-  const double *dpart;
-  int nd;
 };
 
 // component k of entry e, without and with the FP16 site scale
@@ -1103,7 +1181,7 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
   constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7;
   if (gated(gate)) return;
   __shared__ cx<T> prod[8 * 6 * 64];
-  __shared__ T lsc[Sto<S>::H ? 8 * 64 : 1], smax[Sto<S>::H ? 3 * 64 : 1];
+  __shared__ T lsc[Sto<S>::H ? 8 * 64 : 1], smax[Sto<S>::H ? 3 * 64 : 1], bmax[Sto<S>::H && BAND ? 3 * 64 : 1];
   __shared__ double nsh[NORM ? 3 * 64 : 1], dsh[RUPD ? 8 : 1];
   const uint32_t lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t LS = A.LS, ls = fdiv(lane, A.fLS), s = lane - ls * LS;
@@ -1112,15 +1190,14 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
   const bool valid = ls < A.SPW && h0 + ls < H4;
   const uint32_t h = valid ? h0 + ls : h0, o = h * LS + s;  // idle lanes: in-bounds addresses
   double ds = 0;
-  if (RUPD && A.cur)
-    for (int i = threadIdx.x; i < A.nd; i += 512) ds += A.dpart[i];
+  if (RUPD) ds = d_share(ep);
   switch (w) {
 #define GX_SPLIT_LEG(L)   case L: split_leg<S, DAG, L>(A.in[j], A.U[j], g, cb, h, s, LS, lane, prod, lsc); break;
     GX_SPLIT_LEG(0) GX_SPLIT_LEG(1) GX_SPLIT_LEG(2) GX_SPLIT_LEG(3)
     GX_SPLIT_LEG(4) GX_SPLIT_LEG(5) GX_SPLIT_LEG(6) GX_SPLIT_LEG(7)
 #undef GX_SPLIT_LEG
   }
-  if (RUPD && A.cur) {
+  if (RUPD && ep.cur) {
     ds = wave_sum(ds);
     if (lane == 0) dsh[w] = ds;
   }
@@ -1180,8 +1257,13 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
     }
     if constexpr (BAND) {
       uint32_t n[2];
+      bool low[2];
 #pragma unroll
-      for (int chi = 0; chi < 2; chi++) n[chi] = (row + slice_nbr(s, chi, DAG, LS)) & 63;
+      for (int chi = 0; chi < 2; chi++) {
+        const uint32_t sn = slice_nbr(s, chi, DAG, LS);
+        n[chi] = (row + sn) & 63;
+        low[chi] = sn < s;
+      }
       if constexpr (DAG) {
         wave_sync();
 #pragma unroll
@@ -1191,8 +1273,7 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
         for (int sp = 0; sp < 4; sp++) {
           const int chi = sp / 2;
           const T d = ep.alpha * ep.mat[2 * chi * LS + s], f = ep.alpha * ep.mat[(2 * chi + 1) * LS + s];
-          const cx<T> v = stg(sp)[n[chi]];
-          a[3 * sp] = {fma(f, v.r, d * a[3 * sp].r), fma(f, v.i, d * a[3 * sp].i)};
+          a[3 * sp] = band_sum<S>(d, a[3 * sp], f, stg(sp)[n[chi]], low[chi]);
         }
       } else {
 #pragma unroll
@@ -1207,9 +1288,14 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
         const int chi = sp / 2;
         const T d = ep.coef[2 * chi * LS + s], f = ep.coef[(2 * chi + 1) * LS + s];
         const cx<T> v = stg(sp)[n[chi]];
-        a[3 * sp].r = fma(f, v.r, fma(d, fv[sp].r, a[3 * sp].r));
-        a[3 * sp].i = fma(f, v.i, fma(d, fv[sp].i, a[3 * sp].i));
+        if constexpr (Sto<S>::H) {
+          fv[sp] = band_sum<S>(d, fv[sp], f, v, low[chi]);
+        } else {
+          a[3 * sp].r = fma(f, v.r, fma(d, fv[sp].r, a[3 * sp].r));
+          a[3 * sp].i = fma(f, v.i, fma(d, fv[sp].i, a[3 * sp].i));
+        }
       }
+      if constexpr (Sto<S>::H) bmax[c * 64 + lane] = max_part<4>(fv);
     } else if constexpr (EPI != 0) {
       const T al = PHI ? ep.coef[s] : ep.alpha;
 #pragma unroll
@@ -1223,20 +1309,19 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
         }
       }
     }
+  }
+  if (Sto<S>::H && BAND) __syncthreads();
+  if (c < 3) {
+    if constexpr (Sto<S>::H && BAND) {
+      cx<float> b[4];
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) b[sp] = a[3 * sp];
+      add_rounded<4>(b, fv, fmaxf(bmax[lane], fmaxf(bmax[64 + lane], bmax[128 + lane])));
+#pragma unroll
+      for (int sp = 0; sp < 4; sp++) a[3 * sp] = b[sp];
+    }
     if constexpr (RUPD) {
-      double av;
-      if (A.cur) {
-        double d = 0;
-        for (int i = 0; i < 8; i++) d += dsh[i];
-        av = A.cur->c / d;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-          A.nxt->d = d;
-          A.nxt->a = av;
-        }
-      } else {
-        av = ep.acoef[ep.astride * s];
-      }
-      const T ra = (T)(-av);
+      const T ra = (T)(-rupd_coef(ep, dsh, s, blockIdx.x == 0 && threadIdx.x == 0));
 #pragma unroll
       for (int sp = 0; sp < 4; sp++) a[3 * sp] = {fma(ra, a[3 * sp].r, rv[sp].r), fma(ra, a[3 * sp].i, rv[sp].i)};
     }
@@ -1705,19 +1790,18 @@ int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], vo
   A.fLS = make_fdiv(A.LS);
   const uint32_t tiles = (uint32_t)((g.H4 + A.SPW - 1) / A.SPW);
   const bool norm = fz && fz->npart && fz->nparts && (epi == 1 || epi == 3) && (fz->r ? (dag && fz->a) : !dag);
-  HopEpi<S> ep{nullptr, (const T *)mat, (T)alpha, (const T *)coef, nullptr, nullptr, nullptr, 1, fz ? fz->total : 0};
+  HopEpi<S> ep{nullptr, (const T *)mat, (T)alpha, (const T *)coef, nullptr, nullptr, nullptr, 1, fz ? fz->total : 0,
+               nullptr, nullptr, nullptr, 0};
   if (fz && fz->nparts) *fz->nparts = 0;
   if (norm) {
     ep.npart = fz->npart;
     ep.rv = (cx<S> *)fz->r;
     ep.acoef = fz->a;
     ep.astride = fz->astride;
-    if (fz->r) {
-      A.cur = fz->cur;
-      A.nxt = fz->nxt;
-      A.dpart = fz->dpart;
-      A.nd = fz->nd;
-    }
+    ep.cur = fz->cur;
+    ep.nxt = fz->nxt;
+    ep.dpart = fz->dpart;
+    ep.nd = fz->nd;
     *fz->nparts = tiles;
   }
   const KGeom k = kgeom(g);
@@ -1802,7 +1886,8 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   const cx<S> *pU = (const cx<S> *)U;
   HopEpi<S> ep{(const cx<S> *)phi, (const T *)mat, (T)alpha, (const T *)coef,
                fz ? fz->npart : nullptr,  (cx<S> *)(fz ? fz->r : nullptr),  fz ? fz->a : nullptr,
-               fz ? fz->astride : 1,  fz ? fz->total : 0};
+               fz ? fz->astride : 1,  fz ? fz->total : 0,
+               fz ? fz->cur : nullptr, fz ? fz->nxt : nullptr, fz ? fz->dpart : nullptr, fz ? fz->nd : 0};
   if constexpr (std::is_same<S, float>::value) {
     // the link products on the matrix cores: FP32 multi-RHS (Wilson, no matrix epilogue), Ls <= 16
     if (tune_get(GX_TUNE_DHOP_MFMA, prec_of<S>()) && kepi <= 1 && g.Ls >= 2 && g.Ls <= 16 && lb == g.Ls) {
@@ -2125,11 +2210,13 @@ __global__ void __launch_bounds__(256) k_band(const cx<S> *__restrict__ in, cons
   cx<T> f[12], v[12];
   load_site<S>(f, in, e);
   T sc[2] = {(T)1, (T)1};
+  bool low[2];
 #pragma unroll
   for (int chi = 0; chi < 2; chi++) {
-    const uint32_t n = e - s + slice_nbr(s, chi, dag != 0, LS);
+    const uint32_t sn = slice_nbr(s, chi, dag != 0, LS), n = e - s + sn;
     const cx<S> *q = in + bidx<S>(n, 0);
     sc[chi] = site_scale<S>(in, n);
+    low[chi] = sn < s;
     // groups that hold components of this chirality: 6 chi .. 6 chi + 5 (FP16's middle group holds both)
 #pragma unroll
     for (int g = 6 * chi / VW; g <= (6 * chi + 5) / VW; g++) {
@@ -2143,8 +2230,10 @@ __global__ void __launch_bounds__(256) k_band(const cx<S> *__restrict__ in, cons
 #pragma unroll
   for (int k = 0; k < 12; k++) {
     const int chi = k / 6;
-    const T d = bands[2 * chi * LS + s], b = bands[(2 * chi + 1) * LS + s] * sc[chi];
-    f[k] = {fma(b, v[k].r, d * f[k].r), fma(b, v[k].i, d * f[k].i)};
+    const T d = bands[2 * chi * LS + s], b = bands[(2 * chi + 1) * LS + s];
+    cx<T> w = v[k];
+    if constexpr (Sto<S>::H) w = {mul_rounded(w.r, sc[chi]), mul_rounded(w.i, sc[chi])};
+    f[k] = band_sum<S>(d, f[k], b, w, low[chi]);
   }
   if (PHI) axpy_site<S>(f, (T)1, phi, e);
   store_site<S>(out, f, e, false);
@@ -2636,6 +2725,90 @@ __global__ void __launch_bounds__(256) k_cg_update_fin(int64_t nsites, int64_t s
     *nxt = st;
   }
   cg_update<S>(nsites, stride, psi, p, r, a, b, keep_p);
+}
+
+// k_cg_update_fin on whole sites that also writes q = A(p) of the new p, A the two-band operator that the next
+// Mpc starts with (Meooe5D): the pass that read p back for it goes.  256 / Ls sites per workgroup, one entry
+// per thread, the new p of a site's slices exchanged in LDS.  FP64 and FP32 (FP16's p is what its store rounds).
+template <typename S>
+__global__ void __launch_bounds__(256) k_cg_update_band(uint32_t H4, cx<S> *__restrict__ psi, cx<S> *__restrict__ p,
+                                                        const cx<S> *__restrict__ r, cx<S> *__restrict__ q,
+                                                        const S *__restrict__ bands, FDiv fLS, const CGState *cur,
+                                                        CGState *nxt, const double *partial, int np) {
+  const uint32_t LS = fLS.d, spb = 256 / LS, t = threadIdx.x, hl = fdiv(t, fLS), s = t - hl * LS;
+  const uint32_t h = blockIdx.x * spb + hl;
+  const bool on = hl < spb && h < H4, first = blockIdx.x == 0 && t == 0;
+  __shared__ cx<S> stg[12 * 256];
+  __shared__ double sh[4];
+  CGState st = *cur;
+  if (st.k > st.k_conv || st.k > st.kmax) {
+    if (first) {
+      st.k++;
+      *nxt = st;
+    }
+    return;
+  }
+  const uint32_t e = h * LS + s;
+  cx<S> pv[12], xv[12], rv[12];
+  double v = 0;
+  for (int b = t; b < np; b += 256) v += partial[b];
+  if (on) {
+    load_site<S>(pv, p, e);
+    load_site<S>(rv, r, e);
+    load_site<S>(xv, psi, e);
+  }
+  v = wave_sum(v);
+  if ((t & 63) == 0) sh[t >> 6] = v;
+  __syncthreads();
+  st.a = nxt->a;
+  st.d = nxt->d;
+  cg_advance(st, (sh[0] + sh[1]) + (sh[2] + sh[3]));
+  const S a = (S)st.a, b = (S)st.b;
+  const bool keep_p = st.ru == 1;  // the host forms the new p (and its q)
+  if (first) {
+    st.k++;
+    *nxt = st;
+  }
+  if (on) {
+#pragma unroll
+    for (int k = 0; k < 12; k++) {
+      xv[k] = {fma(a, pv[k].r, xv[k].r), fma(a, pv[k].i, xv[k].i)};
+      pv[k] = {fma(b, pv[k].r, rv[k].r), fma(b, pv[k].i, rv[k].i)};
+      stg[k * 256 + t] = pv[k];
+    }
+    store_site<S>(psi, xv, e, false);
+  }
+  if (keep_p) return;  // uniform
+  if (on) store_site<S>(p, pv, e, false);
+  __syncthreads();
+  if (!on) return;
+#pragma unroll
+  for (int chi = 0; chi < 2; chi++) {
+    const uint32_t n = hl * LS + slice_nbr(s, chi, false, LS);
+    const S d = bands[2 * chi * LS + s], f = bands[(2 * chi + 1) * LS + s];
+#pragma unroll
+    for (int k = 6 * chi; k < 6 * chi + 6; k++) {
+      const cx<S> w = stg[k * 256 + n];
+      pv[k] = {fma(f, w.r, d * pv[k].r), fma(f, w.i, d * pv[k].i)};
+    }
+  }
+  store_site<S>(q, pv, e, false);
+}
+
+template <typename S>
+int launch_cg_update_band(Ctx *ctx, const Geom &g, void *psi, void *p, const void *r, void *q, const void *bands,
+                          const CGState *cur, CGState *nxt, const double *partial, int np) {
+  if constexpr (Sto<S>::H) {
+    set_error("CG update with the band: FP64 or FP32");
+    return GX_EINVAL;
+  } else {
+    const int spb = 256 / g.Ls;
+    hipLaunchKernelGGL((k_cg_update_band<S>), dim3((uint32_t)((g.H4 + spb - 1) / spb)), dim3(256), 0, ctx->stream,
+                       (uint32_t)g.H4, (cx<S> *)psi, (cx<S> *)p, (const cx<S> *)r, (cx<S> *)q, (const S *)bands,
+                       make_fdiv((uint32_t)g.Ls), cur, nxt, partial, np);
+    GX_CHECK_HIP(hipGetLastError());
+    return GX_OK;
+  }
 }
 
 template <typename S>
@@ -3906,6 +4079,8 @@ int launch_digest_slices(Ctx *ctx, const Geom &g, const void *full, int s0, int 
   template int launch_reduce<S>(Ctx *, int, int64_t, int64_t, const void *, const void *, void *, double, int);   \
   template int launch_cg_dot<S>(Ctx *, int64_t, int64_t, const void *, const void *, CGState *);                   \
   template int launch_cg_axpy_norm<S>(Ctx *, int64_t, int64_t, void *, const void *, CGState *);                   \
+  template int launch_cg_update_band<S>(Ctx *, const Geom &, void *, void *, const void *, void *, const void *,   \
+                                        const CGState *, CGState *, const double *, int);                          \
   template int launch_cg_update_fin<S>(Ctx *, int64_t, int64_t, void *, void *, const void *, const CGState *,     \
                                        CGState *, const double *, int);                                            \
   template int launch_cg_update<S>(Ctx *, int64_t, int64_t, void *, void *, const void *, CGState *);

@@ -66,7 +66,7 @@ static int run_batch(Ctx *ctx, BatchGraph &g, const void *const key[8], int batc
 }
 
 struct CGWork {
-  CGState *dev = nullptr;   // 2: the state, and its successor (cg_iteration_small)
+  CGState *dev = nullptr;   // 2: the state, and its successor (cg_iteration_fold)
   CGState *host = nullptr;  // pinned, 2 slots
   hipEvent_t ev[2] = {};
   BatchGraph graph[3];  // per precision
@@ -195,12 +195,17 @@ static int cg_iteration(Op *op, Field *psi, Field *p, Field *mmp, Field *r, CGSt
   return GX_OK;
 }
 
-// The same iteration on small lattices (hop_split), where launches are what it costs: the finalisers run
-// inside the kernels that need their results, every workgroup adding the few hundred tile sums for itself in the
-// same order.  The state alternates between cur and nxt, so no kernel writes what another workgroup of it
-// reads.  Wilson: 5 launches instead of 9 (a red-black solve on 8^4 in FP64 2.40 -> 1.50 ms).
+// The same iteration where a reduction leaves at most kFoldTiles tile sums: the finalisers run inside the
+// kernels that need their results, every workgroup adding the tile sums for itself in the same order.  The state
+// alternates between cur and nxt, so no kernel writes what another workgroup of it reads.  q (Cayley in FP64 and
+// FP32, else null) holds Meooe5D p, which the update leaves for the next iteration.  Launches: Wilson 5 instead of
+// 9, Cayley 5 instead of 8.  A red-black solve on 8^4 in FP64 2.40 -> 1.50 ms; Mobius 16^4 x 16 with FP32 inner
+// solves 169.6 -> 167.6 ms (two finalisers of 4.5 us and a pass of 15 us less, of which the last hop's own sum and
+// the update's extra store take 16 back: what bounds those kernels is the fields' traffic).
+constexpr int64_t kFoldTiles = 4096;
 template <typename T>
-static int cg_iteration_small(Op *op, Field *psi, Field *p, Field *mmp, Field *r, CGState *cur, CGState *nxt) {
+static int cg_iteration_fold(Op *op, Field *psi, Field *p, Field *mmp, Field *r, CGState *cur, CGState *nxt,
+                             Field *q) {
   Ctx *ctx = op->ctx;
   const int64_t nsites = p->g.half_pad();
   double *dpart = ctx->red_partial, *rpart = dpart + kRedBlocks * kMaxRhs / 2;
@@ -211,7 +216,7 @@ static int cg_iteration_small(Op *op, Field *psi, Field *p, Field *mmp, Field *r
   f1.npart = dpart;
   f1.nparts = &n1;
   f1.total = 1;
-  GX_TRY(apply_mpc(op, p, t, 0, cur, &f1));
+  GX_TRY(apply_mpc(op, p, t, 0, cur, &f1, q ? q->data : nullptr));
   HopFuse f2 = f1;
   f2.npart = rpart;
   f2.nparts = &n2;
@@ -224,10 +229,28 @@ static int cg_iteration_small(Op *op, Field *psi, Field *p, Field *mmp, Field *r
   f2.nd = (int)n1;
   GX_TRY(apply_mpc(op, t, mmp, 1, cur, &f2));
   if (n1 < 1 || n2 < 1) {
-    set_error("CG: the small-lattice hop left no tile sums");
+    set_error("CG: the hop left no tile sums");
     return GX_EINVAL;
   }
+  if (q) {
+    const void *b;
+    GX_TRY(op_band(op, p->prec, Op::S_MEOOE5D, &b));
+    return launch_cg_update_band<T>(ctx, p->g, psi->data, p->data, r->data, q->data, b, cur, nxt, rpart, (int)n2);
+  }
   return launch_cg_update_fin<T>(ctx, nsites, nsites, psi->data, p->data, r->data, cur, nxt, rpart, (int)n2);
+}
+
+// whether the hop of this operator and precision leaves at most kFoldTiles tile sums (it does so in every
+// launch form but the persistent, row-tile and matrix-core ones)
+static bool cg_folds(const Op *op, int prec) {
+  if (!tune_get(GX_TUNE_FUSED, prec)) return false;
+  if (by_prec(prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g); })) return true;
+  const int Ls = op->g.Ls;
+  if (Ls > kMaxLs || tune_get(GX_TUNE_DHOP_SHAPE, prec) || tune_get(GX_TUNE_DHOP_MFMA, prec) ||
+      tune_get(GX_TUNE_DHOP_TILE, prec))
+    return false;
+  const int64_t spb = 4 * (64 / Ls);
+  return (op->g.H4 + spb - 1) / spb <= kFoldTiles;
 }
 
 // Device-resident CG iterations on (psi, p, mmp, r) of precision prec, from the state in w.dev,
@@ -243,18 +266,26 @@ static int cg_device_loop(Op *op, int prec, Field *psi, Field *p, Field *mmp, Fi
   const bool use_graph = tune_get(GX_TUNE_CG_GRAPH, prec) != 0;
   for (int i = 0; i < 4; i++)
     if (!op_tmp(op, prec, i)) return GX_ENOMEM;  // no allocation inside a capture
-  const bool small = tune_get(GX_TUNE_FUSED, prec) &&
-                     by_prec(prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g); }) != 0;
+  const bool fold = cg_folds(op, prec);
+  Field *q = nullptr;
+  if (fold && op->kind == GX_MOBIUS && prec != GX_F16 && op->g.Ls <= 256) {
+    q = op_tmp(op, prec, 0);
+    const void *b;
+    GX_TRY(op_band(op, prec, Op::S_MEOOE5D, &b));
+    GX_TRY(by_prec(prec, [&](auto t) {
+      return launch_band<decltype(t)>(op->g, p->data, nullptr, q->data, b, 0, nullptr, ctx->stream);
+    }));
+  }
   // tile sums: the operator's own buffer, or with Ls = 1 the context's reduction buffer where it holds them
   double *npart = w.npart;
   if (!npart && op->g.Ls == 1 && hop_norm_tiles(op->g.H4, 1) <= kRedBlocks * kMaxRhs) npart = ctx->red_partial;
-  int par = 0;  // which of the two states the next iteration reads (small)
+  int par = 0;  // which of the two states the next iteration reads (fold)
   auto iterate = [&]() -> int {
     return by_prec(prec, [&](auto t) -> int {
-      if (!small) return cg_iteration<decltype(t)>(op, psi, p, mmp, r, w.dev, npart);
+      if (!fold) return cg_iteration<decltype(t)>(op, psi, p, mmp, r, w.dev, npart);
       CGState *cur = w.dev + par, *nxt = w.dev + (par ^ 1);
       par ^= 1;
-      return cg_iteration_small<decltype(t)>(op, psi, p, mmp, r, cur, nxt);
+      return cg_iteration_fold<decltype(t)>(op, psi, p, mmp, r, cur, nxt, q);
     });
   };
   auto one_batch = [&]() -> int {  // an even number of iterations: the state is back where it was
