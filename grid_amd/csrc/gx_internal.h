@@ -257,6 +257,9 @@ struct HopFuse {
   CGState *nxt = nullptr;
   const double *dpart = nullptr;
   int nd = 0;
+  // FP64, r given: r_s -= a (the result + shift sp)_s
+  const void *sp = nullptr;
+  double shift = 0;
 };
 // Small lattices (hop_split) run the hop with one leg per wave, which launch_dhop_epi then does by
 // itself; ncb = 2 does both checkerboards cb and cb ^ 1 in one launch (operand j of each list).
@@ -366,7 +369,7 @@ int launch_multishift(Ctx *ctx, int64_t n, const void *r, void *p, const MultiSh
 // z (current zc, previous zp), bs and stopping norm rsq; active: shifts still iterating (bit s),
 // closing: the shifts whose psi the next update closes.  k, k_conv gate the kernels as in CGState.
 struct MsState : Gate {
-  double c, cp, a, b, bp, d, m0;
+  double c, cp, a, b, bp, d, m0, mb;   // mb: -b
   double zc[kMaxShift], zp[kMaxShift], bs[kMaxShift], dm[kMaxShift], rsq[kMaxShift];
   uint32_t active, closing;
   int nshift, pad;
@@ -383,7 +386,12 @@ struct MsPtrs {
 // 1 -> after mmp += m0 p
 int launch_ms_dot(Ctx *ctx, int64_t nsites, int64_t stride, const void *p, const void *mmp, MsState *st);
 int launch_ms_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, void *r, const void *mmp, MsState *st);
-int launch_ms_update(Ctx *ctx, int64_t n, const void *r, void *p, const MsPtrs &m, MsState *st);
+// pp: ms_update_blocks(n) partials of the new |p|^2
+constexpr int kMsBlocks = 4096;
+int ms_update_blocks(int64_t n);
+int launch_ms_update(Ctx *ctx, int64_t n, const void *r, void *p, const MsPtrs &m, MsState *st, double *pp);
+// the finalisers on tile sums of the hop: with pp, n partials of Re<p|A p> and np of |p|^2; without, n of |r|^2
+int launch_ms_fold(Ctx *ctx, const double *partial, int64_t n, const double *pp, int np, MsState *st);
 // Sums over the lattice of the six plaquettes' and four links' real traces of a device gauge field
 // ([site][mu][3][3] complex double): out_host[0] (plaquettes), out_host[1] (links); out_host holds
 // 2 nparts doubles.  Synchronises the stream.

@@ -13,6 +13,7 @@
 //   reductions: per-site products in the field precision, sums in double
 //   (Grid/lattice/Lattice_reduction.h:255-287), in a fixed order.
 #include <cfloat>
+#include <algorithm>
 #include <climits>
 #include <cstring>
 #include <type_traits>
@@ -576,7 +577,8 @@ struct HopEpi {
   const T *coef;  // EPI 1, 5, 6: alpha_s; EPI 3, 7, 8: B's bands [2][2][LS]
   // k_dhop and hop_tile.  EPI 5 (EPI 1 result) and 8 (EPI 3 result): out, and the per-tile slice sums of
   // |out|^2 in npart [tile][LS]; EPI 6 (EPI 1 result) and 7 (EPI 3 result): rv_s -= acoef[astride s]
-  // (result)_s in place of storing out, per-tile slice sums of |rv_s|^2
+  // (result)_s in place of storing out, per-tile slice sums of |rv_s|^2; EPI 10 and 9 (FP64): the same with
+  // result + shift sp in place of result
   double *npart;
   cx<S> *rv;
   const double *acoef;
@@ -588,6 +590,8 @@ struct HopEpi {
   CGState *nxt;
   const double *dpart;
   int nd;
+  const cx<S> *sp;
+  T shift;
 };
 
 // this thread's share of the partials of d, and its wave's sum in dsh (one per wave)
@@ -695,8 +699,9 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   constexpr int SPB = 4 * SPW;
   constexpr bool LDSU = (LS > 1) && (SPB * kLinkPad * sizeof(cx<T>) <= 40960);
   constexpr int NLINK = LDSU ? SPB * kLinkPad : 1;
-  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || EPI == 7 || EPI == 8, PHI = EPI == 1 || EPI == 5 || EPI == 6;
-  constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7;
+  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || (EPI >= 7 && EPI <= 9);
+  constexpr bool PHI = EPI == 1 || EPI == 5 || EPI == 6 || EPI == 10;
+  constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7 || EPI >= 9;
   constexpr int NSTAGE = MAT || BAND ? 4 * 12 * 64 : 1;
   __shared__ cx<T> lds[NLINK > NSTAGE ? NLINK : NSTAGE];  // links, then (MAT) the hop results
   const bool sweep = map == 4;  // blocked sweep: tiles are runs of the sweep order, XCD slabs
@@ -853,6 +858,7 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
         cx<T> rv[12];
         load_site<S>(rv, ep.rv, o);
         const T a = (T)(-ra);
+        if (EPI >= 9) axpy_site<S>(acc, ep.shift, ep.sp, o);
 #pragma unroll
         for (int k = 0; k < 12; k++) {
           rv[k] = {fma(a, acc[k].r, rv[k].r), fma(a, acc[k].i, rv[k].i)};
@@ -979,8 +985,9 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
                                          bool sweep, int flags, const HopEpi<S> &ep, const GShape &sh,
                                          cx<typename Sto<S>::C> *lds) {
   typedef typename Sto<S>::C T;
-  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || EPI == 7 || EPI == 8, PHI = EPI == 1 || EPI == 5 || EPI == 6;
-  constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7;
+  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || (EPI >= 7 && EPI <= 9);
+  constexpr bool PHI = EPI == 1 || EPI == 5 || EPI == 6 || EPI == 10;
+  constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7 || EPI >= 9;
   const uint32_t H4 = (uint32_t)g.H4, LS = sh.LS, epb = blockDim.x;
   const uint32_t t = threadIdx.x;
   const uint32_t hl = fdiv(t, sh.fLS), s = t - hl * LS;
@@ -1036,6 +1043,7 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
       cx<T> rv[12];
       load_site<S>(rv, ep.rv, o);
       const T a = (T)(-ra);
+      if (EPI >= 9) axpy_site<S>(acc, ep.shift, ep.sp, o);
 #pragma unroll
       for (int k = 0; k < 12; k++) {
         rv[k] = {fma(a, acc[k].r, rv[k].r), fma(a, acc[k].i, rv[k].i)};
@@ -1177,8 +1185,9 @@ __device__ __forceinline__ void split_recon(cx<typename Sto<S>::C> *a, const cx<
 template <typename S, bool DAG, int EPI>
 __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, const Gate *__restrict__ gate, HopEpi<S> ep) {
   typedef typename Sto<S>::C T;
-  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || EPI == 7 || EPI == 8, PHI = EPI == 1 || EPI == 5 || EPI == 6;
-  constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7;
+  constexpr bool MAT = EPI == 2, BAND = EPI == 3 || (EPI >= 7 && EPI <= 9);
+  constexpr bool PHI = EPI == 1 || EPI == 5 || EPI == 6 || EPI == 10;
+  constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7 || EPI >= 9;
   if (gated(gate)) return;
   __shared__ cx<T> prod[8 * 6 * 64];
   __shared__ T lsc[Sto<S>::H ? 8 * 64 : 1], smax[Sto<S>::H ? 3 * 64 : 1], bmax[Sto<S>::H && BAND ? 3 * 64 : 1];
@@ -1322,6 +1331,12 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
     }
     if constexpr (RUPD) {
       const T ra = (T)(-rupd_coef(ep, dsh, s, blockIdx.x == 0 && threadIdx.x == 0));
+      if (EPI >= 9)
+#pragma unroll
+        for (int sp = 0; sp < 4; sp++) {
+          const cx<T> v = load_comp<S>(ep.sp, o, 3 * sp + c);
+          a[3 * sp] = {fma(ep.shift, v.r, a[3 * sp].r), fma(ep.shift, v.i, a[3 * sp].i)};
+        }
 #pragma unroll
       for (int sp = 0; sp < 4; sp++) a[3 * sp] = {fma(ra, a[3 * sp].r, rv[sp].r), fma(ra, a[3 * sp].i, rv[sp].i)};
     }
@@ -1791,7 +1806,7 @@ int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], vo
   const uint32_t tiles = (uint32_t)((g.H4 + A.SPW - 1) / A.SPW);
   const bool norm = fz && fz->npart && fz->nparts && (epi == 1 || epi == 3) && (fz->r ? (dag && fz->a) : !dag);
   HopEpi<S> ep{nullptr, (const T *)mat, (T)alpha, (const T *)coef, nullptr, nullptr, nullptr, 1, fz ? fz->total : 0,
-               nullptr, nullptr, nullptr, 0};
+               nullptr, nullptr, nullptr, 0, nullptr, (T)0};
   if (fz && fz->nparts) *fz->nparts = 0;
   if (norm) {
     ep.npart = fz->npart;
@@ -1802,6 +1817,8 @@ int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], vo
     ep.nxt = fz->nxt;
     ep.dpart = fz->dpart;
     ep.nd = fz->nd;
+    ep.sp = (const cx<S> *)fz->sp;
+    ep.shift = (T)fz->shift;
     *fz->nparts = tiles;
   }
   const KGeom k = kgeom(g);
@@ -1813,7 +1830,15 @@ int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], vo
     if (!dag && epi == 3) GX_SPLIT_GO(false, 8);
     else if (!dag) GX_SPLIT_GO(false, 5);
     else if (!fz->r) return GX_EINVAL;
-    else if (epi == 3) GX_SPLIT_GO(true, 7);
+    else if (fz->sp) {
+      if constexpr (std::is_same<S, double>::value) {
+        if (epi == 3) GX_SPLIT_GO(true, 9);
+        else GX_SPLIT_GO(true, 10);
+      } else {
+        set_error("dhop: the shifted update is FP64");
+        return GX_EINVAL;
+      }
+    } else if (epi == 3) GX_SPLIT_GO(true, 7);
     else GX_SPLIT_GO(true, 6);
   } else {
     switch (epi) {
@@ -1887,7 +1912,14 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   HopEpi<S> ep{(const cx<S> *)phi, (const T *)mat, (T)alpha, (const T *)coef,
                fz ? fz->npart : nullptr,  (cx<S> *)(fz ? fz->r : nullptr),  fz ? fz->a : nullptr,
                fz ? fz->astride : 1,  fz ? fz->total : 0,
-               fz ? fz->cur : nullptr, fz ? fz->nxt : nullptr, fz ? fz->dpart : nullptr, fz ? fz->nd : 0};
+               fz ? fz->cur : nullptr, fz ? fz->nxt : nullptr, fz ? fz->dpart : nullptr, fz ? fz->nd : 0,
+               (const cx<S> *)(fz ? fz->sp : nullptr), (T)(fz ? fz->shift : 0.0)};
+  // the shifted update exists in FP64
+  constexpr bool kShift = std::is_same<S, double>::value;
+  if (fz && fz->sp && !kShift) {
+    set_error("dhop: the shifted update is FP64");
+    return GX_EINVAL;
+  }
   if constexpr (std::is_same<S, float>::value) {
     // the link products on the matrix cores: FP32 multi-RHS (Wilson, no matrix epilogue), Ls <= 16
     if (tune_get(GX_TUNE_DHOP_MFMA, prec_of<S>()) && kepi <= 1 && g.Ls >= 2 && g.Ls <= 16 && lb == g.Ls) {
@@ -2017,8 +2049,12 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
       *fz->nparts = ntiles;
       if (!dag && kepi == 3) GX_DHOPG_GO(false, 8);
       else if (!dag) GX_DHOPG_GO(false, 5);
-      else if (kepi == 3) GX_DHOPG_GO(true, 7);
-      else GX_DHOPG_GO(true, 6);
+      else if (kepi == 3 && !fz->sp) GX_DHOPG_GO(true, 7);
+      else if (!fz->sp) GX_DHOPG_GO(true, 6);
+      else if constexpr (kShift) {
+        if (kepi == 3) GX_DHOPG_GO(true, 9);
+        else GX_DHOPG_GO(true, 10);
+      }
     } else {
       switch (kepi) {
         case 0: GX_DHOPG_EPI(0); break;
@@ -2054,7 +2090,12 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   case LS:                                                       \
     if (norm && kepi == 3) {                                     \
       if constexpr (LS >= 2) {                                   \
-        if (dag) {                                               \
+        if (dag && fz->sp) {                                     \
+          if constexpr (kShift) {                                \
+            if (pf) GX_DHOP_GO(LS, true, true, 0, 9);            \
+            else GX_DHOP_GO(LS, true, false, 0, 9);              \
+          }                                                      \
+        } else if (dag) {                                        \
           if (pf) GX_DHOP_GO(LS, true, true, 0, 7);              \
           else GX_DHOP_GO(LS, true, false, 0, 7);                \
         } else {                                                 \
@@ -2063,7 +2104,12 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
         }                                                        \
       }                                                          \
     } else if (norm) {                                           \
-      if (dag) {                                                 \
+      if (dag && fz->sp) {                                       \
+        if constexpr (kShift) {                                  \
+          if (pf) GX_DHOP_GO(LS, true, true, 0, 10);             \
+          else GX_DHOP_GO(LS, true, false, 0, 10);               \
+        }                                                        \
+      } else if (dag) {                                          \
         if (pf) GX_DHOP_GO(LS, true, true, 0, 6);                \
         else GX_DHOP_GO(LS, true, false, 0, 6);                  \
       } else {                                                   \
@@ -3451,6 +3497,21 @@ static __global__ void __launch_bounds__(256) k_multishift(int64_t n, const cx<d
 }
 
 // ---------------- device-resident multishift recurrences ----------------
+// sums over a workgroup of 1024 threads, in a fixed order
+template <int NV>
+__device__ __forceinline__ void block_sum16(double (&v)[NV], double (*sh)[16]) {
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    v[j] = wave_sum(v[j]);
+    if ((threadIdx.x & 63) == 0) sh[j][threadIdx.x >> 6] = v[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    v[j] = 0;
+    for (int i = 0; i < 16; i++) v[j] += sh[j][i];
+  }
+}
 // Re<p|A p> and |p|^2 (A p before the m0 shift), block partials
 static __global__ void __launch_bounds__(256) k_ms_dot(int64_t nsites, int64_t stride, const cx<double> *__restrict__ p,
                                                        const cx<double> *__restrict__ mmp, const MsState *st,
@@ -3480,12 +3541,20 @@ static __global__ void __launch_bounds__(256) k_ms_dot(int64_t nsites, int64_t s
 
 // d = Re<p|A p> + m0 |p|^2, b = -cp / d, and the shifts' z and bs (ConjugateGradientMultiShift.h
 // :238-262), with the a of the previous iteration
-static __global__ void __launch_bounds__(256) k_ms_fin_d(const double *partial, int nparts, MsState *st) {
+// (pp: the partials are Re<p|A p> alone, np of |p|^2 at pp; null: pairs of both)
+static __global__ void __launch_bounds__(1024) k_ms_fin_d(const double *partial, int nparts, const double *pp, int np,
+                                                          MsState *st) {
   if (gated(st)) return;
-  __shared__ double sh[2][4];
+  __shared__ double sh[2][16];
   __shared__ double nb[2];  // the new b and the previous one
-  double v[2];
-  sum_partials<2>(v, partial, nparts, sh);
+  double v[2] = {0, 0};
+  const int step = pp ? 1 : 2;
+  for (int i = threadIdx.x; i < nparts; i += 1024) v[0] += partial[(int64_t)step * i];
+  if (pp)
+    for (int i = threadIdx.x; i < np; i += 1024) v[1] += pp[i];
+  else
+    for (int i = threadIdx.x; i < nparts; i += 1024) v[1] += partial[2 * i + 1];
+  block_sum16<2>(v, sh);
   if (threadIdx.x == 0) {
     const double d = v[0] + st->m0 * v[1], cp = st->c, bp = st->b, b = -cp / d;
     st->d = d;
@@ -3493,6 +3562,7 @@ static __global__ void __launch_bounds__(256) k_ms_fin_d(const double *partial, 
     st->bp = bp;
     st->b = b;
     st->bs[0] = b;
+    st->mb = -b;
     nb[0] = b;
     nb[1] = bp;
   }
@@ -3537,11 +3607,14 @@ static __global__ void __launch_bounds__(256) k_ms_axpy_norm(int64_t nsites, int
 
 // c = |r|^2; each active shift's stopping test c z_s^2 < rsq_s; a = c / cp; k += 1 (also once
 // stopped, so the gate of the update that closes the last iteration opens exactly once)
-static __global__ void __launch_bounds__(256) k_ms_fin_c(const double *partial, int nparts, MsState *st) {
+static __global__ void __launch_bounds__(1024) k_ms_fin_c(const double *partial, int nparts, MsState *st) {
   const bool skip = gated(st);
-  __shared__ double sh[1][4];
+  __shared__ double sh[1][16];
   double v[1] = {0};
-  if (!skip) sum_partials<1>(v, partial, nparts, sh);
+  if (!skip) {
+    for (int i = threadIdx.x; i < nparts; i += 1024) v[0] += partial[i];
+    block_sum16<1>(v, sh);
+  }
   if (threadIdx.x == 0) {
     if (!skip) {
       const double c = v[0];
@@ -3562,9 +3635,11 @@ static __global__ void __launch_bounds__(256) k_ms_fin_c(const double *partial, 
 }
 
 // k_multishift with the coefficients of the state (psi_s -= bs_s ps_s for the closing shifts;
-// p = a p + r and ps_s = z_s r + as_s ps_s for the active ones), gated on the iteration it closes
+// p = a p + r and ps_s = z_s r + as_s ps_s for the active ones), gated on the iteration it closes; |p|^2 in
+// one partial per workgroup
 static __global__ void __launch_bounds__(256) k_ms_update(int64_t n, const cx<double> *__restrict__ r,
-                                                          cx<double> *__restrict__ p, MsPtrs m, const MsState *st) {
+                                                          cx<double> *__restrict__ p, MsPtrs m, const MsState *st,
+                                                          double *pp) {
   if (st->k - 1 > st->k_conv || st->k - 1 > st->kmax) return;
   __shared__ double cbs[kMaxShift], cz[kMaxShift], cas[kMaxShift];
   const int ns = st->nshift;
@@ -3578,11 +3653,14 @@ static __global__ void __launch_bounds__(256) k_ms_update(int64_t n, const cx<do
   }
   __syncthreads();
   const bool do_p = active != 0;
+  double v[1] = {0};
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const cx<double> rv = r[i];
     if (do_p) {
-      const cx<double> pv = p[i];
-      p[i] = {fma(a, pv.r, rv.r), fma(a, pv.i, rv.i)};
+      cx<double> pv = p[i];
+      pv = {fma(a, pv.r, rv.r), fma(a, pv.i, rv.i)};
+      p[i] = pv;
+      v[0] = fma(pv.r, pv.r, fma(pv.i, pv.i, v[0]));
     }
     for (int s = 0; s < ns; s++) {
       const bool dpsi = (closing >> s) & 1u, dps = (active >> s) & 1u;
@@ -3600,6 +3678,9 @@ static __global__ void __launch_bounds__(256) k_ms_update(int64_t n, const cx<do
       }
     }
   }
+  __shared__ double sh[1][4];
+  block_sum<1>(v, sh);
+  write_partial<1>(v, pp);
 }
 
 // ---------------- slice matrices (Lattice_reduction.h:717-776) ----------------
@@ -3982,7 +4063,19 @@ int launch_ms_dot(Ctx *ctx, int64_t nsites, int64_t stride, const void *p, const
   const int nb = red_blocks(nsites);
   hipLaunchKernelGGL(k_ms_dot, dim3(nb), dim3(256), 0, ctx->stream, nsites, stride, (const cx<double> *)p,
                      (const cx<double> *)mmp, (const MsState *)st, ctx->red_partial);
-  hipLaunchKernelGGL(k_ms_fin_d, dim3(1), dim3(256), 0, ctx->stream, (const double *)ctx->red_partial, nb, st);
+  hipLaunchKernelGGL(k_ms_fin_d, dim3(1), dim3(1024), 0, ctx->stream, (const double *)ctx->red_partial, nb,
+                     (const double *)nullptr, 0, st);
+  GX_CHECK_HIP(hipGetLastError());
+  return GX_OK;
+}
+
+int launch_ms_fold(Ctx *ctx, const double *partial, int64_t n, const double *pp, int np, MsState *st) {
+  if (n < 1 || n > INT_MAX) {
+    set_error("multishift fold: %lld tiles", (long long)n);
+    return GX_EINVAL;
+  }
+  if (pp) hipLaunchKernelGGL(k_ms_fin_d, dim3(1), dim3(1024), 0, ctx->stream, partial, (int)n, pp, np, st);
+  else hipLaunchKernelGGL(k_ms_fin_c, dim3(1), dim3(1024), 0, ctx->stream, partial, (int)n, st);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
@@ -3991,14 +4084,16 @@ int launch_ms_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, void *r, const
   const int nb = red_blocks(nsites);
   hipLaunchKernelGGL(k_ms_axpy_norm, dim3(nb), dim3(256), 0, ctx->stream, nsites, stride, (cx<double> *)r,
                      (const cx<double> *)mmp, (const MsState *)st, ctx->red_partial);
-  hipLaunchKernelGGL(k_ms_fin_c, dim3(1), dim3(256), 0, ctx->stream, (const double *)ctx->red_partial, nb, st);
+  hipLaunchKernelGGL(k_ms_fin_c, dim3(1), dim3(1024), 0, ctx->stream, (const double *)ctx->red_partial, nb, st);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
 
-int launch_ms_update(Ctx *ctx, int64_t n, const void *r, void *p, const MsPtrs &m, MsState *st) {
-  hipLaunchKernelGGL(k_ms_update, dim3(stream_blocks(n)), dim3(256), 0, ctx->stream, n, (const cx<double> *)r,
-                     (cx<double> *)p, m, (const MsState *)st);
+int ms_update_blocks(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, kMsBlocks); }
+
+int launch_ms_update(Ctx *ctx, int64_t n, const void *r, void *p, const MsPtrs &m, MsState *st, double *pp) {
+  hipLaunchKernelGGL(k_ms_update, dim3(ms_update_blocks(n)), dim3(256), 0, ctx->stream, n, (const cx<double> *)r,
+                     (cx<double> *)p, m, (const MsState *)st, pp);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }

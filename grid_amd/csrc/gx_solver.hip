@@ -1543,13 +1543,50 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
   const int64_t vol = op->g.half_elems();
   const int batch = vol >= (1 << 20) ? 8 : (vol >= (1 << 16) ? 16 : 32);
   int enqueued = 0, slot = 0;
+  // tile sums: the operator's buffer, or with Ls = 1 the front of the context's reduction buffer; the partials
+  // of |p|^2 behind it.  Before the first update |p|^2 is a reduction of its own.
+  Field *t = op_tmp(op, GX_F64, 2);
+  if (!t) return GX_ENOMEM;
+  double *pp = ctx->red_partial + kRedBlocks * kMaxRhs - kMsBlocks, *npart = sw->cg.npart;
+  if (!npart && op->g.Ls == 1 && hop_norm_tiles(op->g.H4, 1) <= kRedBlocks * kMaxRhs - kMsBlocks)
+    npart = ctx->red_partial;
+  constexpr int kMsNorm = 4;  // result slot
+  int npp = 0;
+  GX_TRY(launch_reduce<double>(ctx, 1, nsites, nsites, p->data, nullptr, nullptr, 0, kMsNorm));
   auto enqueue = [&](int sl) -> int {
     for (int i = 0; i < batch && enqueued < maxit; i++, enqueued++) {
-      GX_TRY(apply_mpcdagmpc(op, p, mmp, w.dev));
-      GX_TRY(launch_ms_dot(ctx, nsites, nsites, p->data, mmp->data, w.dev));
-      GX_TRY(blas_axpby(mmp, mass[0], p, 1.0, mmp, w.dev));
-      GX_TRY(launch_ms_axpy_norm(ctx, nsites, nsites, r->data, mmp->data, w.dev));
-      GX_TRY(launch_ms_update(ctx, nst, r->data, p->data, ptrs, w.dev));
+      // Where the tuned hop has the fused epilogues: Re<p|A p> = |t|^2 (t = Mpc p) from its tile sums, |p|^2 from
+      // the update before, and the last hop takes r += b (A p + m0 p) with |r|^2: six field passes less.
+      // (12^3x24 x 8, FP64, per iteration: dot 12, axpby 14, axpy_norm 18 us saved for 7 us more in the hops)
+      int64_t n1 = 0, n2 = 0;
+      HopFuse f1;
+      f1.npart = npart;
+      f1.nparts = &n1;
+      f1.total = 1;
+      GX_TRY(apply_mpc(op, p, t, 0, w.dev, npart ? &f1 : nullptr));
+      if (n1 > 0) {
+        GX_TRY(launch_ms_fold(ctx, npart, n1, npp ? pp : ctx->red_result + kMsNorm, npp ? npp : 1, w.dev));
+        HopFuse f2 = f1;
+        f2.nparts = &n2;
+        f2.r = r->data;
+        f2.a = &w.dev->mb;  // device address (not dereferenced here)
+        f2.astride = 0;
+        f2.sp = p->data;
+        f2.shift = mass[0];
+        GX_TRY(apply_mpc(op, t, mmp, 1, w.dev, &f2));
+        if (n2 < 1) {
+          set_error("multishift CG: the last hop left no tile sums");
+          return GX_EINVAL;
+        }
+        GX_TRY(launch_ms_fold(ctx, npart, n2, nullptr, 0, w.dev));
+      } else {
+        GX_TRY(apply_mpc(op, t, mmp, 1, w.dev));
+        GX_TRY(launch_ms_dot(ctx, nsites, nsites, p->data, mmp->data, w.dev));
+        GX_TRY(blas_axpby(mmp, mass[0], p, 1.0, mmp, w.dev));
+        GX_TRY(launch_ms_axpy_norm(ctx, nsites, nsites, r->data, mmp->data, w.dev));
+      }
+      GX_TRY(launch_ms_update(ctx, nst, r->data, p->data, ptrs, w.dev, pp));
+      npp = ms_update_blocks(nst);
     }
     GX_CHECK_HIP(hipMemcpyAsync(&w.host[sl], w.dev, sizeof(MsState), hipMemcpyDeviceToHost, stream));
     GX_CHECK_HIP(hipEventRecord(w.ev[sl], stream));
