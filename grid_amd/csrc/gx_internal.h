@@ -257,9 +257,10 @@ struct HopFuse {
   CGState *nxt = nullptr;
   const double *dpart = nullptr;
   int nd = 0;
-  // FP64, r given: r_s -= a (the result + shift sp)_s
+  // FP64, r given: ro_s = r_s - a (the result + shift sp)_s; ro may be r
   const void *sp = nullptr;
   double shift = 0;
+  void *ro = nullptr;
 };
 // Small lattices (hop_split) run the hop with one leg per wave, which launch_dhop_epi then does by
 // itself; ncb = 2 does both checkerboards cb and cb ^ 1 in one launch (operand j of each list).
@@ -375,23 +376,38 @@ struct MsState : Gate {
   int nshift, pad;
   int its[kMaxShift];
 };
+// The vector updates of the shifts run for up to kMsGroup iterations at once; co, cl and ac keep what they need
+// of iteration k in slot k mod kMsGroup: coefficients, shifts with a psi update, shifts with a ps update.
+constexpr int kMsGroup = 8;
+struct MsCoef {
+  double bs, z, as;
+};
+struct MsDev : MsState {
+  uint32_t cl[kMsGroup], ac[kMsGroup];
+  MsCoef co[kMsGroup][kMaxShift];
+};
+struct MsResid {
+  const void *r[kMsGroup];  // the residuals of the iterations, oldest first
+};
 struct MsPtrs {
   void *ps[kMaxShift];
   void *psi[kMaxShift];
 };
 // one multishift iteration's reductions and vector updates on FP64 half fields of nsites sites
 // (stride per half) with the state on the device: d from (p, mmp) (mmp = A p, before the m0
-// shift) and the z / bs recurrences; r += b mmp with |r|^2, the stopping tests and a; then the
-// psi / p / ps updates of k_multishift with the state's coefficients.  dot: 0 -> after the hop,
-// 1 -> after mmp += m0 p
+// shift) and the z / bs recurrences; ro = r + b mmp with |ro|^2, the stopping tests and a; p = a p + r;
+// and for cnt iterations from the first-th on the psi / ps updates of k_multishift.  dot: 0 -> after
+// the hop, 1 -> after mmp += m0 p
 int launch_ms_dot(Ctx *ctx, int64_t nsites, int64_t stride, const void *p, const void *mmp, MsState *st);
-int launch_ms_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, void *r, const void *mmp, MsState *st);
-// pp: ms_update_blocks(n) partials of the new |p|^2
+int launch_ms_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, const void *r, void *ro, const void *mmp,
+                        MsDev *st);
+// pp: ms_p_blocks(n) partials of the new |p|^2
 constexpr int kMsBlocks = 4096;
-int ms_update_blocks(int64_t n);
-int launch_ms_update(Ctx *ctx, int64_t n, const void *r, void *p, const MsPtrs &m, MsState *st, double *pp);
+int ms_p_blocks(int64_t n);
+int launch_ms_p(Ctx *ctx, int64_t n, const void *r, void *p, MsDev *st, double *pp);
+int launch_ms_group(Ctx *ctx, int64_t n, const MsResid &rs, const MsPtrs &m, MsDev *st, int first, int cnt);
 // the finalisers on tile sums of the hop: with pp, n partials of Re<p|A p> and np of |p|^2; without, n of |r|^2
-int launch_ms_fold(Ctx *ctx, const double *partial, int64_t n, const double *pp, int np, MsState *st);
+int launch_ms_fold(Ctx *ctx, const double *partial, int64_t n, const double *pp, int np, MsDev *st);
 // Sums over the lattice of the six plaquettes' and four links' real traces of a device gauge field
 // ([site][mu][3][3] complex double): out_host[0] (plaquettes), out_host[1] (links); out_host holds
 // 2 nparts doubles.  Synchronises the stream.

@@ -578,7 +578,7 @@ struct HopEpi {
   // k_dhop and hop_tile.  EPI 5 (EPI 1 result) and 8 (EPI 3 result): out, and the per-tile slice sums of
   // |out|^2 in npart [tile][LS]; EPI 6 (EPI 1 result) and 7 (EPI 3 result): rv_s -= acoef[astride s]
   // (result)_s in place of storing out, per-tile slice sums of |rv_s|^2; EPI 10 and 9 (FP64): the same with
-  // result + shift sp in place of result
+  // result + shift sp in place of result, the new r in ro
   double *npart;
   cx<S> *rv;
   const double *acoef;
@@ -592,6 +592,7 @@ struct HopEpi {
   int nd;
   const cx<S> *sp;
   T shift;
+  cx<S> *ro;
 };
 
 // this thread's share of the partials of d, and its wave's sum in dsh (one per wave)
@@ -864,7 +865,7 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
           rv[k] = {fma(a, acc[k].r, rv[k].r), fma(a, acc[k].i, rv[k].i)};
           nv += (double)fma(rv[k].r, rv[k].r, rv[k].i * rv[k].i);
         }
-        store_site<S>(ep.rv, rv, o, false);
+        store_site<S>(EPI >= 9 ? ep.ro : ep.rv, rv, o, false);
       } else {
 #pragma unroll
         for (int k = 0; k < 12; k++) nv += (double)fma(acc[k].r, acc[k].r, acc[k].i * acc[k].i);
@@ -1049,7 +1050,7 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
         rv[k] = {fma(a, acc[k].r, rv[k].r), fma(a, acc[k].i, rv[k].i)};
         nv += (double)fma(rv[k].r, rv[k].r, rv[k].i * rv[k].i);
       }
-      store_site<S>(ep.rv, rv, o, false);
+      store_site<S>(EPI >= 9 ? ep.ro : ep.rv, rv, o, false);
     } else {
       if (NORM)
 #pragma unroll
@@ -1352,7 +1353,7 @@ __global__ void __launch_bounds__(512) k_hop_split(SplitArgs<S> A, KGeom g, cons
     if (NORM) nsh[c * 64 + lane] = nv;
   }
   if (NORM || Sto<S>::H) __syncthreads();
-  cx<S> *dst = RUPD ? ep.rv : A.out[j];
+  cx<S> *dst = EPI >= 9 ? ep.ro : RUPD ? ep.rv : A.out[j];
   if (c < 3 && valid) {
     T up = (T)1, inv = (T)1;
     if constexpr (Sto<S>::H) {  // the site's scale, as store_site
@@ -1806,7 +1807,7 @@ int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], vo
   const uint32_t tiles = (uint32_t)((g.H4 + A.SPW - 1) / A.SPW);
   const bool norm = fz && fz->npart && fz->nparts && (epi == 1 || epi == 3) && (fz->r ? (dag && fz->a) : !dag);
   HopEpi<S> ep{nullptr, (const T *)mat, (T)alpha, (const T *)coef, nullptr, nullptr, nullptr, 1, fz ? fz->total : 0,
-               nullptr, nullptr, nullptr, 0, nullptr, (T)0};
+               nullptr, nullptr, nullptr, 0, nullptr, (T)0, nullptr};
   if (fz && fz->nparts) *fz->nparts = 0;
   if (norm) {
     ep.npart = fz->npart;
@@ -1819,6 +1820,7 @@ int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], vo
     ep.nd = fz->nd;
     ep.sp = (const cx<S> *)fz->sp;
     ep.shift = (T)fz->shift;
+    ep.ro = (cx<S> *)fz->ro;
     *fz->nparts = tiles;
   }
   const KGeom k = kgeom(g);
@@ -1913,7 +1915,8 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
                fz ? fz->npart : nullptr,  (cx<S> *)(fz ? fz->r : nullptr),  fz ? fz->a : nullptr,
                fz ? fz->astride : 1,  fz ? fz->total : 0,
                fz ? fz->cur : nullptr, fz ? fz->nxt : nullptr, fz ? fz->dpart : nullptr, fz ? fz->nd : 0,
-               (const cx<S> *)(fz ? fz->sp : nullptr), (T)(fz ? fz->shift : 0.0)};
+               (const cx<S> *)(fz ? fz->sp : nullptr), (T)(fz ? fz->shift : 0.0),
+               (cx<S> *)(fz ? fz->ro : nullptr)};
   // the shifted update exists in FP64
   constexpr bool kShift = std::is_same<S, double>::value;
   if (fz && fz->sp && !kShift) {
@@ -3578,10 +3581,10 @@ static __global__ void __launch_bounds__(1024) k_ms_fin_d(const double *partial,
   }
 }
 
-// r += b mmp (mmp shifted by m0) and |r|^2, block partials
-static __global__ void __launch_bounds__(256) k_ms_axpy_norm(int64_t nsites, int64_t stride, cx<double> *__restrict__ r,
-                                                             const cx<double> *__restrict__ mmp, const MsState *st,
-                                                             double *partial) {
+// ro = r + b mmp (mmp shifted by m0; ro may be r) and |ro|^2, block partials
+static __global__ void __launch_bounds__(256) k_ms_axpy_norm(int64_t nsites, int64_t stride, const cx<double> *r,
+                                                             cx<double> *ro, const cx<double> *__restrict__ mmp,
+                                                             const MsState *st, double *partial) {
   if (gated(st)) return;
   __shared__ double sh[1][4];
   const double b = st->b;
@@ -3598,7 +3601,7 @@ static __global__ void __launch_bounds__(256) k_ms_axpy_norm(int64_t nsites, int
       sr = fma(yv[k].r, yv[k].r, sr);
       sr = fma(yv[k].i, yv[k].i, sr);
     }
-    store_site<double>(r + base, yv, i, false);
+    store_site<double>(ro + base, yv, i, false);
     v[0] += sr;
   }
   block_sum<1>(v, sh);
@@ -3606,8 +3609,9 @@ static __global__ void __launch_bounds__(256) k_ms_axpy_norm(int64_t nsites, int
 }
 
 // c = |r|^2; each active shift's stopping test c z_s^2 < rsq_s; a = c / cp; k += 1 (also once
-// stopped, so the gate of the update that closes the last iteration opens exactly once)
-static __global__ void __launch_bounds__(1024) k_ms_fin_c(const double *partial, int nparts, MsState *st) {
+// stopped, so the gate of the update that closes the last iteration opens exactly once).  The shifts and
+// coefficients of the iteration's vector updates stay in slot k mod kMsGroup.
+static __global__ void __launch_bounds__(1024) k_ms_fin_c(const double *partial, int nparts, MsDev *st) {
   const bool skip = gated(st);
   __shared__ double sh[1][16];
   double v[1] = {0};
@@ -3629,58 +3633,109 @@ static __global__ void __launch_bounds__(1024) k_ms_fin_c(const double *partial,
       st->active = active;
       st->a = c / st->cp;
       if (active == 0 && st->k_conv == INT_MAX) st->k_conv = st->k;
+      st->cl[st->k % kMsGroup] = st->closing;
+      st->ac[st->k % kMsGroup] = active;
     }
-    st->k = st->k + 1;
-  }
-}
-
-// k_multishift with the coefficients of the state (psi_s -= bs_s ps_s for the closing shifts;
-// p = a p + r and ps_s = z_s r + as_s ps_s for the active ones), gated on the iteration it closes; |p|^2 in
-// one partial per workgroup
-static __global__ void __launch_bounds__(256) k_ms_update(int64_t n, const cx<double> *__restrict__ r,
-                                                          cx<double> *__restrict__ p, MsPtrs m, const MsState *st,
-                                                          double *pp) {
-  if (st->k - 1 > st->k_conv || st->k - 1 > st->kmax) return;
-  __shared__ double cbs[kMaxShift], cz[kMaxShift], cas[kMaxShift];
-  const int ns = st->nshift;
-  const uint32_t closing = st->closing, active = st->active;
-  const double a = st->a;
-  if (threadIdx.x < ns) {
-    const int s = threadIdx.x;
-    cbs[s] = st->bs[s];
-    cz[s] = s == 0 ? 1.0 : st->zc[s];
-    cas[s] = s == 0 ? a : a * st->zc[s] * st->bs[s] / (st->zp[s] * st->b);
   }
   __syncthreads();
-  const bool do_p = active != 0;
+  const int s = threadIdx.x, k = st->k;
+  if (!skip && s < st->nshift) {
+    const double a = st->a;
+    st->co[k % kMsGroup][s] = {st->bs[s], s == 0 ? 1.0 : st->zc[s],
+                               s == 0 ? a : a * st->zc[s] * st->bs[s] / (st->zp[s] * st->b)};
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) st->k = k + 1;
+}
+
+// p = a p + r while a shift is active, gated on the iteration it closes; |p|^2 in one partial per workgroup
+static __global__ void __launch_bounds__(256) k_ms_p(int64_t n, const cx<double> *__restrict__ r,
+                                                     cx<double> *__restrict__ p, const MsState *st, double *pp) {
+  if (st->k - 1 > st->k_conv || st->k - 1 > st->kmax || st->active == 0) return;
+  const double a = st->a;
   double v[1] = {0};
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const cx<double> rv = r[i];
-    if (do_p) {
-      cx<double> pv = p[i];
-      pv = {fma(a, pv.r, rv.r), fma(a, pv.i, rv.i)};
-      p[i] = pv;
-      v[0] = fma(pv.r, pv.r, fma(pv.i, pv.i, v[0]));
-    }
-    for (int s = 0; s < ns; s++) {
-      const bool dpsi = (closing >> s) & 1u, dps = (active >> s) & 1u;
-      if (!dpsi && !dps) continue;
-      cx<double> *ps = (cx<double> *)m.ps[s];
-      cx<double> pv = ps[i];
-      if (dpsi) {
-        cx<double> *psi = (cx<double> *)m.psi[s];
-        const cx<double> xv = psi[i];
-        psi[i] = {fma(-cbs[s], pv.r, xv.r), fma(-cbs[s], pv.i, xv.i)};
-      }
-      if (dps) {
-        pv = {fma(cz[s], rv.r, cas[s] * pv.r), fma(cz[s], rv.i, cas[s] * pv.i)};
-        ps[i] = pv;
-      }
-    }
+    cx<double> pv = p[i];
+    pv = {fma(a, pv.r, rv.r), fma(a, pv.i, rv.i)};
+    p[i] = pv;
+    v[0] = fma(pv.r, pv.r, fma(pv.i, pv.i, v[0]));
   }
   __shared__ double sh[1][4];
   block_sum<1>(v, sh);
   write_partial<1>(v, pp);
+}
+
+// The shifts' vectors for the iterations first .. first + cnt - 1 at once, in their order: psi_s -= bs_s ps_s
+// where s was iterating, then ps_s = z_s r + as_s ps_s where it goes on, with the residuals rs[j] and the
+// coefficients that k_ms_fin_c left of each.  Bound by memory: four passes over ps_s and psi_s per shift,
+// which a launch per iteration spent for each one of them.  With kMsGroup = 8 at 12^3x24 x 8 and 12 shifts:
+// 29 us per iteration, and 15 for p alone, against 195, and the hops between find more of their fields in the
+// cache (27 us for 34).  The next shift's loads are in flight while one is updated.
+static __global__ void __launch_bounds__(256) k_ms_group(int64_t n, MsResid rs, MsPtrs m, const MsDev *st, int first,
+                                                         int cnt) {
+  __shared__ MsCoef co[kMaxShift][kMsGroup];
+  __shared__ uint32_t cl[kMaxShift], ac[kMaxShift];  // bit j: psi_s (ps_s) updated in iteration first + j
+  __shared__ int list[kMaxShift], nlist;
+  const int last = st->k_conv < st->kmax ? st->k_conv : st->kmax, ns = st->nshift;
+  const int nv = last - first + 1 < cnt ? last - first + 1 : cnt;
+  if (nv <= 0) return;
+  for (int q = threadIdx.x; q < ns * nv; q += blockDim.x) co[q / nv][q % nv] = st->co[(first + q % nv) % kMsGroup][q / nv];
+  if (threadIdx.x < ns) {
+    uint32_t c = 0, a = 0;
+    for (int j = 0; j < nv; j++) {
+      c |= ((st->cl[(first + j) % kMsGroup] >> threadIdx.x) & 1u) << j;
+      a |= ((st->ac[(first + j) % kMsGroup] >> threadIdx.x) & 1u) << j;
+    }
+    cl[threadIdx.x] = c;
+    ac[threadIdx.x] = a;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int k = 0;
+    for (int s = 0; s < ns; s++)
+      if (cl[s] | ac[s]) list[k++] = s;
+    nlist = k;
+  }
+  __syncthreads();
+  const int nl = nlist;
+  if (nl == 0) return;
+  const uint32_t all = (1u << nv) - 1;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    cx<double> rv[kMsGroup];
+#pragma unroll
+    for (int j = 0; j < kMsGroup; j++)
+      if (j < nv) rv[j] = ((const cx<double> *)rs.r[j])[i];
+    cx<double> pn = ((const cx<double> *)m.ps[list[0]])[i], xn = {0, 0};
+    if (cl[list[0]]) xn = ((const cx<double> *)m.psi[list[0]])[i];
+    for (int q = 0; q < nl; q++) {
+      const int s = list[q];
+      cx<double> pv = pn, xv = xn;
+      if (q + 1 < nl) {
+        const int t = list[q + 1];
+        pn = ((const cx<double> *)m.ps[t])[i];
+        if (cl[t]) xn = ((const cx<double> *)m.psi[t])[i];
+      }
+      const uint32_t c = cl[s], a = ac[s];
+      if (nv == kMsGroup && c == all && a == all) {
+#pragma unroll
+        for (int j = 0; j < kMsGroup; j++) {
+          const MsCoef k = co[s][j];
+          xv = {fma(-k.bs, pv.r, xv.r), fma(-k.bs, pv.i, xv.i)};
+          pv = {fma(k.z, rv[j].r, k.as * pv.r), fma(k.z, rv[j].i, k.as * pv.i)};
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < kMsGroup; j++) {
+          const MsCoef k = co[s][j];
+          if ((c >> j) & 1u) xv = {fma(-k.bs, pv.r, xv.r), fma(-k.bs, pv.i, xv.i)};
+          if ((a >> j) & 1u) pv = {fma(k.z, rv[j].r, k.as * pv.r), fma(k.z, rv[j].i, k.as * pv.i)};
+        }
+      }
+      if (c) ((cx<double> *)m.psi[s])[i] = xv;
+      if (a) ((cx<double> *)m.ps[s])[i] = pv;
+    }
+  }
 }
 
 // ---------------- slice matrices (Lattice_reduction.h:717-776) ----------------
@@ -4069,7 +4124,7 @@ int launch_ms_dot(Ctx *ctx, int64_t nsites, int64_t stride, const void *p, const
   return GX_OK;
 }
 
-int launch_ms_fold(Ctx *ctx, const double *partial, int64_t n, const double *pp, int np, MsState *st) {
+int launch_ms_fold(Ctx *ctx, const double *partial, int64_t n, const double *pp, int np, MsDev *st) {
   if (n < 1 || n > INT_MAX) {
     set_error("multishift fold: %lld tiles", (long long)n);
     return GX_EINVAL;
@@ -4080,20 +4135,32 @@ int launch_ms_fold(Ctx *ctx, const double *partial, int64_t n, const double *pp,
   return GX_OK;
 }
 
-int launch_ms_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, void *r, const void *mmp, MsState *st) {
+int launch_ms_axpy_norm(Ctx *ctx, int64_t nsites, int64_t stride, const void *r, void *ro, const void *mmp,
+                        MsDev *st) {
   const int nb = red_blocks(nsites);
-  hipLaunchKernelGGL(k_ms_axpy_norm, dim3(nb), dim3(256), 0, ctx->stream, nsites, stride, (cx<double> *)r,
-                     (const cx<double> *)mmp, (const MsState *)st, ctx->red_partial);
+  hipLaunchKernelGGL(k_ms_axpy_norm, dim3(nb), dim3(256), 0, ctx->stream, nsites, stride, (const cx<double> *)r,
+                     (cx<double> *)ro, (const cx<double> *)mmp, (const MsState *)st, ctx->red_partial);
   hipLaunchKernelGGL(k_ms_fin_c, dim3(1), dim3(1024), 0, ctx->stream, (const double *)ctx->red_partial, nb, st);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
 
-int ms_update_blocks(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, kMsBlocks); }
+int ms_p_blocks(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, kMsBlocks); }
 
-int launch_ms_update(Ctx *ctx, int64_t n, const void *r, void *p, const MsPtrs &m, MsState *st, double *pp) {
-  hipLaunchKernelGGL(k_ms_update, dim3(ms_update_blocks(n)), dim3(256), 0, ctx->stream, n, (const cx<double> *)r,
-                     (cx<double> *)p, m, (const MsState *)st, pp);
+int launch_ms_p(Ctx *ctx, int64_t n, const void *r, void *p, MsDev *st, double *pp) {
+  hipLaunchKernelGGL(k_ms_p, dim3(ms_p_blocks(n)), dim3(256), 0, ctx->stream, n, (const cx<double> *)r,
+                     (cx<double> *)p, (const MsState *)st, pp);
+  GX_CHECK_HIP(hipGetLastError());
+  return GX_OK;
+}
+
+int launch_ms_group(Ctx *ctx, int64_t n, const MsResid &rs, const MsPtrs &m, MsDev *st, int first, int cnt) {
+  if (first < 1 || cnt < 1 || cnt > kMsGroup) {
+    set_error("multishift group: %d iterations from %d", cnt, first);
+    return GX_EINVAL;
+  }
+  hipLaunchKernelGGL(k_ms_group, dim3(stream_blocks(n)), dim3(256), 0, ctx->stream, n, rs, m, (const MsDev *)st, first,
+                     cnt);
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }

@@ -85,7 +85,7 @@ struct MrhsWork {
 };
 
 struct MsWork {
-  MsState *dev = nullptr;
+  MsDev *dev = nullptr;
   MsState *host = nullptr;  // pinned, 2 slots
   hipEvent_t ev[2] = {};
 };
@@ -1413,13 +1413,14 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
   const int cb = src->cb;
   r->cb = p->cb = mmp->cb = tmp->cb = cb;
   std::vector<Field *> ps(nshift, nullptr);
+  std::vector<Field *> ring;
   struct Owned {
     std::vector<Field *> &v;
     ~Owned() {
       for (Field *f : v)
         if (f) field_destroy(f);
     }
-  } owned{ps};
+  } owned{ps}, owned_ring{ring};
   for (int s = 0; s < nshift; s++) {
     GX_TRY(field_create(op->ctx, op->g, GX_F64, GX_EVEN, &ps[s]));
     ps[s]->cb = cb;
@@ -1503,7 +1504,7 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
   GX_TRY(solver_work(op, &sw));
   MsWork &w = sw->ms;
   if (!w.dev) {
-    hipError_t e = hipMalloc(&w.dev, sizeof(MsState));
+    hipError_t e = hipMalloc(&w.dev, sizeof(MsDev));
     if (e == hipSuccess) e = hipHostMalloc(&w.host, 2 * sizeof(MsState), hipHostMallocDefault);
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipEventCreateWithFlags(&w.ev[i], hipEventDisableTiming);
     if (e != hipSuccess) {
@@ -1551,10 +1552,33 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
   if (!npart && op->g.Ls == 1 && hop_norm_tiles(op->g.H4, 1) <= kRedBlocks * kMaxRhs - kMsBlocks)
     npart = ctx->red_partial;
   constexpr int kMsNorm = 4;  // result slot
+  // Each iteration leaves its residual in a new field of a ring, and the shifts' vectors are updated for a
+  // ring's worth of iterations at once (k_ms_group); where there is no room for kMsGroup fields, for fewer.
+  std::vector<void *> rr{r->data};
+  while ((int)rr.size() < kMsGroup && (int)rr.size() < maxit) {
+    Field *f = nullptr;
+    if (field_create(op->ctx, op->g, GX_F64, GX_EVEN, &f) != GX_OK) {
+      (void)hipGetLastError();
+      break;
+    }
+    ring.push_back(f);
+    rr.push_back(f->data);
+  }
+  const int group = (int)rr.size();
+  int done = 0;  // iterations whose shift updates are enqueued
+  auto flush = [&]() -> int {
+    if (done == enqueued) return GX_OK;
+    MsResid rs{};
+    for (int j = done; j < enqueued; j++) rs.r[j - done] = rr[(j + 1) % group];
+    GX_TRY(launch_ms_group(ctx, nst, rs, ptrs, w.dev, done + 1, enqueued - done));
+    done = enqueued;
+    return GX_OK;
+  };
   int npp = 0;
   GX_TRY(launch_reduce<double>(ctx, 1, nsites, nsites, p->data, nullptr, nullptr, 0, kMsNorm));
   auto enqueue = [&](int sl) -> int {
-    for (int i = 0; i < batch && enqueued < maxit; i++, enqueued++) {
+    for (int i = 0; i < batch && enqueued < maxit; i++) {
+      void *rin = rr[enqueued % group], *rout = rr[(enqueued + 1) % group];
       // Where the tuned hop has the fused epilogues: Re<p|A p> = |t|^2 (t = Mpc p) from its tile sums, |p|^2 from
       // the update before, and the last hop takes r += b (A p + m0 p) with |r|^2: six field passes less.
       // (12^3x24 x 8, FP64, per iteration: dot 12, axpby 14, axpy_norm 18 us saved for 7 us more in the hops)
@@ -1568,7 +1592,8 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
         GX_TRY(launch_ms_fold(ctx, npart, n1, npp ? pp : ctx->red_result + kMsNorm, npp ? npp : 1, w.dev));
         HopFuse f2 = f1;
         f2.nparts = &n2;
-        f2.r = r->data;
+        f2.r = rin;
+        f2.ro = rout;
         f2.a = &w.dev->mb;  // device address (not dereferenced here)
         f2.astride = 0;
         f2.sp = p->data;
@@ -1583,10 +1608,12 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
         GX_TRY(apply_mpc(op, t, mmp, 1, w.dev));
         GX_TRY(launch_ms_dot(ctx, nsites, nsites, p->data, mmp->data, w.dev));
         GX_TRY(blas_axpby(mmp, mass[0], p, 1.0, mmp, w.dev));
-        GX_TRY(launch_ms_axpy_norm(ctx, nsites, nsites, r->data, mmp->data, w.dev));
+        GX_TRY(launch_ms_axpy_norm(ctx, nsites, nsites, rin, rout, mmp->data, w.dev));
       }
-      GX_TRY(launch_ms_update(ctx, nst, r->data, p->data, ptrs, w.dev, pp));
-      npp = ms_update_blocks(nst);
+      GX_TRY(launch_ms_p(ctx, nst, rout, p->data, w.dev, pp));
+      npp = ms_p_blocks(nst);
+      enqueued++;
+      if (enqueued - done == group) GX_TRY(flush());
     }
     GX_CHECK_HIP(hipMemcpyAsync(&w.host[sl], w.dev, sizeof(MsState), hipMemcpyDeviceToHost, stream));
     GX_CHECK_HIP(hipEventRecord(w.ev[sl], stream));
@@ -1607,6 +1634,7 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
     GX_TRY(enqueue(slot));
     slot = 1 - slot;
   }
+  GX_TRY(flush());
   // the final state (launches past the stop leave it as the stop found it, but for k)
   GX_CHECK_HIP(hipMemcpyAsync(&w.host[0], w.dev, sizeof(MsState), hipMemcpyDeviceToHost, stream));
   GX_CHECK_HIP(hipStreamSynchronize(stream));

@@ -43,3 +43,21 @@ def test_cg_fold(kind, Ls, dims, graph):
         assert np.linalg.norm(u - v) < tol * np.linalg.norm(v)
     D.close()
     ctx.close()
+
+
+@pytest.mark.parametrize('maxit', [1, 7, 8, 9, 19])
+def test_multishift_stopped(maxit):
+    """Stopped anywhere in a group of iterations, the unshifted system is at the iterate of CG (whose count
+    includes the multishift's first one)."""
+    dims, Ls = (8, 4, 6, 8), 4
+    ctx = gx.Context(0)
+    D = gx.FermionOp(ctx, gx.random_gauge(dims, 61, 0.3), dims, Ls, 'mobius', mass=0.1)
+    src = D.field(gx.F64, gx.ODD).upload(R.pick(gx.gaussian_fermion(dims, Ls, 62), dims, gx.ODD))
+    x, ms = D.field(gx.F64, gx.ODD), [D.field(gx.F64, gx.ODD) for _ in range(2)]
+    D.cg(src, x, tol=1e-30, maxit=maxit + 1)
+    st = D.cg_multishift(src, ms, [0.0, 1.0], [1e-30] * 2, maxit=maxit)
+    assert not st[0]['converged'] and st[0]['iterations'] == maxit
+    # 20 iterations of the same recurrences, rounded in another order
+    assert np.linalg.norm(ms[0].download() - x.download()) < 1e-10 * np.linalg.norm(x.download())
+    D.close()
+    ctx.close()
