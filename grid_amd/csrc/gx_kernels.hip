@@ -260,7 +260,7 @@ struct KGeom {
   // blocked sweep (tile map 4): blocks of Lxh x by x bz sites in one t-slice; a block's t-slices
   // are consecutive in the sweep (t fastest), blocks ordered y-block first
   int by, bz, nby;
-  FDiv fLxh, fL1, fL2, fL3, fby, fnby, fbs;  // division by Lxh, Ly, Lz, Lt, by, nby, Lxh*by*bz
+  FDiv fLxh, fL1, fL2, fL3, fby, fnby, fbs, fbp;  // division by Lxh, Ly, Lz, Lt, by, nby, Lxh*by*bz, Lxh*by
 };
 
 static void set_sweep_blocks(KGeom &k, int by, int bz) {
@@ -270,6 +270,7 @@ static void set_sweep_blocks(KGeom &k, int by, int bz) {
   k.fby = make_fdiv(by);
   k.fnby = make_fdiv(k.nby);
   k.fbs = make_fdiv((uint32_t)k.Lxh * by * bz);
+  k.fbp = make_fdiv((uint32_t)k.Lxh * by);
 }
 
 static KGeom kgeom(const Geom &g) {
@@ -298,6 +299,79 @@ __device__ __forceinline__ uint32_t sweep_site(const KGeom &g, uint32_t r) {
   const uint32_t zz = fdiv(w2, g.fby), yy = w2 - zz * (uint32_t)g.by;
   const uint32_t y = byi * g.by + yy, z = bzi * g.bz + zz;
   return xh + (uint32_t)g.Lxh * (y + (uint32_t)g.L[1] * (z + (uint32_t)g.L[2] * t));
+}
+
+// A half-site and its coordinates (xh: x / 2).
+struct SiteAt {
+  uint32_t h, xh, y, z, t;
+};
+
+__device__ __forceinline__ SiteAt site_at(const KGeom &g, uint32_t h) {
+  const uint32_t r1 = fdiv(h, g.fLxh), r2 = fdiv(r1, g.fL1), r3 = fdiv(r2, g.fL2);
+  return {h, h - r1 * (uint32_t)g.Lxh, r1 - r2 * (uint32_t)g.L[1], r2 - r3 * (uint32_t)g.L[2], r3};
+}
+
+// The blocked sweep from a position that is uniform over the workgroup: its block-slice (origin y, z, t) and the
+// position w in it are found once, in scalar registers; the lanes' positions then need the divisions inside
+// a block only, where the eight divisions of sweep_site and site_at each take two quarter-rate multiplies in a
+// dependent chain ahead of the first load (FP16 24^3x48 x 12 Schur operator, bound by its instructions: 708 us
+// for 718; FP64 and FP32, bound by the memory, are unchanged).
+struct SweepAt {
+  uint32_t w, y, z, t;
+};
+
+__device__ __forceinline__ SweepAt sweep_at(const KGeom &g, uint32_t r) {
+  const uint32_t q = fdiv(r, g.fbs), yzb = fdiv(q, g.fL3), bzi = fdiv(yzb, g.fnby);
+  return {r - q * g.fbs.d, (yzb - bzi * (uint32_t)g.nby) * (uint32_t)g.by, bzi * (uint32_t)g.bz,
+          q - yzb * (uint32_t)g.L[3]};
+}
+
+// the half-site off positions on (XYZ: with its coordinates); off may reach into the next block-slices
+template <bool XYZ>
+__device__ __forceinline__ SiteAt sweep_off(const KGeom &g, const SweepAt &b, uint32_t off) {
+  uint32_t w = b.w + off, y = b.y, z = b.z, t = b.t;
+  while (w >= g.fbs.d) {
+    w -= g.fbs.d;
+    if (++t == (uint32_t)g.L[3]) {
+      t = 0;
+      y += (uint32_t)g.by;
+      if (y == (uint32_t)g.L[1]) {
+        y = 0;
+        z += (uint32_t)g.bz;
+      }
+    }
+  }
+  // h = x-y plane position of the block origin + w, stepped from planes of the block to planes of the lattice
+  const uint32_t zz = fdiv(w, g.fbp);
+  SiteAt a;
+  a.h = (uint32_t)g.sY * y + (uint32_t)g.sZ * z + (uint32_t)g.sT * t + w + zz * ((uint32_t)g.sZ - g.fbp.d);
+  if (XYZ) {
+    const uint32_t v = w - zz * g.fbp.d, yy = fdiv(v, g.fLxh);
+    a.xh = v - yy * (uint32_t)g.Lxh;
+    a.y = y + yy;
+    a.z = z + zz;
+    a.t = t;
+  }
+  return a;
+}
+
+// Field entries (site Ls + s) of the 8 neighbours (x+, y+, z+, t+, x-, y-, z-, t-) of a site of checkerboard
+// cb_out: the site's own entry and one of two uniform steps per direction, so the only multiply is its own.
+__device__ __forceinline__ void entry_neighbours(const KGeom &g, const SiteAt &a, int cb_out, uint32_t LS, uint32_t s,
+                                                 uint32_t *ne) {
+  const uint32_t e = a.h * LS + s, Lxh = (uint32_t)g.Lxh;
+  const uint32_t dY = (uint32_t)g.sY * LS, dZ = (uint32_t)g.sZ * LS, dT = (uint32_t)g.sT * LS;
+  const uint32_t wX = (Lxh - 1) * LS, wY = ((uint32_t)g.L[1] - 1) * dY, wZ = ((uint32_t)g.L[2] - 1) * dZ,
+                 wT = ((uint32_t)g.L[3] - 1) * dT;
+  const bool odd = ((uint32_t)cb_out + a.y + a.z + a.t) & 1u;  // x = 2 xh + odd
+  ne[0] = odd ? (a.xh + 1 == Lxh ? e - wX : e + LS) : e;
+  ne[4] = odd ? e : (a.xh == 0 ? e + wX : e - LS);
+  ne[1] = a.y + 1 == (uint32_t)g.L[1] ? e - wY : e + dY;
+  ne[5] = a.y == 0 ? e + wY : e - dY;
+  ne[2] = a.z + 1 == (uint32_t)g.L[2] ? e - wZ : e + dZ;
+  ne[6] = a.z == 0 ? e + wZ : e - dZ;
+  ne[3] = a.t + 1 == (uint32_t)g.L[3] ? e - wT : e + dT;
+  ne[7] = a.t == 0 ? e + wT : e - dT;
 }
 
 __device__ __forceinline__ bool gated(const Gate *gate) {
@@ -679,18 +753,8 @@ __device__ __forceinline__ void wave_sync() {
 // One lane per (4D half-site h, s): s fastest, 64/LS sites per wave, 4 waves per workgroup, so a
 // wave reads each neighbour's s-row contiguously and the lanes of one site share its links.
 // flags: bit 0 = non-temporal output stores.  ORD: leg order (0 Grid's, 1 paired directions).
-// Waves per SIMD the compiler must leave VGPRs for (512 / waves each).  The FP16-storage hop with
-// prefetch in Grid's leg order fits three waves (168 VGPRs) with at most two spilled against 174
-// unbounded (two waves), which made its 12-RHS form 16% and the 16^4 x 16 one 8% faster; the other
-// FP16 forms (and Ls < 4) spill up to 35 VGPRs under the same bound and stay unbounded.
-template <typename S, int LS, bool PF, int ORD>
-constexpr int dhop_waves() {
-  return (Sto<S>::H && PF && ORD == 0 && LS >= 4) ? 3 : 1;
-}
-
 template <typename S, int LS, bool DAG, bool PF, int ORD, int EPI>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(dhop_waves<S, LS, PF, ORD>())))
-k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
+__global__ void __launch_bounds__(256) k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
                                               const cx<S> *__restrict__ U, KGeom g, int cb_out,
                                               const Gate *__restrict__ gate, uint32_t ntiles, int map, int flags,
                                               HopEpi<S> ep) {
@@ -717,9 +781,12 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   const int lsb = w * SPW + ls;
   const bool valid = (ls < SPW) && (h0 + lsb < H4);
   // idle lanes compute in-bounds addresses and skip the work
-  const uint32_t h = sweep ? sweep_site(g, valid ? h0 + lsb : h0) : (valid ? h0 + lsb : h0);
-  uint32_t nb[8];
-  site_neighbours(g, h, cb_out, nb);
+  const uint32_t off = valid ? (uint32_t)lsb : 0u;
+  const SweepAt sw = sweep ? sweep_at(g, h0) : SweepAt{};
+  const SiteAt at = sweep ? sweep_off<true>(g, sw, off) : site_at(g, h0 + off);
+  const uint32_t h = at.h;
+  uint32_t ne[8];
+  entry_neighbours(g, at, cb_out, LS, (uint32_t)s, ne);
   // Link tile of the workgroup: global -> registers first, then the first neighbour loads, then
   // registers -> LDS and a barrier that waits for LDS traffic only, so the neighbour loads stay in
   // flight across it.
@@ -733,16 +800,18 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   double ds = 0;  // loaded first: loads return in order, and this one is waited for first
   if (RUPD) ds = d_share(ep);
   if (LDSU) {
-    const uint32_t hs = sweep && ustage ? sweep_site(g, h0 + usite) : h0 + usite;
 #pragma unroll
-    for (int j = 0; j < NU; j++) {
-      const uint32_t pk = ugrp + G * j;
-      ureg[j] = ustage && pk < 72 ? ldc<S>(U, pk * H4 + hs) : cx<T>{0, 0};
+    for (int j = 0; j < NU; j++) ureg[j] = {0, 0};
+    if (ustage) {
+      uint32_t i = ugrp * H4 + (sweep ? sweep_off<false>(g, sw, usite).h : h0 + usite);
+#pragma unroll
+      for (int j = 0; j < NU; j++, i += G * H4)
+        if (G * (j + 1) <= 72 || ugrp + G * j < 72) ureg[j] = ldc<S>(U, i);
     }
   }
   cx<T> fa[12], fb[12];
-  T sa = load_site_raw<S>(fa, in, leg_idx<DAG, ORD, 0>(nb, LS, s)), sb = (T)1;
-  if (PF) sb = load_site_raw<S>(fb, in, leg_idx<DAG, ORD, 1>(nb, LS, s));
+  T sa = load_site_raw<S>(fa, in, leg_idx<DAG, ORD, 0>(ne, 1, 0)), sb = (T)1;
+  if (PF) sb = load_site_raw<S>(fb, in, leg_idx<DAG, ORD, 1>(ne, 1, 0));
   __shared__ double dsh[RUPD ? 4 : 1];
   if (RUPD && ep.cur) {
     ds = wave_sum(ds);
@@ -751,10 +820,8 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   if (LDSU) {
     if (ugrp < (uint32_t)G) {
 #pragma unroll
-      for (int j = 0; j < NU; j++) {
-        const uint32_t pk = ugrp + G * j;
-        if (pk < 72) lds[usite * kLinkPad + pk] = ureg[j];
-      }
+      for (int j = 0; j < NU; j++)
+        if (G * (j + 1) <= 72 || ugrp + G * j < 72) lds[usite * kLinkPad + ugrp + G * j] = ureg[j];
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
@@ -769,7 +836,7 @@ k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
   cx<T> acc[12];
 #pragma unroll
   for (int k = 0; k < 12; k++) acc[k] = {0, 0};
-  if (valid) hop_site<T, S, DAG, PF, ORD, LDSU>(acc, fa, fb, sa, sb, in, U, ul, nb, LS, s, h, H4);
+  if (valid) hop_site<T, S, DAG, PF, ORD, LDSU>(acc, fa, fb, sa, sb, in, U, ul, ne, 1, 0, h, H4);
   const uint32_t o = h * LS + s;
   if (MAT) {
     // every wave has finished reading links: reuse the LDS for the hop results [w][k][lane]
@@ -995,10 +1062,11 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
   const uint32_t p0 = tile * sh.SPB;
   const bool valid = p0 + hl < H4;
   // lanes past the lattice take the tile's first site: in-bounds addresses, work skipped
-  const uint32_t pos = valid ? p0 + hl : p0;
-  const uint32_t h = sweep ? sweep_site(g, pos) : pos;
-  uint32_t nb[8];
-  site_neighbours(g, h, cb_out, nb);
+  const uint32_t off = valid ? hl : 0u;
+  const SiteAt at = sweep ? sweep_off<true>(g, sweep_at(g, p0), off) : site_at(g, p0 + off);
+  const uint32_t h = at.h;
+  uint32_t ne[8];
+  entry_neighbours(g, at, cb_out, LS, s, ne);
   double ds = 0;
   if (RUPD) ds = d_share(ep);
   // links of tile site hl: thread (hl, s) loads entries s, s + LS, ... (< 72)
@@ -1009,8 +1077,8 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
     ureg[j] = pk < 72 ? ldc<S>(U, pk * H4 + h) : cx<T>{0, 0};
   }
   cx<T> fa[12], fb[12];
-  T sa = load_site_raw<S>(fa, in, leg_idx<DAG, 0, 0>(nb, LS, s));
-  T sb = load_site_raw<S>(fb, in, leg_idx<DAG, 0, 1>(nb, LS, s));
+  T sa = load_site_raw<S>(fa, in, leg_idx<DAG, 0, 0>(ne, 1, 0));
+  T sb = load_site_raw<S>(fb, in, leg_idx<DAG, 0, 1>(ne, 1, 0));
   __shared__ double dsh[RUPD ? kGenMaxWaves : 1];
   if (RUPD && ep.cur) {
     ds = wave_sum(ds);
@@ -1027,7 +1095,7 @@ __device__ __forceinline__ void hop_tile(const cx<S> *__restrict__ in, cx<S> *__
   cx<T> acc[12];
 #pragma unroll
   for (int k = 0; k < 12; k++) acc[k] = {0, 0};
-  if (valid) hop_site<T, S, DAG, true, 0, true>(acc, fa, fb, sa, sb, in, U, lds + hl * kLinkPad, nb, LS, s, h, H4);
+  if (valid) hop_site<T, S, DAG, true, 0, true>(acc, fa, fb, sa, sb, in, U, lds + hl * kLinkPad, ne, 1, 0, h, H4);
   const uint32_t o = h * LS + s;
   if (MAT) group_matrix<T>(acc, lds, ep.mat, sh, t, hl, s, epb);
   if constexpr (BAND) group_band<S, DAG>(acc, lds, ep, sh, t, hl, s, epb, o);
