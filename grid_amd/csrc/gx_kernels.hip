@@ -753,6 +753,23 @@ __device__ __forceinline__ void wave_sync() {
 // One lane per (4D half-site h, s): s fastest, 64/LS sites per wave, 4 waves per workgroup, so a
 // wave reads each neighbour's s-row contiguously and the lanes of one site share its links.
 // flags: bit 0 = non-temporal output stores.  ORD: leg order (0 Grid's, 1 paired directions).
+// complex numbers of LDS: the links of a tile (0: read from memory) and the slices staged by an epilogue
+template <typename T, int LS>
+constexpr int dhop_links() {
+  return LS > 1 && 4 * (64 / LS) * kLinkPad * sizeof(cx<T>) <= 40960 ? 4 * (64 / LS) * kLinkPad : 0;
+}
+template <int EPI>
+constexpr int dhop_stage() {
+  return EPI == 2 || EPI == 3 || (EPI >= 7 && EPI <= 9) ? 4 * 12 * 64 : 0;
+}
+// unused LDS that leaves room for two workgroups in the 160 KB of a CU, not for three
+template <typename S, int LS, int EPI>
+constexpr int dhop_pad() {
+  const int n = dhop_links<typename Sto<S>::C, LS>(), m = dhop_stage<EPI>();
+  const int used = (n > m ? n : m) * (int)sizeof(cx<typename Sto<S>::C>);
+  return used < 55296 ? 55296 - used : 0;
+}
+
 template <typename S, int LS, bool DAG, bool PF, int ORD, int EPI>
 __global__ void __launch_bounds__(256) k_dhop(const cx<S> *__restrict__ in, cx<S> *__restrict__ out,
                                               const cx<S> *__restrict__ U, KGeom g, int cb_out,
@@ -762,12 +779,12 @@ __global__ void __launch_bounds__(256) k_dhop(const cx<S> *__restrict__ in, cx<S
   if (gated(gate)) return;
   constexpr int SPW = 64 / LS;
   constexpr int SPB = 4 * SPW;
-  constexpr bool LDSU = (LS > 1) && (SPB * kLinkPad * sizeof(cx<T>) <= 40960);
-  constexpr int NLINK = LDSU ? SPB * kLinkPad : 1;
+  constexpr bool LDSU = dhop_links<T, LS>() > 0;
+  constexpr int NLINK = LDSU ? dhop_links<T, LS>() : 1;
   constexpr bool MAT = EPI == 2, BAND = EPI == 3 || (EPI >= 7 && EPI <= 9);
   constexpr bool PHI = EPI == 1 || EPI == 5 || EPI == 6 || EPI == 10;
   constexpr bool NORM = EPI >= 5, RUPD = EPI == 6 || EPI == 7 || EPI >= 9;
-  constexpr int NSTAGE = MAT || BAND ? 4 * 12 * 64 : 1;
+  constexpr int NSTAGE = MAT || BAND ? dhop_stage<EPI>() : 1;
   __shared__ cx<T> lds[NLINK > NSTAGE ? NLINK : NSTAGE];  // links, then (MAT) the hop results
   const bool sweep = map == 4;  // blocked sweep: tiles are runs of the sweep order, XCD slabs
   const uint32_t tile = tile_of_block(blockIdx.x, gridDim.x, sweep ? 1 : map);
@@ -1961,12 +1978,18 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   if (map == 4 && g.Ls == 1) map = g.H4 >= (1 << 19) ? 2 : 1;
   KGeom k = kgeom(g);
   if (map == 4) {
-    // blocks of Lxh x by x bz sites per t-slice with three t-slices of the input (and the links)
-    // within 3.5 MB of an XCD's L2; halve by or bz while they are even and the block is too big
+    // blocks of Lxh x by x bz sites per t-slice with three t-slices of the input (and the links) within
+    // 4.5 MB, about an XCD's L2 (4.2 where phi streams through it too), halving by or bz while they are even
+    // and the block is too big.  by stays at twice bz or more, as the rows of an x-y plane are one run of
+    // memory, but for few slices, where the links are half of the traffic (32^3x48 x 4 FP32: 267 us for 282).
+    // Hop, against 3.5 MB with by next to bz: 24^4 x 12 FP64 266 us for 272 (12 x 3 for 6 x 3; Mdag on its
+    // way through phi 677 for 664), FP32 with the occupancy below 126 for 143 (12 x 6 for 6 x 6); 32^4 x 8
+    // FP64 567 for 577 and Mdag 1439 for 1467 (8 x 4 for 4 x 4); 32^3x64 x 12 FP16 565 for 576.
+    const double room = epi == 1 || epi == 3 ? 4.2e6 : 4.5e6;
     const double site_bytes = (double)g.Ls * 12 * sizeof(cx<S>) + 72.0 * sizeof(cx<S>);
     int by = g.L[1], bz = g.L[2];
-    while (3.0 * k.Lxh * by * bz * site_bytes > 3.5e6) {
-      if (bz >= by && bz % 2 == 0) bz /= 2;
+    while (3.0 * k.Lxh * by * bz * site_bytes > room) {
+      if ((g.Ls > 4 ? 2 * bz : bz) >= by && bz % 2 == 0) bz /= 2;
       else if (by % 2 == 0) by /= 2;
       else if (bz % 2 == 0) bz /= 2;
       else break;
@@ -2146,9 +2169,15 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
   // EPI 5: kepi 1, dag 0; EPI 8: kepi 3, dag 0; EPI 6: kepi 1, dag 1, r; EPI 7: kepi 3, dag 1, r
   const bool norm = fz && fz->npart && fz->nparts && (kepi == 1 || kepi == 3) && (fz->r ? (dag && fz->a) : !dag);
   if (norm) *fz->nparts = ntiles;
-#define GX_DHOP_GO(LS, DAG, PF, ORD, EPI)                                                                         \
-  hipLaunchKernelGGL((k_dhop<S, LS, DAG, PF, ORD, EPI>), dim3(blocks), dim3(256), 0, st, pin, pout, pU, k, cb_out, \
-                     gate, ntiles, map, flags, ep)
+  // FP32 fields and links beyond the 256 MB Infinity Cache: two workgroups per CU instead of four, by unused LDS.
+  // What the XCD has in flight then still finds its neighbours in the L2: 24^4 x 12 124 us for 143 (with the
+  // blocks above), 32^3x64 x 12 852 for 919.  Inside the cache it is 5-8% slower, and FP64 (whose registers
+  // leave two or three anyway) and FP16 (bound by its instructions) gain nothing.
+  const double moved = (double)g.H4 * sizeof(cx<S>) * ((epi == 1 || epi == 3 ? 36.0 : 24.0) * g.Ls + 72.0);
+  const bool thin = std::is_same<S, float>::value && moved > 256e6;
+#define GX_DHOP_GO(LS, DAG, PF, ORD, EPI)                                                                          \
+  hipLaunchKernelGGL((k_dhop<S, LS, DAG, PF, ORD, EPI>), dim3(blocks), dim3(256),                                  \
+                     (thin ? dhop_pad<S, LS, EPI>() : 0), st, pin, pout, pU, k, cb_out, gate, ntiles, map, flags, ep)
 #define GX_DHOP_CASE_O(LS, ORD, EPI)                   \
   if (dag) {                                           \
     if (pf) GX_DHOP_GO(LS, true, true, ORD, EPI);      \
