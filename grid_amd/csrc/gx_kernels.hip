@@ -645,10 +645,10 @@ template <typename S>
 struct HopEpi {
   typedef typename Sto<S>::C T;
   const cx<S> *phi;
-  const T *mat;   // EPI 1, 5, 6: beta_s; EPI 2: [2][LS][LS], chirality 0 = spins 0,1; EPI 3, 7 with dag:
+  const T *mat;   // EPI 1, 5, 6, 10: beta_s; EPI 2: [2][LS][LS], chirality 0 = spins 0,1; EPI 3, 7, 9 with dag:
                   // A's bands [2][2][LS]
   T alpha;        // EPI 2, 3
-  const T *coef;  // EPI 1, 5, 6: alpha_s; EPI 3, 7, 8: B's bands [2][2][LS]
+  const T *coef;  // EPI 1, 5, 6, 10: alpha_s; EPI 3, 7, 8, 9: B's bands [2][2][LS]
   // k_dhop and hop_tile.  EPI 5 (EPI 1 result) and 8 (EPI 3 result): out, and the per-tile slice sums of
   // |out|^2 in npart [tile][LS]; EPI 6 (EPI 1 result) and 7 (EPI 3 result): rv_s -= acoef[astride s]
   // (result)_s in place of storing out, per-tile slice sums of |rv_s|^2; EPI 10 and 9 (FP64): the same with
