@@ -2342,24 +2342,28 @@ int launch_smat(const Geom &g, const void *in, void *out, const void *mats, cons
 // out = A(in) (+ phi with PHI) with A a two-band fifth-dimension matrix (slice_nbr; bands: [2][2][Ls]).
 // One thread per entry; its neighbour slices' halves are entries of the same or the next cache line that
 // the neighbouring lanes load as their own, so they come from the L1 and the pass moves what it must:
-// out may be phi, not in.
-template <typename S, bool PHI>
+// out may be phi, not in.  I: the index type, 64 bits where a position in the field does not fit 32.
+template <typename S, bool PHI, typename I>
 __global__ void __launch_bounds__(256) k_band(const cx<S> *__restrict__ in, const cx<S> *phi, cx<S> *out,
-                                              const typename Sto<S>::C *__restrict__ bands, uint32_t nent, int dag,
+                                              const typename Sto<S>::C *__restrict__ bands, I nent, int dag,
                                               const Gate *__restrict__ gate, FDiv fLS) {
   typedef typename Sto<S>::C T;
   constexpr int VW = Sto<S>::VW;
   if (gated(gate)) return;
-  const uint32_t e = blockIdx.x * 256 + threadIdx.x, LS = fLS.d;
+  const uint32_t LS = fLS.d;
+  const I e = (I)blockIdx.x * 256 + threadIdx.x;
   if (e >= nent) return;
-  const uint32_t s = e - fdiv(e, fLS) * LS;
+  uint32_t s;
+  if constexpr (sizeof(I) == 4) s = e - fdiv(e, fLS) * LS;
+  else s = (uint32_t)(e % LS);
   cx<T> f[12], v[12];
   load_site<S>(f, in, e);
   T sc[2] = {(T)1, (T)1};
   bool low[2];
 #pragma unroll
   for (int chi = 0; chi < 2; chi++) {
-    const uint32_t sn = slice_nbr(s, chi, dag != 0, LS), n = e - s + sn;
+    const uint32_t sn = slice_nbr(s, chi, dag != 0, LS);
+    const I n = e - s + sn;
     const cx<S> *q = in + bidx<S>(n, 0);
     sc[chi] = site_scale<S>(in, n);
     low[chi] = sn < s;
@@ -2389,15 +2393,26 @@ template <typename S>
 int launch_band(const Geom &g, const void *in, const void *phi, void *out, const void *bands, int dag, const Gate *gate,
                 hipStream_t st) {
   typedef typename Sto<S>::C T;
-  const uint32_t nent = (uint32_t)(g.H4 * g.Ls), nb = (nent + 255) / 256;
+  const int64_t nent = g.half_elems();
+  const uint32_t nb = (uint32_t)((nent + 255) / 256);
   const FDiv f = make_fdiv((uint32_t)g.Ls);
   const cx<S> *pin = (const cx<S> *)in, *pphi = (const cx<S> *)phi;
   cx<S> *pout = (cx<S> *)out;
   const T *pb = (const T *)bands;
-  if (phi)
-    hipLaunchKernelGGL((k_band<S, true>), dim3(nb), dim3(256), 0, st, pin, pphi, pout, pb, nent, dag, gate, f);
-  else
-    hipLaunchKernelGGL((k_band<S, false>), dim3(nb), dim3(256), 0, st, pin, pphi, pout, pb, nent, dag, gate, f);
+  // 32-bit positions up to 2^32 stored complex numbers of a half field (33 GB in FP32); the hop itself ends
+  // below that, these operators do not
+  const bool wide = Sto<S>::NCOL * g.half_pad() >= (int64_t)1 << 32;
+#define GX_BAND(PHI)                                                                                               \
+  if (wide) hipLaunchKernelGGL((k_band<S, PHI, uint64_t>), dim3(nb), dim3(256), 0, st, pin, pphi, pout, pb,         \
+                               (uint64_t)nent, dag, gate, f);                                                      \
+  else hipLaunchKernelGGL((k_band<S, PHI, uint32_t>), dim3(nb), dim3(256), 0, st, pin, pphi, pout, pb,              \
+                          (uint32_t)nent, dag, gate, f)
+  if (phi) {
+    GX_BAND(true);
+  } else {
+    GX_BAND(false);
+  }
+#undef GX_BAND
   GX_CHECK_HIP(hipGetLastError());
   return GX_OK;
 }
