@@ -3350,6 +3350,14 @@ __global__ void __launch_bounds__(kHostEnt) k_host_layout(HostGeom hg, uint32_t 
   cx<S> *half = field + (size_t)cb * Sto<S>::NCOL * hg.g.stride;
   cx<T> v[12];
   if (IMPORT) {
+    // the padding entries (fewer than a block per half) are zero after an import, whatever they held: an earlier
+    // non-finite factor leaves NaN there, which norms would read
+    if (site0 == 0 && blockIdx.x == 0 && t < (uint32_t)kBlk * (hg.full ? 2 : 1)) {
+      const int64_t pe = (int64_t)hg.g.H4 * hg.fLs.d + (t & (kBlk - 1));
+#pragma unroll
+      for (int k = 0; k < 12; k++) v[k] = {0, 0};
+      if (pe < hg.g.stride) store_site<S>(field + (size_t)(t / kBlk) * Sto<S>::NCOL * hg.g.stride, v, pe, false);
+    }
     for (uint32_t i = t; i < 12 * m; i += kHostEnt) sh[i] = row[i];
     __syncthreads();
     if (t >= m) return;
