@@ -165,9 +165,11 @@ struct HostPipe {
 // Eight threads at most: a transfer of n MB takes n of them (below that a thread costs what it saves).
 // Moves `units` units of `unit` bytes between the user's memory and the GPU in pinned chunks, in order.
 // launch(chunk, u0, u1) enqueues the kernel that fills (to_host) or reads the chunk of units u0 .. u1 - 1;
-// copy(chunk, b, e, u0) copies units b .. e - 1 of it from or to the user's memory.  Done on return.
+// copy(chunk, b, e, u0) copies units b .. e - 1 of it from or to the user's memory.  Done on return.  One transfer
+// of a context at a time.
 template <class Launch, class Copy>
 static int host_pipe(Ctx *ctx, int64_t units, size_t unit, bool to_host, Launch launch, Copy copy) {
+  std::lock_guard<std::mutex> lk(ctx->pipe_mu);
   if (!ctx->pipe && !(ctx->pipe = new (std::nothrow) HostPipe())) return GX_ENOMEM;
   HostPipe &hp = *ctx->pipe;
   const size_t bytes = units * unit;

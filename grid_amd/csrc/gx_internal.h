@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -132,6 +133,9 @@ struct Ctx {
   double *red_result = nullptr;      // [kRedSlots]
   double *pinned = nullptr;          // host mirror of red_result
   int next_slot = 0;
+  // Workspaces kept between calls; each call holds the lock while it uses one, so threads that transfer
+  // through one context, or take its block products, queue for it.
+  std::mutex pipe_mu, block_mu;
   HostPipe *pipe = nullptr;          // pinned chunks of host transfers, from the first one on
   BlockWork *block = nullptr;        // created by the first block-algebra call, released with the context
 };

@@ -1075,7 +1075,8 @@ static bool cm_chol(const CMat &m, CMat &L) {
 constexpr int kIpmParts = 2048;  // room for the workgroup partials of the inner-product matrices
 
 // Workspace of the block algebra, kept by its context from the first call on (9 MB; allocating and freeing
-// it in every slice-matrix call took 65 us of each, and the frees synchronised the device).
+// it in every slice-matrix call took 65 us of each, and the frees synchronised the device).  Each product holds
+// the context's lock from its first use of the workspace to its last.
 struct BlockWork {
   static constexpr int kRing = 8;
   Ctx *ctx = nullptr;
@@ -1116,11 +1117,13 @@ struct BlockWork {
   }
   // m(s, t) = <x_s, y_t> (sliceInnerProductMatrix); synchronises the stream
   int ipm(const Geom &g, int nhalf, Field *x, Field *y, CMat &m) {
+    std::lock_guard<std::mutex> lk(ctx->block_mu);
     GX_TRY(launch_slice_ipm(ctx, g, nhalf, x->data, y->data, partial, nparts, mat_dev));
     return read(g.Ls, m);
   }
   // InnerProductMatrix over n fields of nelem stored complex numbers; synchronises the stream
   int ipm_vec(int n, int64_t nelem, const VecPtrs &x, const VecPtrs &y, CMat &m) {
+    std::lock_guard<std::mutex> lk(ctx->block_mu);
     GX_TRY(launch_vec_ipm(ctx, nelem, n, x, y, partial, nparts, mat_dev));
     return read(n, m);
   }
@@ -1146,6 +1149,7 @@ struct BlockWork {
   }
   // MaddMatrix over n fields
   int madd_vec(int n, int64_t nelem, const VecPtrs &r, const CMat &a, const VecPtrs &x, const VecPtrs &y, double scale) {
+    std::lock_guard<std::mutex> lk(ctx->block_mu);
     double2 *d;
     GX_TRY(coefficients(a, &d));
     GX_TRY(launch_vec_madd(ctx, nelem, n, d, scale, x, y, r));
@@ -1153,6 +1157,7 @@ struct BlockWork {
   }
   // r_t = y_t + scale sum_s x_s a(s, t) (sliceMaddMatrix; y = null: sliceMulMatrix)
   int madd(const Geom &g, int nhalf, Field *r, const CMat &a, Field *x, Field *y, double scale) {
+    std::lock_guard<std::mutex> lk(ctx->block_mu);
     double2 *d;
     GX_TRY(coefficients(a, &d));
     GX_TRY(launch_slice_madd(ctx, g, nhalf, d, scale, x->data, y ? y->data : nullptr, r->data));
@@ -1162,6 +1167,7 @@ struct BlockWork {
 };
 
 static int block_work(Ctx *ctx, BlockWork **out) {
+  std::lock_guard<std::mutex> lk(ctx->block_mu);
   if (!ctx->block) {
     BlockWork *w = new BlockWork();
     const int rc = w->init(ctx);
