@@ -1939,6 +1939,8 @@ int gx_slice_inner_product_matrix_noalloc(gx_field lhs, gx_field rhs, double *ma
   return GX_OK;
 }
 
+// The updates run on the stream of X's context.  Fields of other contexts, whose streams do not wait for it, are done
+// with on return.
 int gx_slice_madd_matrix(gx_field R, const double *aa, gx_field X, gx_field Y, double scale) {
   if (!slice_conformable(R, X) || (Y && !slice_conformable(R, Y)) || !aa) {
     set_error("slice_madd_matrix: needs F64 fields of one lattice and subset");
@@ -1949,7 +1951,9 @@ int gx_slice_madd_matrix(gx_field R, const double *aa, gx_field X, gx_field Y, d
   for (int i = 0; i < n * n; i++) a.a[i] = cd(aa[2 * i], aa[2 * i + 1]);
   BlockWork *bw;
   GX_TRY(block_work(X->ctx, &bw));
-  return bw->madd(X->g, X->subset == GX_FULL ? 2 : 1, R, a, X, Y, scale);
+  GX_TRY(bw->madd(X->g, X->subset == GX_FULL ? 2 : 1, R, a, X, Y, scale));
+  if (R->ctx != X->ctx || (Y && Y->ctx != X->ctx)) GX_CHECK_HIP(hipStreamSynchronize(X->ctx->stream));
+  return GX_OK;
 }
 
 // n fields of one lattice, subset and precision (F64) as a pointer list; false if they are not
@@ -2000,7 +2004,12 @@ int gx_madd_matrix(int n, gx_field *R, const double *aa, gx_field *X, gx_field *
   BlockWork *bw;
   GX_TRY(block_work(fx->ctx, &bw));
   GX_TRY(bw->madd_vec(n, fx->stored(), pr, a, px, py, scale));
-  for (int b = 0; b < n; b++) R[b]->cb = X[b]->cb;
+  bool other = false;
+  for (int b = 0; b < n; b++) {
+    R[b]->cb = X[b]->cb;
+    other = other || X[b]->ctx != fx->ctx || R[b]->ctx != fx->ctx || (Y && Y[b]->ctx != fx->ctx);
+  }
+  if (other) GX_CHECK_HIP(hipStreamSynchronize(fx->ctx->stream));
   return GX_OK;
 }
 

@@ -1,5 +1,5 @@
 """Host threads that share one context: its pinned chunks and block workspace serve one call at a time, so transfers, force
-matrices and block products that run side by side each get their own data."""
+matrices and block products that run side by side each get their own data.  And block updates into fields of another context, which are complete on return."""
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -52,3 +52,24 @@ def test_block_products():
 
     each(4, work)
     ctx.close()
+
+
+def test_updates_across_contexts():
+    dims, n = (16, 16, 16, 16), 6
+    one, two = gx.Context(0), gx.Context(0)
+    a = gx.gaussian_fermion(dims, n, 120)
+    x, y = gx.Field(one, dims, n).upload(a), gx.Field(two, dims, n).upload(a)
+    r, z = gx.Field(two, dims, n), gx.Field(two, dims, n)
+    c = np.eye(n)
+    # slices as lists of fields of both contexts
+    xs, rs = ([gx.Field(k, dims, 1).upload(np.ascontiguousarray(a[:, :, :, :, s:s + 1])) for s in range(n)] for k in (one, two))
+    for k in range(1, 20):
+        gx.slice_madd_matrix(r, k * c, x, y, 1.0)
+        gx.axpby(z, 1.0, 0.0, r, r)  # on the other context's stream
+        gx.madd_matrix(rs, c, xs, rs, 1.0)
+        gx.axpby(rs[0], 0.5, 0.5, rs[0], rs[0])
+    # small whole factors and halves: exact sums up to the rounding of one product each
+    assert np.abs(z.download() - 20 * a).max() < 1e-13 * 20 * np.abs(a).max()
+    for s in range(n):
+        assert np.abs(rs[s].download()[..., 0, :, :] - 20 * a[..., s, :, :]).max() < 1e-13 * 20 * np.abs(a).max()
+    one.close(), two.close()
