@@ -792,7 +792,18 @@ int op_band(Op *op, int prec, int which, const void **bands) {
 }
 
 // ---------------- operator building blocks (half fields) ----------------
+// A Cayley operator runs on the extents whose dense matrices have a kernel, whatever the size of its lattice.  hop: the
+// call is a hop alone, which the row tiles also take for others.
+static int extent_check(const Op *op, int prec, bool hop = false) {
+  const int Ls = op->g.Ls;
+  if (op->kind == GX_WILSON || Ls <= kMaxLs || general_extent(Ls) || (hop && tune_get(GX_TUNE_DHOP_TILE, prec)))
+    return GX_OK;
+  set_error("mobius: Ls=%d: Ls > %d needs an odd part of at most 7", Ls, kMaxLs);
+  return GX_EINVAL;
+}
+
 int apply_dhop_half(Op *op, Field *in, Field *out, int cb_out, int dag, const Gate *gate) {
+  GX_TRY(extent_check(op, in->prec, true));
   void *Ue, *Uo;
   GX_TRY(op_gauge(op, in->prec, &Ue, &Uo));
   void *U = cb_out == 0 ? Ue : Uo;
@@ -804,6 +815,7 @@ int apply_dhop_half(Op *op, Field *in, Field *out, int cb_out, int dag, const Ga
 
 // out = A(in) (+ phi): the two-band operators through launch_band (phi: these only), the others dense
 static int apply_smat(Op *op, Field *in, Field *phi, Field *out, int which, const Gate *gate) {
+  GX_TRY(extent_check(op, in->prec));
   const void *m;
   const bool dense = which == Op::S_MOOEEINV || which == Op::S_MOOEEINVDAG;
   GX_TRY(dense ? op_smat(op, in->prec, which, &m) : op_band(op, in->prec, which, &m));
@@ -859,6 +871,7 @@ int apply_mooee(Op *op, Field *in, Field *out, int which, const Gate *gate) {
 template <typename T>
 static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, const HopFuse *fz, const void *first) {
   const int prec = in->prec, cb_in = in->cb, cb_mid = 1 - cb_in;
+  GX_TRY(extent_check(op, prec));
   void *Ue, *Uo;
   GX_TRY(op_gauge(op, prec, &Ue, &Uo));
   void *U_mid = cb_mid == 0 ? Ue : Uo, *U_in = cb_in == 0 ? Ue : Uo;
@@ -901,6 +914,7 @@ static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, c
 template <typename T>
 static int full_m_fused(Op *op, Field *in, Field *out, int dag) {
   const int prec = in->prec;
+  GX_TRY(extent_check(op, prec));
   void *U[2];
   GX_TRY(op_gauge(op, prec, &U[0], &U[1]));
   hipStream_t st = op->ctx->stream;
@@ -1582,6 +1596,7 @@ int gx_MooeeInvDag(gx_op op, gx_field in, gx_field out) {
 }
 int gx_Dhop(gx_op op, gx_field in, gx_field out, int dag) {
   GX_TRY(check_io(O(op), F(in), F(out), true));
+  GX_TRY(extent_check(O(op), in->prec, true));
   void *U[2];
   GX_TRY(op_gauge(O(op), in->prec, &U[0], &U[1]));
   const int split = by_prec(in->prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g); });

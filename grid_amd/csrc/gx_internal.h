@@ -64,6 +64,13 @@ int tune_version();
   } while (0)
 
 constexpr int kMaxLs = 16;         // largest extent of the templated kernels and of the block solvers' blocks
+// extents whose whole sites fill the general kernels' tiles of at most 8 waves: an odd part of at most 7.  Past kMaxLs
+// the others (up to 64) run the leg-per-wave hop on lattices of every size, and have no kernel for dense
+// fifth-dimension matrices: Cayley operators refuse them.
+inline bool general_extent(int Ls) {
+  while (Ls % 2 == 0) Ls /= 2;
+  return Ls <= 7;
+}
 constexpr int kMaxFifth = 128;     // largest fifth-dimension extent (Ls, or right-hand sides x Ls)
 constexpr int kMaxRhs = 64;        // right-hand sides of one multi-RHS solve
 constexpr int kRedBlocks = 1024;   // fixed grid of the deterministic reductions

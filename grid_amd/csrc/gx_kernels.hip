@@ -1962,11 +1962,12 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
     set_error("dhop: epilogue operand missing");
     return GX_EINVAL;
   }
-  if (lb == g.Ls && hop_split<S>(g)) {
+  auto split = [&]() -> int {
     const void *pi[2] = {in, nullptr}, *pu[2] = {U, nullptr}, *pp[2] = {phi, nullptr};
     void *po[2] = {out, nullptr};
     return launch_hop_split<S>(g, cb_out, 1, pi, po, pu, pp, dag, gate, st, epi, mat, alpha, coef, fz);
-  }
+  };
+  if (lb == g.Ls && hop_split<S>(g)) return split();
   const int kepi = epi;
   // The blocked sweep (map 4, the default) keeps the t-neighbours' rows in the XCD's L2 between slices:
   // FP64 16^4 x 16 53.6 us against 68.7 as plain slabs (map 1), FP32 32^3x64 x 12 893 against 1080, and
@@ -2116,8 +2117,9 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
     }
   }
   const int W = general_waves(g.Ls, tune_get(GX_TUNE_DHOP_SHAPE, prec_of<S>()), sizeof(cx<T>), kepi >= 2, lb);
+  if (W < 0 && lb == g.Ls && g.Ls <= 64 && !general_extent(g.Ls)) return split();  // no other kernel has this extent
   if (W < 0 || g.Ls % lb != 0) {
-    set_error("dhop: no tile shape for Ls=%d (matrix group %d): Ls > 16 needs an odd part of at most 7", g.Ls, lb);
+    set_error("dhop: no tile shape for Ls=%d (matrix group %d): Ls > 64 needs an odd part of at most 7", g.Ls, lb);
     return GX_EINVAL;
   }
   if (W > 0) {

@@ -100,7 +100,10 @@ int gx_inner_product_norm(gx_field x, gx_field y, double *re, double *im, double
  * pairs (NULL = periodic; Grid WilsonImplParams::boundary_phases, ActionParams.h:49-65).
  * For GX_WILSON, Ls > 1 gives Ls independent copies of the 4D operator sharing the gauge
  * links: the multi-right-hand-side operator (Grid: WilsonFermion5D with Ls = Nrhs,
- * WilsonFermion5D.h:40-65). ---- */
+ * WilsonFermion5D.h:40-65).
+ * Ls <= 128.  Wilson operators apply with every Ls up to 64 and Mobius operators with every Ls up to 16; past that
+ * the odd part of Ls is at most 7 (24, 48, 96, ...), and the applications of others return GX_EINVAL.  Neither depends
+ * on the lattice. ---- */
 int gx_wilson_create(gx_ctx ctx, const int dims[4], int Ls, double mass, const double *U,
                      const double *phases, gx_op *out);
 int gx_mobius_create(gx_ctx ctx, const int dims[4], int Ls, double mass, double M5, double b, double c,
@@ -404,7 +407,9 @@ enum gx_tune_knob {
                                products on the matrix cores (v_mfma_f32_16x16x4f32) */
   GX_TUNE_DHOP_TILE = 9,    /* 1: hops in tiles of 2 x 2 rows of x staged in LDS (x, y and z legs from the tile;
                                when 4 Lx/2 Ls threads and the tile fit a workgroup) */
-  GX_TUNE_DHOP_SPLIT = 10,  /* 1 (default): hops of small lattices run one leg per wave (with SHAPE, MFMA and TILE at 0) */
+  GX_TUNE_DHOP_SPLIT = 10,  /* 1 (default): hops of small lattices run one leg per wave (with SHAPE, MFMA and TILE at 0),
+                               whatever MAP, PF, NT, ORDER and PERSIST say; 0: only the Ls of 17 .. 64 that have no
+                               other tile do, on lattices of every size */
   GX_TUNE_COUNT = 12
 };
 int gx_tune_set(int knob, int value);   /* every precision's value */
