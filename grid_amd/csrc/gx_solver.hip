@@ -1559,9 +1559,13 @@ static int multishift_run(Op *op, Field *src, int nshift, const double *mass, co
     npart = ctx->red_partial;
   constexpr int kMsNorm = 4;  // result slot
   // Each iteration leaves its residual in a new field of a ring, and the shifts' vectors are updated for a
-  // ring's worth of iterations at once (k_ms_group); where there is no room for kMsGroup fields, for fewer.
+  // ring's worth of iterations at once (k_ms_group).  The ring takes at most a quarter of the memory that is free, as the
+  // device's other users allocate too; where that does not hold kMsGroup fields, iterations are grouped by fewer.
   std::vector<void *> rr{r->data};
-  while ((int)rr.size() < kMsGroup && (int)rr.size() < maxit) {
+  size_t mem_free = 0, mem_total = 0;
+  GX_CHECK_HIP(hipMemGetInfo(&mem_free, &mem_total));
+  const int64_t room = (int64_t)(mem_free / 4 / r->bytes);
+  while ((int)rr.size() < kMsGroup && (int)rr.size() < maxit && (int64_t)rr.size() <= room) {
     Field *f = nullptr;
     if (field_create(op->ctx, op->g, GX_F64, GX_EVEN, &f) != GX_OK) {
       (void)hipGetLastError();
