@@ -16,9 +16,10 @@ precision prec only, so the FP64 and inner-precision operators of a mixed solve 
 The hop knobs are chosen by timing DhopEO on the caller's own lattice, Ls and precision (HIP
 events over repeated launches, best of several rounds), by coordinate search: map, prefetch,
 stores and leg order in the default tile shape, then the tile shape (W-wave shapes with and
-without the persistent grid, and the LDS row tiles), then the map again in the chosen shape.  For
-FP32 and FP16 storage, whose CG folds its reductions into hop epilogues, a persistent winner and
-the fastest hop of the other prefetch setting are then compared by CG iteration time.  The
+without the persistent grid, and the LDS row tiles), then the map again in the chosen shape.  Lattices whose
+default hop is the leg-per-wave one keep the default map, prefetch, stores and order, which it ignores.  A winner
+other than the default form, and for FP32 and FP16 storage the fastest hop of the other prefetch setting, are
+then compared by CG iteration time, as the CG takes its reductions in hop epilogues that not every form has.  The
 solver knobs are chosen by timing a fixed number of CG iterations.  Results are cached in a JSON file keyed
 by device and workload, so a later
 process applies them without measuring.  No Grid counterpart: Grid fixes its launch shape when it
@@ -33,9 +34,12 @@ import time
 import numpy as np
 
 from . import (EVEN, F16, F32, F64, ODD, TUNE_CG_GRAPH, TUNE_DHOP_MAP, TUNE_DHOP_NT, TUNE_DHOP_ORDER,
-               TUNE_DHOP_PERSIST, TUNE_DHOP_PF, TUNE_DHOP_SHAPE, TUNE_DHOP_TILE, TUNE_FUSED, tune_get, tune_set)
+               TUNE_DHOP_PERSIST, TUNE_DHOP_PF, TUNE_DHOP_SHAPE, TUNE_DHOP_SPLIT, TUNE_DHOP_TILE, TUNE_FUSED, tune_get,
+               tune_set)
 
 HOP_KNOBS = (TUNE_DHOP_MAP, TUNE_DHOP_PF, TUNE_DHOP_NT, TUNE_DHOP_ORDER)
+HOP_DEFAULTS = tuple(zip(HOP_KNOBS, (4, 1, 1, 0)))
+SPLIT_ENTRIES = 40960   # the library's kSplitMax: entries per checkerboard up to which a hop runs one leg per wave
 SOLVER_KNOBS = (TUNE_FUSED, TUNE_CG_GRAPH)
 KNOB_NAMES = {TUNE_DHOP_MAP: 'dhop_map', TUNE_DHOP_PF: 'dhop_pf', TUNE_DHOP_NT: 'dhop_nt',
               TUNE_DHOP_ORDER: 'dhop_order', TUNE_FUSED: 'fused', TUNE_CG_GRAPH: 'cg_graph',
@@ -182,9 +186,13 @@ class Autotuner:
             with Knobs(c, prec):
                 return self._time_dhop(D, fi, fo, dhop_iters)
 
-        shapes = shape_candidates(D.Ls, prec)
+        shapes = shape_candidates(D.Ls, prec) or [0]   # none: the leg-per-wave hop whatever the knobs say
         default_shape = ((TUNE_DHOP_SHAPE, shapes[0]), (TUNE_DHOP_PERSIST, 0), (TUNE_DHOP_TILE, 0))
-        first, hop_times = search([c + default_shape for c in hop_candidates(D.Ls)], hop, rounds)
+        # with every form at its default, the leg-per-wave hop of small lattices takes no notice of map, prefetch,
+        # stores and order: their defaults stay
+        split = D.Ls <= 64 and math.prod(D.dims) // 2 * D.Ls <= SPLIT_ENTRIES and tune_get(TUNE_DHOP_SPLIT, prec)
+        hops = [HOP_DEFAULTS] if split else hop_candidates(D.Ls)
+        first, hop_times = search([c + default_shape for c in hops], hop, rounds)
         others = tuple(kv for kv in first if kv[0] not in LAUNCH_KNOBS)
         launch = launch_candidates(shapes)
         if len(launch) > 1:
@@ -194,8 +202,11 @@ class Autotuner:
             hop_times.update(t2)
             chosen = tuple(kv for kv in best_shape if kv[0] in LAUNCH_KNOBS)
             rest = tuple(kv for kv in others if kv[0] != TUNE_DHOP_MAP)
-            hop_best, t3 = search([((TUNE_DHOP_MAP, m),) + rest + chosen for m in range(5)], hop, rounds)
-            hop_times.update(t3)
+            if split and chosen == launch[0]:
+                hop_best = others + chosen
+            else:
+                hop_best, t3 = search([((TUNE_DHOP_MAP, m),) + rest + chosen for m in range(5)], hop, rounds)
+                hop_times.update(t3)
         else:
             hop_best = first
         fs, fx = D.field(prec, ODD).upload(psi), D.field(prec, ODD)
@@ -204,20 +215,28 @@ class Autotuner:
             with Knobs(hop_best + c, prec):
                 return self._time_cg(D, fs, fx, cg_iters)
 
-        # FP32 / FP16 CG folds its reductions into hop epilogues that only the one-workgroup-per-tile
-        # launches have: when the fastest hop is a persistent grid, keep it only if a CG iteration
-        # under it beats one under the fastest non-persistent launch.  The epilogue kernels also
-        # use registers differently from the plain hop (the FP16 ones fit fewer waves without
-        # prefetch), so the fastest hop of the other prefetch setting is compared by CG time too.
+        # The CG takes its reductions in hop epilogues that only the one-workgroup-per-tile launches have (not the
+        # persistent grid and the row tiles), and on small and medium lattices runs its finalisers inside the
+        # default form's kernels alone.  So a fastest hop in another form is compared with the fastest hop that has
+        # the epilogues, and with the fastest one of the default form, by CG iteration time; a W-wave form gives way
+        # to the default one for more than 2%.
         def cg_hop(h):
             with Knobs(h, prec):
                 return self._time_cg(D, fs, fx, cg_iters)
 
-        if prec != F64 and dict(hop_best).get(TUNE_DHOP_PERSIST, 0):
-            plain = [c for c in hop_times if not dict(c).get(TUNE_DHOP_PERSIST, 0)]
-            if plain:
-                alt = min(plain, key=lambda c: hop_times[c])
-                hop_best, t4 = search([hop_best, alt], cg_hop, rounds)
+        def fastest(cond):
+            return min((c for c in hop_times if cond(dict(c))), key=lambda c: hop_times[c])
+
+        def plain(d):
+            return not d.get(TUNE_DHOP_PERSIST, 0) and not d.get(TUNE_DHOP_TILE, 0)
+
+        if not plain(dict(hop_best)):
+            hop_best, _ = search([hop_best, fastest(plain)], cg_hop, rounds)
+        if dict(hop_best)[TUNE_DHOP_SHAPE] != shapes[0]:
+            alt = fastest(lambda d: plain(d) and d[TUNE_DHOP_SHAPE] == shapes[0])
+            hop_best, _ = search([hop_best, alt], cg_hop, rounds, margin=0.02)
+        # The epilogue kernels also use registers differently from the plain hop, so the fastest FP32 or FP16 hop
+        # of the other prefetch setting is compared by CG time too.
         if prec != F64:
             pf = dict(hop_best).get(TUNE_DHOP_PF, 0)
             other = [c for c in hop_times
