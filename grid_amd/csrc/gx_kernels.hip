@@ -2768,6 +2768,20 @@ __device__ __forceinline__ void cg_advance(CGState &st, double cp) {
   }
 }
 
+// all of the next state but a and d, which the hop left there and other workgroups may be reading
+__device__ __forceinline__ void cg_store(CGState *nxt, const CGState &st) {
+  *static_cast<Gate *>(nxt) = st;
+  nxt->c = st.c;
+  nxt->cp = st.cp;
+  nxt->b = st.b;
+  nxt->rsq = st.rsq;
+  nxt->delta = st.delta;
+  nxt->maxres = st.maxres;
+  nxt->cprev = st.cprev;
+  nxt->fbtol = st.fbtol;
+  nxt->ru = st.ru;
+}
+
 // which = 0: d = sum, a = c / d.   which = 1: cp = sum, b = cp / c, c = cp, convergence test.
 // The which = 1 finaliser advances k in every iteration, also once the solve has stopped, so the
 // gate of the following solution update (k-1) closes after the last real iteration.
@@ -2885,7 +2899,7 @@ __global__ void __launch_bounds__(256) k_cg_update_fin(int64_t nsites, int64_t s
   const bool keep_p = st.ru == 1;
   if (first) {
     st.k++;
-    *nxt = st;
+    cg_store(nxt, st);
   }
   cg_update<S>(nsites, stride, psi, p, r, a, b, keep_p);
 }
@@ -2930,7 +2944,7 @@ __global__ void __launch_bounds__(256) k_cg_update_band(uint32_t H4, cx<S> *__re
   const bool keep_p = st.ru == 1;  // the host forms the new p (and its q)
   if (first) {
     st.k++;
-    *nxt = st;
+    cg_store(nxt, st);
   }
   if (on) {
 #pragma unroll
