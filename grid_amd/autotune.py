@@ -39,7 +39,7 @@ from . import (EVEN, F16, F32, F64, ODD, TUNE_CG_GRAPH, TUNE_DHOP_MAP, TUNE_DHOP
 
 HOP_KNOBS = (TUNE_DHOP_MAP, TUNE_DHOP_PF, TUNE_DHOP_NT, TUNE_DHOP_ORDER)
 HOP_DEFAULTS = tuple(zip(HOP_KNOBS, (4, 1, 1, 0)))
-SPLIT_ENTRIES = 40960   # the library's kSplitMax: entries per checkerboard up to which a hop runs one leg per wave
+SPLIT_ENTRIES = 40960   # the library's kSplitMax: entries per checkerboard up to which a hop may run one leg per wave
 SOLVER_KNOBS = (TUNE_FUSED, TUNE_CG_GRAPH)
 KNOB_NAMES = {TUNE_DHOP_MAP: 'dhop_map', TUNE_DHOP_PF: 'dhop_pf', TUNE_DHOP_NT: 'dhop_nt',
               TUNE_DHOP_ORDER: 'dhop_order', TUNE_FUSED: 'fused', TUNE_CG_GRAPH: 'cg_graph',
@@ -73,6 +73,16 @@ def hop_candidates(Ls):
     """Hop knob settings to try, each a tuple of (knob, value) pairs."""
     orders = (0, 1) if Ls in (1, 12, 16) else (0,)
     return [tuple(zip(HOP_KNOBS, v)) for v in itertools.product((0, 1, 2, 3, 4), (0, 1), (0, 1), orders)]
+
+
+def leg_per_wave(dims, Ls, prec):
+    """Whether DhopEO runs one leg per wave in the library's default form (its hop_split for a bare hop)."""
+    half = math.prod(dims) // 2
+    if not tune_get(TUNE_DHOP_SPLIT, prec) or Ls > 64 or half * Ls > SPLIT_ENTRIES:
+        return False
+    if Ls < 8 or prec == F16 or (prec == F32 and Ls > 16):
+        return True
+    return -(-half // (64 // Ls)) <= (512 if prec == F32 else 768 if Ls > 16 else 448 if 64 % Ls else 512)
 
 
 def shape_candidates(Ls, prec=F64):
@@ -190,7 +200,7 @@ class Autotuner:
         default_shape = ((TUNE_DHOP_SHAPE, shapes[0]), (TUNE_DHOP_PERSIST, 0), (TUNE_DHOP_TILE, 0))
         # with every form at its default, the leg-per-wave hop of small lattices takes no notice of map, prefetch,
         # stores and order: their defaults stay
-        split = D.Ls <= 64 and math.prod(D.dims) // 2 * D.Ls <= SPLIT_ENTRIES and tune_get(TUNE_DHOP_SPLIT, prec)
+        split = leg_per_wave(D.dims, D.Ls, prec)
         hops = [HOP_DEFAULTS] if split else hop_candidates(D.Ls)
         first, hop_times = search([c + default_shape for c in hops], hop, rounds)
         others = tuple(kv for kv in first if kv[0] not in LAUNCH_KNOBS)

@@ -928,7 +928,7 @@ static int full_m_fused(Op *op, Field *in, Field *out, int dag) {
     GX_TRY(op_band(op, prec, dag ? Op::S_MOOEEDAG : Op::S_MOOEE, &b_mooee));
     if (!dag && !(t = op_tmp(op, prec, 3))) return GX_ENOMEM;
   }
-  if (hop_split<T>(g)) {  // both checkerboards in one launch
+  if (hop_split<T>(g, op->kind == GX_WILSON ? 1 : 3, 2)) {  // both checkerboards in one launch
     const void *src[2] = {in->half(1), in->half(0)}, *same[2] = {in->half(0), in->half(1)}, *pu[2] = {U[0], U[1]};
     void *po[2] = {out->half(0), out->half(1)};
     if (t) {
@@ -1599,7 +1599,7 @@ int gx_Dhop(gx_op op, gx_field in, gx_field out, int dag) {
   GX_TRY(extent_check(O(op), in->prec, true));
   void *U[2];
   GX_TRY(op_gauge(O(op), in->prec, &U[0], &U[1]));
-  const int split = by_prec(in->prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g); });
+  const int split = by_prec(in->prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g, 0, 2); });
   if (split) {  // both checkerboards in one launch
     const void *src[2] = {in->half(1), in->half(0)}, *pu[2] = {U[0], U[1]};
     void *po[2] = {out->half(0), out->half(1)};

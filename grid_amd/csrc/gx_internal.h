@@ -277,10 +277,10 @@ struct HopFuse {
 // itself; ncb = 2 does both checkerboards cb and cb ^ 1 in one launch (operand j of each list).
 // Up to 32768 entries (H4 Ls) it is the faster in every precision (FP64 8^4: 8.6 -> 4.3 us, 8^4 x 8: 7.2 ->
 // 4.6, 8^4 x 16: 7.7 -> 6.5, 16^4: 13.6 -> 12.1); at 65536 the LDS round trip costs more than the latency it
-// hides (8^3 x 16 x 16: 9.5 -> 11.9).
+// hides (8^3 x 16 x 16: 9.5 -> 11.9), and from one round of workgroups on that depends (hop_split).
 constexpr int64_t kSplitMax = 40960;
 template <typename S>
-bool hop_split(const Geom &g);
+bool hop_split(const Geom &g, int epi, int ncb);
 template <typename S>
 int launch_hop_split(const Geom &g, int cb, int ncb, const void *const in[2], void *const out[2], const void *const U[2],
                      const void *const phi[2], int dag, const Gate *gate, hipStream_t st, int epi, const void *mat,

@@ -1865,12 +1865,30 @@ static GShape make_shape(int LS, int LB, int W) {
   M(1) M(2) M(3) M(4) M(5) M(6) M(7) M(8) M(9) M(10) M(11) M(12) M(13) M(14) M(15) M(16)
 #endif
 
-// The leg-per-wave kernel's range: up to kSplitMax entries per checkerboard
+// The leg-per-wave kernel's range: kSplitMax entries per checkerboard, and for a single checkerboard mostly one round of
+// resident workgroups, two per CU: a second, partly filled round costs more than the latency that is hidden.  One
+// checkerboard against the 4-wave kernel, FP64: 8^3x16 x 16 rows of 512 tiles 0.88, of 576 and 640 tiles (8^3x18,
+// 8^3x20 x 8) 1.1; 8^3x12 x 12 (615 tiles, 60 of 64 lanes) hop 11.0 us for 7.5, MpcDagMpc 50 for 36, CG iteration 65 for
+// 50, and at 512 tiles 8.9 for 7.3, at 432 6.3 for 7.1.  Fewer slices than 8 in FP64 are bound by the links and gain up to
+// kSplitMax (0.8-0.95); one or two slices in every precision (0.9-1.0).  FP32 and FP16 from 3 slices on are at 1.0-1.15 past
+// 512 tiles, but a bare hop (epi 0), whose registers let a third workgroup in, stays at 0.9 in FP16 and 0.95-1.0 in FP32
+// with fewer than 8, and the matrix epilogues (epi 2, 3) of full waves at 0.92.  Past 16 slices the other form is the
+// general tile, whose CG has no folded finalisers: FP64 with 24 slices (three workgroups of 48 KB of LDS per CU) 1.0 at
+// 768 tiles and 1.2 at 851, with matrix epilogues 1.02 and the CG 0.94; FP32 and FP16 0.75-0.95.  Both checkerboards in one
+// launch save the second launch: M of these sizes takes 0.7-0.95 of the time, but for Wilson FP64 with 10 or 12 slices (1.2).
 template <typename S>
-bool hop_split(const Geom &g) {
-  const int p = prec_of<S>();
-  return tune_get(GX_TUNE_DHOP_SPLIT, p) && !tune_get(GX_TUNE_DHOP_SHAPE, p) && !tune_get(GX_TUNE_DHOP_MFMA, p) &&
-         !tune_get(GX_TUNE_DHOP_TILE, p) && g.Ls <= 64 && g.H4 * g.Ls <= kSplitMax;
+bool hop_split(const Geom &g, int epi, int ncb) {
+  const int p = prec_of<S>(), Ls = g.Ls;
+  if (!tune_get(GX_TUNE_DHOP_SPLIT, p) || tune_get(GX_TUNE_DHOP_SHAPE, p) || tune_get(GX_TUNE_DHOP_MFMA, p) ||
+      tune_get(GX_TUNE_DHOP_TILE, p) || Ls > 64 || g.H4 * Ls > kSplitMax)
+    return false;
+  if (ncb == 2) return true;
+  const int spw = 64 / Ls;
+  const int64_t tiles = (g.H4 + spw - 1) / spw;
+  if (Ls > kMaxLs) return p != GX_F64 || epi >= 2 || tiles <= 768;
+  if (p == GX_F64) return Ls < 8 || tiles <= (64 % Ls != 0 ? 448 : 512);
+  if (epi == 0 && (p == GX_F16 || Ls < 8)) return true;
+  return Ls <= 2 || tiles <= 512 || (epi >= 2 && 64 % Ls == 0);
 }
 
 template <typename S>
@@ -1967,7 +1985,7 @@ int launch_dhop_epi(const Geom &g, const void *in, void *out, const void *U, int
     void *po[2] = {out, nullptr};
     return launch_hop_split<S>(g, cb_out, 1, pi, po, pu, pp, dag, gate, st, epi, mat, alpha, coef, fz);
   };
-  if (lb == g.Ls && hop_split<S>(g)) return split();
+  if (lb == g.Ls && hop_split<S>(g, epi, 1)) return split();
   const int kepi = epi;
   // The blocked sweep (map 4, the default) keeps the t-neighbours' rows in the XCD's L2 between slices:
   // FP64 16^4 x 16 53.6 us against 68.7 as plain slabs (map 1), FP32 32^3x64 x 12 893 against 1080, and
@@ -4362,7 +4380,7 @@ int launch_digest_slices(Ctx *ctx, const Geom &g, const void *full, int s0, int 
                                   hipStream_t, int, const void *, const void *, double, int, const void *,         \
                                   const HopFuse *);                                                                \
   template int launch_host_layout<S>(const Geom &, int, int, int64_t, int64_t, void *, void *, hipStream_t);       \
-  template bool hop_split<S>(const Geom &);                                                                        \
+  template bool hop_split<S>(const Geom &, int, int);                                                              \
   template int launch_hop_split<S>(const Geom &, int, int, const void *const[2], void *const[2],                   \
                                    const void *const[2], const void *const[2], int, const Gate *, hipStream_t,    \
                                    int, const void *, double, const void *, const HopFuse *);                      \

@@ -244,7 +244,8 @@ static int cg_iteration_fold(Op *op, Field *psi, Field *p, Field *mmp, Field *r,
 // launch form but the persistent, row-tile and matrix-core ones)
 static bool cg_folds(const Op *op, int prec) {
   if (!tune_get(GX_TUNE_FUSED, prec)) return false;
-  if (by_prec(prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g); })) return true;
+  const int epi = op->kind == GX_WILSON ? 1 : 3;
+  if (by_prec(prec, [&](auto t) -> int { return hop_split<decltype(t)>(op->g, epi, 1); })) return true;
   const int Ls = op->g.Ls;
   if (Ls > kMaxLs || tune_get(GX_TUNE_DHOP_SHAPE, prec) || tune_get(GX_TUNE_DHOP_MFMA, prec) ||
       tune_get(GX_TUNE_DHOP_TILE, prec))

@@ -75,6 +75,15 @@ def test_small_lattices_keep_ignored_knobs(prec):
     assert (got['dhop_map'], got['dhop_pf'], got['dhop_nt'], got['dhop_order'], got['dhop_shape']) == (4, 1, 1, 0, 0)
 
 
+def test_leg_per_wave_range():
+    ask = at.leg_per_wave
+    assert all(ask((8, 8, 8, 8), 16, p) for p in at.PRECS)            # 512 workgroups
+    assert [ask((8, 8, 8, 9), 16, p) for p in at.PRECS] == [False, False, True]
+    assert [ask((8, 8, 8, 10), 12, p) for p in at.PRECS] == [False, True, True]   # 512 of 60 lanes
+    assert all(ask((16, 16, 16, 20), 1, p) for p in at.PRECS) and not any(ask((16, 16, 16, 22), 1, p) for p in at.PRECS)
+    assert not any(ask((2, 2, 2, 2), 128, p) for p in at.PRECS)
+
+
 def test_extent_without_tiles():
     got = tuned(SMALL, 33, gx.F64, lambda k: 1.0, lambda k: 1.0)
     assert got['dhop_shape'] == 0 and got['dhop_tile'] == 0
