@@ -909,8 +909,9 @@ static int mpc_fused(Op *op, Field *in, Field *out, int dag, const Gate *gate, c
 //   Wilson  M    = Dhop in + d in                              3 field passes per checkerboard
 //   Cayley  M    = Dhop(Meooe5D in) + Mooee in                 5 (Meooe5D in its own kernel)
 //           Mdag = MeooeDag5D Dhop^dag in + MooeeDag in        3
-// Mdag in FP64 on 24^4 x 12: 842 us, 1653 us as four kernels and 9 passes per checkerboard (the floor, one
-// read and one write of the field and the links, is 306 us at 6.25 TB/s; the hops' neighbours bound it).
+// Mdag in FP64 on 24^4 x 12: 662 us, 1653 us as four kernels and 9 passes per checkerboard (the floor, one
+// read and one write of the field and the links, is 306 us at 6.25 TB/s; as each launch reads one half of in as
+// neighbours and the other as phi, in is read twice: 1.34 GB a launch, of which 1.5 are moved).
 template <typename T>
 static int full_m_fused(Op *op, Field *in, Field *out, int dag) {
   const int prec = in->prec;

@@ -3463,8 +3463,8 @@ static __global__ void __launch_bounds__(256) k_hop_leg(KGeom g, FDiv fLS, int c
 // in mask (the others' places are left alone).  The projector acts on A as well and the link factors out of the
 // sum: mat = Uds[mu] sum_s sum_j (P B)_j (x) (P A)_j^dag over the two projected spins, half the products and one
 // link multiplication per site and direction.  One wave takes 64 / LP whole sites, LP = min(Ls, 64) lanes each;
-// A is read once for the four directions, the lanes' matrices are added in LDS, and the result goes to pinned
-// host memory in the user's order: 16^3 x 32 x 8, both checkerboards, 1.9 ms of kernels (one thread per site,
+// the four forward directions follow one another in it (A is loaded for each, after the first from the caches), the
+// lanes' matrices are added in LDS, and the result goes to pinned host memory in the user's order: 16^3 x 32 x 8, both checkerboards, 1.9 ms of kernels (one thread per site,
 // every slice after another, a launch per direction) and 20.4 ms a call before, 3.3 ms a call now, which is the
 // 75 MB over PCIe and into the user's array.
 template <bool PLUS, int MU>

@@ -65,6 +65,8 @@ int gx_ctx_event_elapsed(gx_ctx ctx, int slot0, int slot1, double *ms);
 /* subset: GX_FULL for the whole lattice, GX_EVEN / GX_ODD for a half (checkerboarded) field. */
 int gx_field_create(gx_ctx ctx, const int dims[4], int Ls, int prec, int subset, gx_field *out);
 int gx_field_destroy(gx_field f);
+/* Done on return.  They use pinned chunks of the field's context (16 MB, from its first large transfer on), one
+ * transfer of a context at a time; transfers of several contexts run side by side. */
 int gx_field_import(gx_field f, const double *host);        /* host layout above */
 int gx_field_export(gx_field f, double *host);
 int gx_field_checkerboard(gx_field f, int *cb);              /* Grid: Lattice::Checkerboard() */
@@ -288,6 +290,7 @@ int gx_block_cgrq_vec(gx_op op, int herm, int n, gx_field *src, gx_field *psi, d
  * ConjugateGradientMultiShift.h:89-343: solves (MpcDagMpc + shifts[s]) psi[s] = src for nshift
  * shifts at once (poles = shifts, tolerances = per-shift relative residuals), from the Krylov
  * space of shifts[0], which must be the smallest.  Guesses are ignored (zero), as in Grid.
+ * Work memory: nshift half fields, and up to seven more while they take at most a quarter of what is then free.
  * 1 <= nshift <= 32.  psi: nshift distinct F64 half fields; st: nshift statistics (iterations until each shift
  * converged, true residual |(A + shift) psi - src| / |src|).  GX_ENOCONV when a shift is not
  * converged after maxit iterations. */
@@ -302,8 +305,8 @@ int gx_slice_inner_product_matrix(gx_field lhs, gx_field rhs, double *mat);
 /* No counterpart in the reference (Grid allocates freely).  For callers that cannot allocate device
  * memory (code under hipGraph capture, tight serving loops, harnesses that forbid hipMalloc):
  * gx_slice_inner_product_matrix with its workspace (workgroup partials and the result matrix,
- * 8.4 MB) in a fixed device array that each GPU holds until the process ends, instead of memory
- * allocated per call.  Same result, bit for bit.  Ls <= 16.  Calls that overlap on one GPU race on
+ * 8.4 MB) in a fixed device array that each GPU holds until the process ends, instead of the memory
+ * that a context allocates in its first block-algebra call.  Same result, bit for bit.  Ls <= 16.  Calls that overlap on one GPU race on
  * that array. */
 int gx_slice_inner_product_matrix_noalloc(gx_field lhs, gx_field rhs, double *mat);
 
