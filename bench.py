@@ -206,7 +206,7 @@ def bench_dhop_large(gx, ctx, tune):
                                 ((32, 32, 32, 32), gx.F32, 'mobius_32x32x32x32_ls16_f32', 8)):
         U = gx.random_gauge(dims, 1012, EPS)
         D = gx.FermionOp(ctx, U, dims, LS, 'mobius', **PARAMS)
-        tune('dhop_' + name, D, prec)
+        tune('dhop_' + name, D, prec, hop_only=True)
         fi = D.field(prec, 1)
         full = D.field(prec)
         full.gaussian(2012)
@@ -595,7 +595,7 @@ def main():
     kernel64, shape64 = None, 0
     for prec, name, c in ((gx.F64, 'f64', 16), (gx.F32, 'f32', 8), (gx.F16, 'f16', 4)):
         print(f'bench: dhop {name} ... ({time.perf_counter() - T_START:.0f} s)', file=sys.stderr, flush=True)
-        tune('dhop_' + name, D, prec, dhop_iters=50, rounds=5)
+        tune('dhop_' + name, D, prec, dhop_iters=50, rounds=5, hop_only=True)
         if prec == gx.F64:
             kernel64, shape64 = dhop_kernel_name(gx), gx.tune_get(gx.TUNE_DHOP_SHAPE)
         fi = D.field(prec, 1).upload(psi_o)
@@ -618,6 +618,7 @@ def main():
     cg = None
     if not args.no_cg:
         print(f'bench: cg ... ({time.perf_counter() - T_START:.0f} s)', file=sys.stderr, flush=True)
+        tune('cg_f64', D, gx.F64)
         tune('cg', D, gx.F32)
         src_full = gx.gaussian_fermion(DIMS, LS, 3003)
         fs, fsol = D.field().upload(src_full), D.field()

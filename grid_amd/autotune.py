@@ -181,9 +181,10 @@ class Autotuner:
         self.ctx.sync()
         return (time.perf_counter() - t0) / iters
 
-    def tune(self, D, prec=F64, dhop_iters=20, cg_iters=64, rounds=3, force=False):
-        """Tune for operator D at precision prec; returns the chosen knob values (and applies them)."""
-        key = workload_key(self.device, D.kind, D.dims, D.Ls, prec)
+    def tune(self, D, prec=F64, dhop_iters=20, cg_iters=64, rounds=3, force=False, hop_only=False):
+        """Tune for operator D at precision prec; returns the chosen knob values (and applies them).
+        hop_only: for programs that apply hops and do not solve, the fastest hop whatever a CG makes of its form."""
+        key = workload_key(self.device, D.kind, D.dims, D.Ls, prec) + ('|hop' if hop_only else '')
         if key in self.cache and not force:
             return self.apply_entry(self.cache[key])
         lt, lz, ly, lx = D.dims[3], D.dims[2], D.dims[1], D.dims[0]
@@ -240,20 +241,21 @@ class Autotuner:
         def plain(d):
             return not d.get(TUNE_DHOP_PERSIST, 0) and not d.get(TUNE_DHOP_TILE, 0)
 
-        if not plain(dict(hop_best)):
-            hop_best, _ = search([hop_best, fastest(plain)], cg_hop, rounds)
-        if dict(hop_best)[TUNE_DHOP_SHAPE] != shapes[0]:
-            alt = fastest(lambda d: plain(d) and d[TUNE_DHOP_SHAPE] == shapes[0])
-            hop_best, _ = search([hop_best, alt], cg_hop, rounds, margin=0.02)
-        # The epilogue kernels also use registers differently from the plain hop, so the fastest FP32 or FP16 hop
-        # of the other prefetch setting is compared by CG time too.
-        if prec != F64:
-            pf = dict(hop_best).get(TUNE_DHOP_PF, 0)
-            other = [c for c in hop_times
-                     if dict(c).get(TUNE_DHOP_PF, 0) != pf and not dict(c).get(TUNE_DHOP_PERSIST, 0)]
-            if other:
-                alt = min(other, key=lambda c: hop_times[c])
-                hop_best, t5 = search([hop_best, alt], cg_hop, rounds)
+        if not hop_only:
+            if not plain(dict(hop_best)):
+                hop_best, _ = search([hop_best, fastest(plain)], cg_hop, rounds)
+            if dict(hop_best)[TUNE_DHOP_SHAPE] != shapes[0]:
+                alt = fastest(lambda d: plain(d) and d[TUNE_DHOP_SHAPE] == shapes[0])
+                hop_best, _ = search([hop_best, alt], cg_hop, rounds, margin=0.02)
+            # The epilogue kernels also use registers differently from the plain hop, so the fastest FP32 or FP16 hop
+            # of the other prefetch setting is compared by CG time too.
+            if prec != F64:
+                pf = dict(hop_best).get(TUNE_DHOP_PF, 0)
+                other = [c for c in hop_times
+                         if dict(c).get(TUNE_DHOP_PF, 0) != pf and not dict(c).get(TUNE_DHOP_PERSIST, 0)]
+                if other:
+                    alt = min(other, key=lambda c: hop_times[c])
+                    hop_best, t5 = search([hop_best, alt], cg_hop, rounds)
 
         solver_best, solver_times = search(solver_candidates(), cg, rounds)
         entry = {'knobs': {KNOB_NAMES[k]: v for k, v in hop_best + solver_best},

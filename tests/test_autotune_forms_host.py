@@ -93,3 +93,19 @@ def test_split_range_is_the_librarys():
     with open(os.path.join(os.path.dirname(at.__file__), 'csrc', 'gx_internal.h')) as f:
         assert int(re.search(r'kSplitMax = (\d+);', f.read()).group(1)) == at.SPLIT_ENTRIES
     assert all(gx.tune_get(k, p) == v for k, v in at.HOP_DEFAULTS for p in at.PRECS)
+
+
+def test_hop_only():
+    """The hop's own winner stays where the program does not solve, whatever the CG takes."""
+    saved = {(k, p): gx.tune_get(k, p) for k in at.KNOB_NAMES for p in at.PRECS}
+    t = at.Autotuner(ctx=None, cache_path=None, device='gfx950')
+    fast = lambda: gx.tune_get(gx.TUNE_DHOP_SHAPE) == 4 and gx.tune_get(gx.TUNE_DHOP_PERSIST) == 1
+    t._time_dhop = lambda *a: 0.9 if fast() else 1.0
+    t._time_cg = lambda *a: 1.3 if fast() else 1.0
+    try:
+        D = FakeOp(BIG, 16)
+        assert t.tune(D, gx.F64, rounds=1, hop_only=True)[gx.TUNE_DHOP_PERSIST] == 1
+        assert t.tune(D, gx.F64, rounds=1)[gx.TUNE_DHOP_PERSIST] == 0  # and is not kept for solves
+    finally:
+        for (k, p), v in saved.items():
+            gx.tune_set(k, v, p)
