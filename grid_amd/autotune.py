@@ -186,7 +186,7 @@ class Autotuner:
         hop_only: for programs that apply hops and do not solve, the fastest hop whatever a CG makes of its form."""
         key = workload_key(self.device, D.kind, D.dims, D.Ls, prec) + ('|hop' if hop_only else '')
         if key in self.cache and not force:
-            return self.apply_entry(self.cache[key])
+            return self.apply_entry(self.cache[key], prec)
         lt, lz, ly, lx = D.dims[3], D.dims[2], D.dims[1], D.dims[0]
         rng = np.random.default_rng(1)
         shape = (lt, lz, ly, lx // 2, D.Ls, 4, 3)

@@ -109,3 +109,15 @@ def test_hop_only():
     finally:
         for (k, p), v in saved.items():
             gx.tune_set(k, v, p)
+
+
+def test_cached_workload_sets_its_precision_only():
+    saved = {(k, p): gx.tune_get(k, p) for k in at.KNOB_NAMES for p in at.PRECS}
+    t = at.Autotuner(ctx=None, cache_path=None, device='gfx950')
+    t.cache[at.workload_key('gfx950', 'wilson', BIG, 16, gx.F32)] = {'knobs': {'dhop_map': 2}}
+    try:
+        assert t.tune(FakeOp(BIG, 16), gx.F32) == {gx.TUNE_DHOP_MAP: 2}
+        assert [gx.tune_get(gx.TUNE_DHOP_MAP, p) for p in (gx.F64, gx.F32, gx.F16)] == [4, 2, 4]
+    finally:
+        for (k, p), v in saved.items():
+            gx.tune_set(k, v, p)
