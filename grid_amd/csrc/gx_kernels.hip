@@ -1867,8 +1867,8 @@ static GShape make_shape(int LS, int LB, int W) {
 
 // The leg-per-wave kernel's range: kSplitMax entries per checkerboard, and for a single checkerboard mostly one round of
 // resident workgroups, two per CU: a second, partly filled round costs more than the latency that is hidden.  One
-// checkerboard against the 4-wave kernel, FP64: 8^3x16 x 16 rows of 512 tiles 0.88, of 576 and 640 tiles (8^3x18,
-// 8^3x20 x 8) 1.1; 8^3x12 x 12 (615 tiles, 60 of 64 lanes) hop 11.0 us for 7.5, MpcDagMpc 50 for 36, CG iteration 65 for
+// checkerboard against the 4-wave kernel, FP64: hop on 8^4 x 16 (512 tiles) 0.88 of the time, 8^3x9 x 16 and 8^3x10 x 16
+// (576, 640) 1.11 and 1.13; 8^3x12 x 12 (615 tiles, 60 of 64 lanes) hop 11.0 us for 7.5, MpcDagMpc 50 for 36, CG iteration 65 for
 // 50, and at 512 tiles 8.9 for 7.3, at 432 6.3 for 7.1.  Fewer slices than 8 in FP64 are bound by the links and gain up to
 // kSplitMax (0.8-0.95); one or two slices in every precision (0.9-1.0).  FP32 and FP16 from 3 slices on are at 1.0-1.15 past
 // 512 tiles, but a bare hop (epi 0), whose registers let a third workgroup in, stays at 0.9 in FP16 and 0.95-1.0 in FP32

@@ -312,7 +312,8 @@ int gx_slice_inner_product_matrix_noalloc(gx_field lhs, gx_field rhs, double *ma
 
 /* Grid: sliceMaddMatrix(R, aa, X, Y, Orthog = 0, scale), Lattice_reduction.h:717-742:
  * R_t = Y_t + scale sum_s X_s aa(s, t).  aa: 2 Ls^2 doubles, row-major.  Y = NULL gives
- * sliceMulMatrix (R_t = scale sum_s X_s aa(s, t)).  R may be X or Y. */
+ * sliceMulMatrix (R_t = scale sum_s X_s aa(s, t)).  R may be X or Y.  This and gx_madd_matrix run on the
+ * stream of X's context; they wait for it when R or Y belongs to another one. */
 int gx_slice_madd_matrix(gx_field R, const double *aa, gx_field X, gx_field Y, double scale);
 
 /* Grid: InnerProductMatrix(m, X, Y) over std::vector<Field> (BlockConjugateGradient.h:35-42):
